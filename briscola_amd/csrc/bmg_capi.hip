@@ -542,7 +542,7 @@ void bmg_ctx::coarseSolve()
         throw Error(BMG_ERR_STATE, "coarse level not factorised");
     // the FP32 cycles solve by the inverse; FP64 keeps the reference's
     // substitutions, bit for bit
-    if (std::is_same<T, float>::value && dCoarseInv)
+    if (std::is_same<T, float>::value && coarseInvReady)
         launch_coarse_inv(lv[l].L, op<T>(l), X<T>(l), cst(B<T>(l)), dCoarseInv,
                           nc, l == 0, &bcval, stream);
     else
@@ -745,43 +745,13 @@ void bmg_ctx::prepareCoarse()
             for (int i = j + 1; i < n; i++) D[size_t(i)*n + j] *= rr;
         }
     }
-    // the inverse for the FP32 cycles (at most 64 cells): the factors'
-    // substitutions (LUBacksubstitute's order) on every unit vector
-    devFree(dCoarseInv);
-    if (n <= 64)
-    {
-        std::vector<double> G(64*64, 0.0), e(n);
-        for (int k = 0; k < n; k++)
-        {
-            std::fill(e.begin(), e.end(), 0.0);
-            e[k] = 1.0;
-            int ii = 0;
-            for (int i = 0; i < n; i++)
-            {
-                const int ip = piv[i];
-                double sum = e[ip];
-                e[ip] = e[i];
-                if (ii)
-                    for (int j = ii - 1; j < i; j++) sum -= D[size_t(i)*n + j]*e[j];
-                else if (sum != 0.0)
-                    ii = i + 1;
-                e[i] = sum;
-            }
-            for (int i = n - 1; i >= 0; i--)
-            {
-                double sum = e[i];
-                for (int j = i + 1; j < n; j++) sum -= D[size_t(i)*n + j]*e[j];
-                e[i] = sum/D[size_t(i)*n + i];
-            }
-            // column k of the inverse; lane i reads entry (i, j) at j*64 + i
-            for (int i = 0; i < n; i++) G[size_t(k)*64 + i] = e[i];
-        }
-        dCoarseInv = devUpload(G);
-        gen++;
-    }
-    // a coarse level that fits one wavefront is solved from padded
-    // column-major factors and the final row permutation (the pivot swaps
-    // applied in order to the identity)
+    // the row permutation (the pivot swaps applied in order to the identity)
+    // and the factors as the solve reads them: padded column-major for one
+    // wavefront, else row-major followed by column-major
+    std::vector<int> perm(n);
+    for (int i = 0; i < n; i++) perm[i] = i;
+    for (int i = 0; i < n; i++) std::swap(perm[piv[i]], perm[i]);
+    piv.swap(perm);
     const int w = coarse_wave_width(n);
     if (w)
     {
@@ -790,11 +760,14 @@ void bmg_ctx::prepareCoarse()
             for (int j = 0; j < w; j++)
                 F[size_t(j)*w + i] = i < n && j < n ? D[size_t(i)*n + j]
                                                     : double(i == j);
-        std::vector<int> perm(n);
-        for (int i = 0; i < n; i++) perm[i] = i;
-        for (int i = 0; i < n; i++) std::swap(perm[piv[i]], perm[i]);
         D.swap(F);
-        piv.swap(perm);
+    }
+    else
+    {
+        D.resize(2*size_t(n)*n);
+        for (int i = 0; i < n; i++)
+            for (int j = 0; j < n; j++)
+                D[size_t(n)*n + size_t(j)*n + i] = D[size_t(i)*n + j];
     }
     if (dLU && nc == n)
     {
@@ -807,6 +780,7 @@ void bmg_ctx::prepareCoarse()
     {
         devFree(dLU);
         devFree(dPiv);
+        devFree(dCoarseInv);
         dLU = devUpload(D);
         dPiv = devUpload(piv);
         gen++;
@@ -814,6 +788,24 @@ void bmg_ctx::prepareCoarse()
     nc = n;
     prepared = true;
     preparedCoarse = l;
+    coarseInvReady = false;
+}
+
+// The inverse the FP32 cycles solve the coarse system with, from the current
+// factors.
+void bmg_ctx::ensureCoarseInverse()
+{
+    if (coarseInvReady || opts.coarse_mode != BMG_COARSE_DIRECT ||
+        !prepared || preparedCoarse != coarseLevel())
+        return;
+    if (!dCoarseInv)
+    {
+        dCoarseInv = devAlloc<double>(size_t(nc)*nc);
+        gen++;
+    }
+    launch_lu_inverse(dLU, dPiv, nc, dCoarseInv, stream);
+    HIPCK(hipGetLastError());
+    coarseInvReady = true;
 }
 
 // MG.C:431-459: singularity pin of the coarse level, ghost elimination
@@ -872,6 +864,7 @@ void bmg_ctx::prepare(bool constMatrix)
 // FP32 copies of the operator and transfer data for mixed-precision cycles.
 void bmg_ctx::ensureMixed()
 {
+    ensureCoarseInverse();
     if (mixedReady) return;
     gen++;
     for (int l = 0; l < nLevels(); l++)

@@ -177,9 +177,10 @@ struct bmg_ctx
     int preparedCoarse = -1;
     // coarse LU
     double* dLU = nullptr;
-    // inverse of the coarse matrix (64 x 64 column-major, zero-padded) for
-    // the FP32 cycles, when the coarsest level has at most 64 cells
+    // inverse of the coarse matrix (nc x nc, row-major) for the FP32 cycles,
+    // and whether it is that of the current factors
     double* dCoarseInv = nullptr;
+    bool coarseInvReady = false;
     int* dPiv = nullptr;
     int nc = 0;
     // reductions
@@ -446,6 +447,7 @@ struct bmg_ctx
     void runFCG(bool constMatrix, bmg_stats* st);
     void prepare(bool constMatrix);
     void prepareCoarse();
+    void ensureCoarseInverse();
     void ensureMixed();
     void runSolve(bool constMatrix, bmg_stats* st);
     // runSolve in phases, each enqueued without synchronisation (and so

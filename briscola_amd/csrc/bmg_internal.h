@@ -261,8 +261,12 @@ void launch_defl_correct(const unsigned* cell, const int* comp, long ncells,
                          const double* einv, const double* part,
                          const int* coff, int m, double sign, Pair<T> f,
                          hipStream_t s);
-// Coarsest-level solve by a precomputed inverse (column-major, 64 x 64,
-// at most 64 cells), the ghost update after it.
+// Rows of the inverse (row-major n x n) from the factors and permutation of
+// launch_coarse_solve.
+void launch_lu_inverse(const double* lu, const int* perm, int n, double* inv,
+                       hipStream_t s);
+// Coarsest-level solve by a precomputed inverse (row-major n x n), the ghost
+// update with it.
 template <typename T>
 void launch_coarse_inv(const LevelDims& L, const OpView<T>& op, Pair<T> x,
                        Pair<const T> b, const double* inv, int n, int level0,
@@ -321,9 +325,9 @@ void launch_face_flux(const LevelDims& L, const double* x, const double* lam,
 // Width of the one-wavefront coarse solve for an n-cell coarse level (a
 // power of two >= n, at least 8), or 0 when n exceeds one wavefront.  With a
 // width N the factors are stored column-major in an N x N array padded with
-// unit rows (lu[j*N + i] = LU(i, j)) and piv holds the row permutation
-// (row i of the permuted right-hand side is row piv[i] of the original);
-// otherwise lu is the n x n row-major LU and piv the pivot sequence.
+// unit rows (lu[j*N + i] = LU(i, j)); otherwise lu holds the n x n factors
+// row-major, then once more column-major.  piv is the row permutation either
+// way (row i of the permuted right-hand side is row piv[i] of the original).
 inline int coarse_wave_width(int n)
 {
     if (n > 64) return 0;

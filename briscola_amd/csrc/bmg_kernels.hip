@@ -2707,38 +2707,61 @@ __global__ void k_split_div(LevelDims L, const double* b, double lam0,
 }
 
 // ---------------------------------------------------------------------------
-// Coarsest-level direct solve, one workgroup (APLU.C:91-128 with rhsSource,
-// linearSystemAggregation.C:336-430).  The permutation is applied first and
-// the unit-lower forward substitution runs column by column; for each row
-// the subtractions still happen in column order, exactly as the row-wise
-// LUBacksubstitute.  The upper back substitution is row-wise in one lane.
-// The factors are staged in LDS when they fit.  Then the full ghost update
-// of the level (APLU.C:126).
-template <typename T, bool LDS>
+// Value of lane `lane` (uniform) in every lane.
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane(int(b), lane);
+    const int hi = __builtin_amdgcn_readlane(int(b >> 32), lane);
+    return __longlong_as_double((long long)(unsigned)lo |
+                                ((long long)hi << 32));
+}
+
+// Coarsest-level direct solve of more than 64 cells, one workgroup
+// (APLU.C:91-128 with rhsSource, linearSystemAggregation.C:336-430), bit for
+// bit LUBacksubstitute's subtractions: every row's terms in increasing
+// column order.  lug holds the n x n factors twice, row-major and then
+// column-major; perm the final row permutation.
+//
+// Forward (unit lower): blocks of 64 columns.  One wavefront solves the
+// block's 64 rows (lane = row, each solved value broadcast by a lane read),
+// then all threads subtract the block's 64 terms from the rows below it, in
+// column order; two barriers per block instead of one per column.
+//
+// Backward (upper): row i's sum y_i - U(i,i+1) y_(i+1) - U(i,i+2) y_(i+2) -
+// ... starts with the value solved last, so the n^2/2 subtractions are one
+// chain that no other order may shorten: it bounds the kernel.  STAGED: the
+// first wavefront only runs that chain, on products the other three formed
+// in LDS one row ahead (U's rows loaded three rows ahead); only
+// U(i,i+1) y_(i+1) is formed in the chain.  216 cells (a 6^3 level): 873 us
+// with the loads and products in the chain, 291 us staged, 212 us with the
+// products at the start of the row and read two per LDS load; the 23 000
+// dependent FP64 subtractions alone are about 100 us.  Then the full ghost
+// update of the level (APLU.C:126).
+constexpr int COARSE_STAGED_MAX = 1600;   // 5n + 4 doubles below 64 KB
+
+template <typename T, bool STAGED>
 __device__ __forceinline__ void coarse_solve_body(const Bid bid,
                                                   const LevelDims& L,
                                                   const OpView<T>& op,
                                                   Pair<T> x,
                                                   Pair<const T> b,
                                                   const double* lug,
-                                                  const int* piv, int n,
+                                                  const int* perm, int n,
                                                   int level0, const BcVals& bv)
 {
     extern __shared__ double smem[];
     double* y = smem;
-    const double* lu = lug;
+    const double* lu = lug;                   // (i, j) at i*n + j
+    const double* luc = lug + size_t(n)*n;    // (i, j) at j*n + i
     const int tid = threadIdx.x, nt = blockDim.x;
-    if constexpr (LDS)
-    {
-        double* l = smem + n;
-        for (int t = tid; t < n*n; t += nt) l[t] = lug[t];
-        lu = l;
-    }
     const int N1 = L.N[1], N2 = L.N[2];
     const int off[7][3] = {{0,0,0},{-1,0,0},{1,0,0},{0,-1,0},{0,1,0},
                            {0,0,-1},{0,0,1}};
-    for (int q = tid; q < n; q += nt)
+    for (int i = tid; i < n; i += nt)
     {
+        // row i of the permuted right-hand side
+        const int q = perm[i];
         const int I = 1 + q/(N1*N2), J = 1 + (q/N2) % N1, K = 1 + q % N2;
         const int colour = (I + J + K) & 1;
         const int idx = cidx(L, I, J, K);
@@ -2758,41 +2781,192 @@ __device__ __forceinline__ void coarse_solve_body(const Bid bid,
                 v = v - t;
             }
         }
-        y[q] = v;
+        y[i] = v;
     }
-    __syncthreads();
-    if (tid == 0)
-        for (int i = 0; i < n; i++)
+    double* const dg = smem + n;              // U(i, i)
+    double* const su = smem + 2*n;            // U(i, i+1)
+    if constexpr (STAGED)
+        for (int i = tid; i < n; i += nt)
         {
-            const int ip = piv[i];
-            const double t = y[ip];
-            y[ip] = y[i];
-            y[i] = t;
+            dg[i] = lu[size_t(i)*n + i];
+            su[i] = i + 1 < n ? lu[size_t(i)*n + i + 1] : 0.0;
         }
     __syncthreads();
-    for (int j = 0; j < n; j++)
+    for (int j0 = 0; j0 < n; j0 += 64)
     {
-        const double yj = y[j];
-        for (int i = j + 1 + tid; i < n; i += nt)
+        const int nb = min(64, n - j0);
+        if (tid < 64)
         {
-            const double t = lu[i*n + j]*yj;
-            y[i] = y[i] - t;
+            const int r = j0 + tid;
+            const bool own = tid < nb;
+            double s = own ? y[r] : 0.0;
+            // rows past the block load the block's last row instead
+            const double* c = luc + size_t(j0)*n + j0 + min(tid, nb - 1);
+            for (int k0 = 0; k0 < nb; k0 += 8)
+            {
+                double l[8];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    l[u] = c[size_t(min(k0 + u, nb - 1))*n];
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    if (k0 + u < nb)
+                    {
+                        const double yj = lane_value(s, k0 + u);
+                        const double t = l[u]*yj;
+                        const double sn = s - t;
+                        s = tid > k0 + u ? sn : s;
+                    }
+            }
+            if (own) y[r] = s;
+        }
+        __syncthreads();
+        // a block before the last is 64 columns wide
+        for (int i = j0 + 64 + tid; i < n; i += nt)
+        {
+            double s = y[i];
+            const double* c = luc + size_t(j0)*n + i;
+            for (int k0 = 0; k0 < 64; k0 += 16)
+            {
+                double l[16];
+#pragma unroll
+                for (int u = 0; u < 16; u++) l[u] = c[size_t(k0 + u)*n];
+#pragma unroll
+                for (int u = 0; u < 16; u++)
+                {
+                    const double t = l[u]*y[j0 + k0 + u];
+                    s = s - t;
+                }
+            }
+            y[i] = s;
         }
         __syncthreads();
     }
-    if (tid == 0)
-        for (int i = n - 1; i >= 0; i--)
+    if constexpr (STAGED)
+    {
+        // two rows of products, 16-byte aligned
+        const int ps = (n + 1) & ~1;
+        double* const prod = smem + ((3*n + 1) & ~1);
+        const int pt = tid - 64, np = nt - 64;
+        // U(r, c) of the rows three stages ahead, at most two columns a
+        // thread (n <= 2 np); larger systems load when they multiply, their
+        // chain being long enough to hide it
+        const bool ring = n <= 2*np;
+        double u[4][2];
+        auto row_at = [&](int t) { return max(n - 2 - t, 0); };
+        auto fetch = [&](int t, double (&d)[2])
         {
-            const double* row = lu + i*n;
-            double sum = y[i];
-            for (int j = i + 1; j < n; j++)
-            {
-                const double t = row[j]*y[j];
-                sum = sum - t;
-            }
-            y[i] = sum/row[i];
+            const double* rp = lu + size_t(row_at(t))*n;
+            d[0] = rp[min(pt, n - 1)];
+            d[1] = rp[min(pt + np, n - 1)];
+        };
+        if (tid >= 64 && ring)
+        {
+            fetch(0, u[0]);
+            fetch(1, u[1]);
+            fetch(2, u[2]);
         }
-    __syncthreads();
+        for (int t0 = 0; t0 < n; t0 += 4)
+        {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+            {
+                const int t = t0 + k;
+                if (t >= n) break;
+                const int i = n - 1 - t;
+                if (tid < 64)
+                {
+                    // m products at p[0..m), from column i+2
+                    const double* p = prod + (i & 1)*ps;
+                    const double2* p2 = reinterpret_cast<const double2*>(p);
+                    const int m = n - i - 2;
+                    double sum = y[i];
+                    const double dii = dg[i];
+                    if (i + 1 < n)
+                    {
+                        const double first = su[i]*y[i + 1];
+                        sum = sum - first;
+                    }
+                    int j = 0;
+                    double2 c[8], d[8];
+                    auto get = [&](double2 (&v)[8], int at)
+                    {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) v[e] = p2[at/2 + e];
+                    };
+                    auto take = [&](const double2 (&v)[8])
+                    {
+#pragma unroll
+                        for (int e = 0; e < 8; e++)
+                        {
+                            sum = sum - v[e].x;
+                            sum = sum - v[e].y;
+                        }
+                    };
+                    if (m >= 16)
+                    {
+                        get(c, 0);
+                        for (; j + 48 <= m; j += 32)
+                        {
+                            get(d, j + 16);
+                            take(c);
+                            get(c, j + 32);
+                            take(d);
+                        }
+                        take(c);
+                        j += 16;
+                    }
+                    for (; j + 4 <= m; j += 4)
+                    {
+                        const double2 e0 = p2[j/2], e1 = p2[j/2 + 1];
+                        sum = sum - e0.x;
+                        sum = sum - e0.y;
+                        sum = sum - e1.x;
+                        sum = sum - e1.y;
+                    }
+                    for (; j < m; j++) sum = sum - p[j];
+                    if (tid == 0) y[i] = sum/dii;
+                }
+                else
+                {
+                    // products of row i-1 with the values already solved,
+                    // column c at c - (i+1)
+                    const int r = i - 1;
+                    double* p = prod + (r & 1)*ps - (r + 2);
+                    if (ring)
+                    {
+                        fetch(t + 3, u[(k + 3) & 3]);
+                        if (r >= 0)
+                        {
+                            if (pt >= r + 2 && pt < n) p[pt] = u[k][0]*y[pt];
+                            const int c2 = pt + np;
+                            if (c2 >= r + 2 && c2 < n) p[c2] = u[k][1]*y[c2];
+                        }
+                    }
+                    else if (r >= 0)
+                        for (int c2 = r + 2 + pt; c2 < n; c2 += np)
+                            p[c2] = lu[size_t(r)*n + c2]*y[c2];
+                }
+                __syncthreads();
+            }
+        }
+    }
+    else
+    {
+        if (tid == 0)
+            for (int i = n - 1; i >= 0; i--)
+            {
+                const double* row = lu + size_t(i)*n;
+                double sum = y[i];
+                for (int j = i + 1; j < n; j++)
+                {
+                    const double t = row[j]*y[j];
+                    sum = sum - t;
+                }
+                y[i] = sum/row[i];
+            }
+        __syncthreads();
+    }
     for (int q = tid; q < n; q += nt)
     {
         const int I = 1 + q/(N1*N2), J = 1 + (q/N2) % N1, K = 1 + q % N2;
@@ -2809,19 +2983,19 @@ __device__ __forceinline__ void coarse_solve_body(const Bid bid,
     }
 }
 
-template <typename T, bool LDS>
+template <typename T, bool STAGED>
 __global__ __launch_bounds__(256) void k_coarse_solve(LevelDims L,
                                                       OpView<T> op, Pair<T> x,
                                                       Pair<const T> b,
                                                       const double* lug,
-                                                      const int* piv, int n,
+                                                      const int* perm, int n,
                                                       int level0, BcVals bv)
 {
     const Bid bid{blockIdx.x, blockIdx.y, blockIdx.z};
-    coarse_solve_body<T, LDS>(bid, L, op, x, b, lug, piv, n, level0, bv);
+    coarse_solve_body<T, STAGED>(bid, L, op, x, b, lug, perm, n, level0, bv);
 }
 
-template <typename T, bool LDS>
+template <typename T, bool STAGED>
 struct KCoarse
 {
     static constexpr int bx = 256, by = 1;
@@ -2833,34 +3007,24 @@ struct KCoarse
         Pair<T> x;
         Pair<const T> b;
         const double* lug;
-        const int* piv;
+        const int* perm;
         int n;
         int level0;
         BcVals bv;
     };
     __device__ static void run(const Bid bid, const Args& a)
     {
-        coarse_solve_body<T, LDS>(bid, a.L, a.op, a.x, a.b, a.lug, a.piv, a.n,
-                                  a.level0, a.bv);
+        coarse_solve_body<T, STAGED>(bid, a.L, a.op, a.x, a.b, a.lug, a.perm,
+                                     a.n, a.level0, a.bv);
     }
     static void launch(dim3 g, size_t shm, hipStream_t s, const Args& a)
     {
-        hipLaunchKernelGGL((k_coarse_solve<T, LDS>), g, dim3(bx, by), shm, s,
-                           a.L, a.op, a.x, a.b, a.lug, a.piv, a.n, a.level0,
-                           a.bv);
+        hipLaunchKernelGGL((k_coarse_solve<T, STAGED>), g, dim3(bx, by), shm,
+                           s, a.L, a.op, a.x, a.b, a.lug, a.perm, a.n,
+                           a.level0, a.bv);
     }
 };
 
-
-// Value of lane `lane` (a compile-time lane) in every lane.
-__device__ __forceinline__ double lane_value(double v, int lane)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane(int(b), lane);
-    const int hi = __builtin_amdgcn_readlane(int(b >> 32), lane);
-    return __longlong_as_double((long long)(unsigned)lo |
-                                ((long long)hi << 32));
-}
 
 // Coarsest-level direct solve of at most N <= 64 cells in one wavefront,
 // with the same operations in the same order as k_coarse_solve (APLU.C:
@@ -2952,75 +3116,153 @@ __device__ __forceinline__ void coarse_solve_wave_body(const Bid bid,
     }
 }
 
+// Rows of the inverse of the coarse matrix from its factors, one wavefront
+// per row: w U = e_i, then v L = w, and row i of the inverse is v with its
+// entries moved by the row permutation (entry c to column perm[c]).  Both
+// substitutions subtract a multiple of one row of the factors (entry (i, j)
+// at i*rs + j*cs) from the rest of w, lanes along the row; the next row is
+// loaded while the current one is subtracted.  Once per factorisation, in
+// FP64, off the critical path of the cycles.
+__global__ __launch_bounds__(64) void k_lu_inverse(const double* lu, int rs,
+                                                   int cs, const int* perm,
+                                                   int n, double* inv)
+{
+    extern __shared__ double wv[];
+    const int lane = threadIdx.x;
+    const int i = blockIdx.x;
+    auto at = [&](int r, int c) { return lu[size_t(r)*rs + size_t(c)*cs]; };
+    // the first four entries of a row that a lane holds, zero past the row
+    auto load = [&](int r, double (&v)[4])
+    {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            const int c = lane + 64*u;
+            v[u] = r >= 0 && r < n && c < n ? at(r, c) : 0.0;
+        }
+    };
+    for (int c = lane; c < n; c += 64) wv[c] = c == i ? 1.0 : 0.0;
+    __syncthreads();
+    double cur[4], nxt[4];
+    load(i, cur);
+    double diag = at(i, i);
+    for (int k = i; k < n; k++)
+    {
+        load(k + 1, nxt);
+        const double diagNext = k + 1 < n ? at(k + 1, k + 1) : 1.0;
+        const double wk = wv[k]/diag;
+        diag = diagNext;
+        __syncthreads();
+        if (lane == 0) wv[k] = wk;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            const int c = lane + 64*u;
+            if (c > k && c < n) wv[c] = __builtin_fma(-wk, cur[u], wv[c]);
+            cur[u] = nxt[u];
+        }
+        for (int c = lane + 256; c < n; c += 64)
+            if (c > k) wv[c] = __builtin_fma(-wk, at(k, c), wv[c]);
+        __syncthreads();
+    }
+    load(n - 1, cur);
+    for (int j = n - 1; j > 0; j--)
+    {
+        load(j - 1, nxt);
+        const double vj = wv[j];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            const int c = lane + 64*u;
+            if (c < j) wv[c] = __builtin_fma(-vj, cur[u], wv[c]);
+            cur[u] = nxt[u];
+        }
+        for (int c = lane + 256; c < j; c += 64)
+            wv[c] = __builtin_fma(-vj, at(j, c), wv[c]);
+        __syncthreads();
+    }
+    for (int c = lane; c < n; c += 64) inv[size_t(i)*n + perm[c]] = wv[c];
+}
+
 // The coarsest-level solve of the FP32 cycles of mixed precision (no
-// bitwise contract), for at most 64 cells: x = A^-1 (b - out-of-system
-// couplings) with the inverse precomputed in FP64 from the LU factors
-// (column-major, padded to 64 with zeros), one wavefront, lane i forming row
-// i from broadcasts of the right-hand side -- 64 independent multiply-adds
-// instead of the substitutions' chain of dependent ones.  Right-hand side
-// and ghost update as in coarse_solve_wave_body.
+// bitwise contract): x = A^-1 b with the rows of the inverse formed once in
+// FP64 (k_lu_inverse).  One wavefront per row, lanes along it, the sums in
+// FP64.  The couplings to ghosts that the substitutions subtract from b are
+// left out: prepare() eliminates every coarse stencil, so they are exactly
+// zero.  A ghost of the level is a function of one interior cell
+// (ghost_cell, mode 1), so the wavefront that owns the cell writes the up
+// to 26 ghosts that take their value from it, one per lane, and nothing
+// waits for the other rows.
+// Bound by the latency of one load of b and the row: 4.0 us at 72 cells,
+// 5.4 us at 64, 7.0 us at 216 (the 6^3 level under 3*2^k sizes), where the
+// substitutions' n^2/2 dependent subtractions took 70.6 us (72) and 1241 us
+// (216) and one wavefront with all 64 rows of an inverse 12.8 us.
 template <typename T>
-__device__ __forceinline__ void coarse_inv_body(const Bid, const LevelDims& L,
+__device__ __forceinline__ void coarse_inv_body(const Bid bid,
+                                                const LevelDims& L,
                                                 const OpView<T>& op, Pair<T> x,
                                                 Pair<const T> b,
                                                 const double* inv, int n,
                                                 int level0, const BcVals& bv)
 {
-    const int lane = threadIdx.x;
+    const int lane = int(threadIdx.x) & 63;
+    const int row = int(bid.x)*4 + (int(threadIdx.x) >> 6);
+    if (row >= n) return;
     const int N1 = L.N[1], N2 = L.N[2];
-    const int off[7][3] = {{0,0,0},{-1,0,0},{1,0,0},{0,-1,0},{0,1,0},
-                           {0,0,-1},{0,0,1}};
-    double v = 0.0;
-    if (lane < n)
+    const double* g = inv + size_t(row)*n;
+    double y = 0.0;
+#pragma unroll 4
+    for (int q = lane; q < n; q += 64)
     {
-        const int q = lane;
         const int I = 1 + q/(N1*N2), J = 1 + (q/N2) % N1, K = 1 + q % N2;
-        const int colour = (I + J + K) & 1;
-        const int idx = cidx(L, I, J, K);
-        v = double(col(b, colour)[idx]);
-        for (int s = 1; s < 7; s++)
+        y = __builtin_fma(g[q], double(ld(col(b, (I + J + K) & 1),
+                                          unsigned(cidx(L, I, J, K)))), y);
+    }
+    for (int o = 32; o > 0; o >>= 1) y += __shfl_xor(y, o, 64);
+    const T v = T(y);
+    if (lane >= 27) return;
+    // lane: offset (-1, 0, 1) of the target along each axis
+    const int s[3] = {1 + row/(N1*N2), 1 + (row/N2) % N1, 1 + row % N2};
+    const int bo[3] = {lane/9 - 1, lane/3 % 3 - 1, lane % 3 - 1};
+    int nout = 0;
+    bool allPer = true;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+    {
+        const int bcf = bo[d] > 0 ? L.bc[2*d + 1] : L.bc[2*d];
+        nout += bo[d] != 0;
+        if (bo[d] != 0 && bcf != PER) allPer = false;
+    }
+    int t[3];
+    T val = v;
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+    {
+        t[d] = bo[d] == 0 ? s[d] : (bo[d] < 0 ? 0 : L.N[d] + 1);
+        // the ghost's source along d: the cell beside it, or its image
+        const bool low = (bo[d] < 0) != allPer;
+        if (bo[d] != 0 && s[d] != (low ? 1 : L.N[d])) return;
+        if (nout == 1 && !allPer && bo[d] != 0)
         {
-            const int g[3] = {I + off[s][0], J + off[s][1], K + off[s][2]};
-            bool out = false;
-            for (int d = 0; d < 3; d++)
-                if ((g[d] < 1 || g[d] > L.N[d]) &&
-                    L.bc[2*d + (g[d] > L.N[d])] != PER)
-                    out = true;
-            if (out)
-            {
-                const double a = double(op.a7[colour][s*nci(L) + idx]);
-                v = v - a*double(col(x, colour ^ 1)[cidx(L, g[0], g[1], g[2])]);
-            }
+            const int f = 2*d + (bo[d] > 0);
+            const T H = T(level0 ? 1.0 : 0.0);
+            const T bvf = T(level0 ? bc_value(L, bv, f, s) : 0.0);
+            if (L.bc[f] == NEU)
+                val = v + H*bvf/op.dl[d][bo[d] > 0 ? L.N[d] + 1 : 1];
+            else
+                val = H*T(2.0)*bvf - v;
         }
     }
-    // inv is 64 x 64 with zeros beyond n, v zero beyond n: a fixed trip
-    // count lets the loads of 16 columns be issued together
-    double y = 0.0;
-#pragma unroll 16
-    for (int j = 0; j < 64; j++)
-        y += inv[j*64 + lane]*__shfl(v, j, 64);
-    if (lane < n)
-    {
-        const int q = lane;
-        const int I = 1 + q/(N1*N2), J = 1 + (q/N2) % N1, K = 1 + q % N2;
-        col(x, (I + J + K) & 1)[cidx(L, I, J, K)] = T(y);
-    }
-    __syncthreads();
-    const Shell sh = shell_all(L);
-    const int ns = sh.nA + sh.nB + sh.nC;
-    for (int t = lane; t < ns; t += 64)
-    {
-        int I, J, K;
-        if (shell_cell(L, sh, t, I, J, K))
-            ghost_cell(L, op, x, 1, level0, bv, I, J, K);
-    }
+    st(col(x, (t[0] + t[1] + t[2]) & 1), unsigned(cidx(L, t[0], t[1], t[2])),
+       val);
 }
 
 template <typename T>
-__global__ __launch_bounds__(64) void k_coarse_inv(LevelDims L, OpView<T> op,
-                                                   Pair<T> x, Pair<const T> b,
-                                                   const double* inv, int n,
-                                                   int level0, BcVals bv)
+__global__ __launch_bounds__(256) void k_coarse_inv(LevelDims L, OpView<T> op,
+                                                    Pair<T> x,
+                                                    Pair<const T> b,
+                                                    const double* inv, int n,
+                                                    int level0, BcVals bv)
 {
     const Bid bid{blockIdx.x, blockIdx.y, blockIdx.z};
     coarse_inv_body<T>(bid, L, op, x, b, inv, n, level0, bv);
@@ -3029,7 +3271,7 @@ __global__ __launch_bounds__(64) void k_coarse_inv(LevelDims L, OpView<T> op,
 template <typename T>
 struct KCoarseInv
 {
-    static constexpr int bx = 64, by = 1;
+    static constexpr int bx = 256, by = 1;
     static constexpr bool lds = false;
     struct Args
     {
@@ -5260,9 +5502,19 @@ void launch_coarse_inv(const LevelDims& L, const OpView<T>& op, Pair<T> x,
                        Pair<const T> b, const double* inv, int n, int level0,
                        const BcData* bcval, hipStream_t s)
 {
-    if (n > 64) throw std::runtime_error("coarse inverse: more than 64 cells");
-    dispatch<KCoarseInv<T>>(dim3(1), 0, s,
+    dispatch<KCoarseInv<T>>(dim3(unsigned(n + 3)/4), 0, s,
                             {L, op, x, b, inv, n, level0, bcvals(bcval)});
+}
+
+void launch_lu_inverse(const double* lu, const int* perm, int n, double* inv,
+                       hipStream_t s)
+{
+    direct_only("coarse inverse");
+    // at most 64 cells: column-major of width w; else row-major
+    const int w = coarse_wave_width(n);
+    hipLaunchKernelGGL(k_lu_inverse, dim3(unsigned(n)), dim3(64),
+                       size_t(n)*sizeof(double), s, lu, w ? 1 : n, w ? w : 1,
+                       perm, n, inv);
 }
 
 template <typename T>
@@ -5271,6 +5523,9 @@ void launch_coarse_solve(const LevelDims& L, const OpView<T>& op, Pair<T> x,
                          int n, int level0, const BcData* bcval,
                          hipStream_t s)
 {
+    // up to 64 cells one wavefront holds a row per lane; above, the staged
+    // form wherever its LDS fits (216 cells: 212 us against 873 us with the
+    // rows read inside the chain)
     switch (coarse_wave_width(n))
     {
     case 8:
@@ -5296,8 +5551,9 @@ void launch_coarse_solve(const LevelDims& L, const OpView<T>& op, Pair<T> x,
     default:
         break;
     }
-    if (size_t(n)*(n + 1)*sizeof(double) <= 56*1024)
-        dispatch<KCoarse<T, true>>(dim3(1), size_t(n)*(n + 1)*sizeof(double), s,
+    if (n <= COARSE_STAGED_MAX)
+        dispatch<KCoarse<T, true>>(dim3(1), (5*size_t(n) + 4)*sizeof(double),
+                                   s,
                                    {L, op, x, b, lu, piv, n, level0,
                                     bcvals(bcval)});
     else

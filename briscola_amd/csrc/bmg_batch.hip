@@ -724,6 +724,7 @@ void batch_solve(bmg_batch* B, double* const* db, double* const* dx,
                 c->prepareFCG();
                 HIPCK(hipStreamSynchronize(c->stream));
             }
+            mixedOf(c) ? c->ensureTail<float>() : c->ensureTail<double>();
         }
         std::vector<double> init(n), cur(n);
         std::vector<int> iter(n, 0);

@@ -497,8 +497,9 @@ template <typename T>
 void bmg_ctx::prolongFrom(int l, int skipColour)
 {
     // the coarse ghosts are used, so correct them first
-    // (linearProlongationScheme.C:128)
-    launch_bc_fill(lv[l + 1].L, op<T>(l + 1), X<T>(l + 1), 1, (l + 1) == 0,
+    // (linearProlongationScheme.C:128); the tail leaves them so
+    if (tailLevel<T>() != l + 1)
+        launch_bc_fill(lv[l + 1].L, op<T>(l + 1), X<T>(l + 1), 1, (l + 1) == 0,
                    &bcval, stream);
     launch_prolong(lv[l].L, lv[l + 1].L, transfer<T>(l), cst(X<T>(l + 1)),
                    X<T>(l), stream, skipColour);
@@ -550,6 +551,165 @@ void bmg_ctx::coarseSolve()
                             dPiv, nc, l == 0, &bcval, stream);
 }
 
+// The steps of smooth<T> on level l for a given number of sweeps as the
+// one-workgroup tail runs them (same phases, same skipped repetitions);
+// zeroStart: from x = 0 with every ghost 0.  -1 when they do not fit.
+template <typename T>
+int bmg_ctx::tailSteps(int l, int sweeps, bool zeroStart,
+                       bmg::TailStep* out) const
+{
+    int n = 0;
+    auto add = [&](int type, int axis, int c0, int c1)
+    {
+        if (n >= 0 && n < bmg::TAIL_STEPS)
+            out[n++] = bmg::TailStep{(unsigned char)type, (unsigned char)axis,
+                                     (signed char)c0, (signed char)c1};
+        else
+            n = -1;
+    };
+    if (sweeps <= 0) return 0;
+    const int wrap = wrapAxes<T>(l);
+    const bool slabs = anyPeriodic() && !wrap;
+    if (wrap && !zeroStart) add(bmg::TAIL_GHOSTS, 0, -1, -1);
+    int prev = -1;
+    for (int s = 0; s < sweeps; s++)
+    {
+        int cols[4];
+        const int nc = phase_colours(interior(l, wrap ? 0 : 1), cols);
+        for (int i = 0; i < nc; i++)
+        {
+            if (cols[i] != prev) add(bmg::TAIL_PHASE, 0, cols[i], -1);
+            prev = cols[i];
+        }
+        if (!slabs) continue;
+        add(bmg::TAIL_GHOSTS, 0, -1, -1);
+        for (int d = 0; d < 3; d++)
+        {
+            if (!periodic(2*d)) continue;
+            int c0[4], c1[4];
+            const int n0 = phase_colours(slab(l, 2*d), c0);
+            const int n1 = phase_colours(slab(l, 2*d + 1), c1);
+            if (lv[l].L.N[d] >= 3 && n0 == n1)
+                for (int i = 0; i < n0; i++)
+                    add(bmg::TAIL_SLAB, d, c0[i], c1[i]);
+            else
+            {
+                for (int i = 0; i < n0; i++) add(bmg::TAIL_SLAB, d, c0[i], -1);
+                for (int i = 0; i < n1; i++) add(bmg::TAIL_SLAB, d, -1, c1[i]);
+            }
+        }
+        prev = -1;
+    }
+    return n;
+}
+
+// The plan of the small levels' one-workgroup leg for the current operator
+// and options (launch_tail), or none: V-cycles with the direct coarse solve
+// and red-black smoothing, from the first level of at most TAIL_CELLS
+// cells whose coarser levels are all refined by 2 on every axis and stored
+// as stencils, as far as their x fits LDS.  Before a capture or a recording
+// (it copies to the device); the cycles use it while its generation holds.
+template <typename T>
+void bmg_ctx::ensureTail()
+{
+    TailState<T>& ts = tail<T>();
+    if (ts.gen == gen) return;
+    ts.gen = gen;
+    ts.level = -1;
+    const int lc = coarseLevel();
+    if (opts.smoother != BMG_RBGS || opts.cycle != BMG_VCYCLE ||
+        opts.coarse_mode != BMG_COARSE_DIRECT || fuseSmoothing != 0 ||
+        !prepared || preparedCoarse != lc)
+        return;
+    const bool whole = std::is_same<T, float>::value && coarseInvReady;
+    int top = lc;
+    size_t need = 0;
+    // pitches of a level's x in LDS: the lanes of a half wavefront (both
+    // planes of a block, then along K, then J) fall into different banks
+    auto dims = [&](int l)
+    {
+        bmg::TailDims L;
+        static_cast<LevelDims&>(L) = lv[l].L;
+        const int banks = sizeof(T) == 4 ? 32 : 16;
+        L.pJ = L.P[2];
+        if (sizeof(T) == 4 && L.N[2] % 2 == 0 && 2*L.N[2] <= banks)
+            while (2*L.pJ % banks != L.N[2] % banks) L.pJ++;
+        L.pI = (L.P[1]*L.pJ + banks - 1)/banks*banks;
+        auto magic = [](int d) { return unsigned((1ULL << 32)/d + 1); };
+        L.mP1 = magic(L.P[1]);
+        L.mP2 = magic(L.P[2]);
+        L.mN1 = magic(std::max(2, L.N[1]));
+        return L;
+    };
+    // x of a level and b of the next coarser one
+    auto bytes = [&](int l)
+    {
+        const bmg::TailDims L = dims(l);
+        const size_t b = l < lc ? size_t(lv[l + 1].cells()) : 0;
+        return sizeof(T)*(size_t(L.P[0])*L.pI + ((b + 3) & ~size_t(3)));
+    };
+    for (int l = lc; l >= 1; l--)
+    {
+        const Level& q = lv[l];
+        const bool stored = std::is_same<T, float>::value ? q.a7f[0] != nullptr
+                                                          : q.a7[0] != nullptr;
+        if (q.opkind != bmg::OP_STENCIL || !stored ||
+            q.cells() > bmg::TAIL_CELLS || need + bytes(l) > 65536 ||
+            lc - l + 1 > bmg::TAIL_LEVELS)
+            break;
+        if (l < lc && (lv[l + 1].L.R[0] != 2 || lv[l + 1].L.R[1] != 2 ||
+                       lv[l + 1].L.R[2] != 2))
+            break;
+        need += bytes(l);
+        top = l;
+    }
+    if (top >= lc) return;
+    std::unique_ptr<bmg::TailPlan<T>> p(new bmg::TailPlan<T>());
+    p->nl = lc - top + 1;
+    p->singular = singular();
+    p->nc = nc;
+    p->inv = whole ? dCoarseInv : nullptr;
+    p->lds = need;
+    size_t at = 0;
+    for (int l = top; l <= lc; l++)
+    {
+        bmg::TailLevel<T>& t = p->lv[l - top];
+        const OpView<T> o = op<T>(l);
+        t.L = dims(l);
+        const Pair<T> xx = X<T>(l), bb = B<T>(l);
+        for (int c = 0; c < 2; c++)
+        {
+            t.a7[c] = o.a7[c];
+            t.x[c] = xx.c[c];
+            t.b[c] = bb.c[c];
+        }
+        if (l < lc) t.tv = transfer<T>(l);
+        t.wrap = wrapAxes<T>(l);
+        t.refresh = anyPeriodic() && t.wrap == 0;
+        t.xo = int(at);
+        at += size_t(t.L.P[0])*t.L.pI;
+        t.bo = 0;
+        if (l > top)
+        {
+            t.bo = int(at);
+            at += (size_t(lv[l].cells()) + 3) & ~size_t(3);
+        }
+        t.nPre = l < lc ? tailSteps<T>(l, opts.n_sweeps_pre, true, t.pre) : 0;
+        t.nPost = l < lc ? tailSteps<T>(l, opts.n_sweeps_post, false, t.post)
+                         : 0;
+        if (t.nPre < 0 || t.nPost < 0) return;
+    }
+    if (!ts.plan) ts.plan = devAlloc<bmg::TailPlan<T>>(1);
+    HIPCK(hipStreamSynchronize(stream));   // no earlier leg still reads it
+    HIPCK(hipMemcpy(ts.plan, p.get(), sizeof(*p), hipMemcpyHostToDevice));
+    ts.lds = need;
+    ts.whole = whole;
+    ts.level = top;
+}
+
+template void bmg_ctx::ensureTail<double>();
+template void bmg_ctx::ensureTail<float>();
+
 // MG::cycle (MG.C:19-129).  On the coarsest level in direct mode the
 // pre-smoothing is skipped: APLU::solve overwrites every interior value and
 // reads ghosts only through eliminated (zero) couplings, so the result is the
@@ -568,6 +728,22 @@ void bmg_ctx::cycle(std::vector<int>& visits, int l, bool zeroX)
     Level& q = lv[l];
     const int lc = coarseLevel();
     record_tag(cycleTag(lc - l, false));
+    if (tailLevel<T>() == l)
+    {
+        // this level and the coarser ones in one workgroup: one launch with
+        // the coarse inverse, else the coarse solve between its two halves
+        const TailState<T>& ts = tail<T>();
+        if (ts.whole)
+            launch_tail<T>(ts.plan, ts.lds, 0, stream);
+        else
+        {
+            launch_tail<T>(ts.plan, ts.lds, 1, stream);
+            coarseSolve<T>();
+            launch_tail<T>(ts.plan, ts.lds, 2, stream);
+        }
+        for (int k = l; k <= lc; k++) visits[k]++;
+        return;
+    }
     if (singular() && l == lc)
         launch_set_cell<T>(B<T>(l), ((long)1*q.L.P[1] + 1)*q.L.Hz + 0,
                            (1 + 1 + 1) & 1, T(0), stream);
@@ -975,6 +1151,7 @@ void bmg_ctx::enqueueIteration(bool mixed)
 // Runs one iteration and returns the sum of squared level-0 residuals.
 double bmg_ctx::iterate(bool mixed)
 {
+    mixed ? ensureTail<float>() : ensureTail<double>();
     if (useGraphs)
     {
         ensureSmootherBuffers(mixed);
@@ -1137,6 +1314,7 @@ void bmg_ctx::prepareLearned()
 
 void bmg_ctx::fcgIteration(int mode)
 {
+    if (mode != 2) mode == 1 ? ensureTail<float>() : ensureTail<double>();
     if (!useGraphs)
     {
         enqueueFCGIteration(mode);
@@ -1171,6 +1349,7 @@ void bmg_ctx::fcgIteration(int mode)
 
 void bmg_ctx::precondition(bool mixed)
 {
+    mixed ? ensureTail<float>() : ensureTail<double>();
     if (!useGraphs)
     {
         enqueuePrecondition(mixed);
@@ -1623,7 +1802,10 @@ void bmg_ctx::runFCG(bool constMatrix, bmg_stats* st)
                     if (deflating()) enqueueDeflate();
                 }
                 else
+                {
+                    mixed ? ensureTail<float>() : ensureTail<double>();
                     enqueueFCGRestart(mixed);
+                }
             }
             restart = false;
         }

@@ -13,6 +13,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 namespace bmg {
@@ -253,6 +254,32 @@ struct bmg_ctx
     // 1 on levels whose launch has at least 256 workgroups, 2 on every level
     // whose rows fit the LDS ring
     int fuseSmoothing = 0;
+    // one-workgroup leg of the small levels (launch_tail): its device plan,
+    // valid while gen is the context's; level -1: none
+    template <typename T>
+    struct TailState
+    {
+        bmg::TailPlan<T>* plan = nullptr;
+        long gen = -1;
+        int level = -1;
+        size_t lds = 0;
+        bool whole = false;   // with the coarse solve inside
+    };
+    TailState<double> tailD;
+    TailState<float> tailF;
+    template <typename T>
+    TailState<T>& tail()
+    {
+        if constexpr (std::is_same<T, float>::value) return tailF;
+        else return tailD;
+    }
+    // the level whose cycle the tail runs, -1: none
+    template <typename T>
+    int tailLevel()
+    {
+        const TailState<T>& t = tail<T>();
+        return t.gen == gen ? t.level : -1;
+    }
     // cycles on periodic levels: 1 (default) red-black phases over the
     // whole interior that keep the periodic ghosts current (wrapAxes) in the
     // FP32 cycles, 2 in the FP64 ones too, 0 nowhere (the reference's
@@ -315,6 +342,8 @@ struct bmg_ctx
         devFree(dLU);
         devFree(dPiv);
         devFree(dCoarseInv);
+        devFree(tailD.plan);
+        devFree(tailF.plan);
         devFree(partials);
         devFree(dScalar);
         if (hScalar) (void)hipHostFree(hScalar);
@@ -400,6 +429,11 @@ struct bmg_ctx
     bool fusedLevel(int l) const;
     template <typename T>
     void smoothFused(int l, int sweeps);
+    template <typename T>
+    int tailSteps(int l, int sweeps, bool zeroStart,
+                  bmg::TailStep* out) const;
+    template <typename T>
+    void ensureTail();
     // buffers the smoothers use, allocated before any graph capture
     void ensureSmootherBuffers(bool mixed);
     // deflation of flexible CG

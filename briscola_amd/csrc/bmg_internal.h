@@ -176,6 +176,53 @@ void launch_rbgs_fill(const LevelDims& L, const OpView<T>& op, Pair<T> x,
                       Pair<const T> b, int colour, const Region& rg,
                       int level0, const BcData* bcval, T* const (*snap)[2],
                       hipStream_t s);
+// ---- the small levels of a V-cycle in one workgroup (k_tail) ----
+// Levels from the first of at most TAIL_CELLS cells down to the coarsest,
+// each refined by 2 on every axis and stored as stencils.  The plan lives in
+// device memory; a smoothing call is a list of steps.
+enum { TAIL_LEVELS = 8, TAIL_STEPS = 64 };
+constexpr long TAIL_CELLS = 4096;
+// Steps of a smoothing call: a phase over the interior, the periodic face
+// ghosts, a phase of one or both boundary planes normal to an axis.
+enum { TAIL_PHASE = 0, TAIL_GHOSTS = 1, TAIL_SLAB = 2 };
+struct TailStep {
+    unsigned char type;
+    unsigned char axis;
+    signed char c0, c1;   // colour (of the planes 1 and N; -1: not swept)
+};
+// A level in LDS: row and plane pitch of x, and ceil(2^32/d) of P1, P2, N1.
+struct TailDims : LevelDims {
+    int pJ, pI;
+    unsigned mP1, mP2, mN1;
+};
+template <typename T>
+struct TailLevel {
+    TailDims L;
+    const T* a7[2];
+    T* x[2];
+    T* b[2];
+    TransferView<T> tv;   // to the next coarser level
+    int wrap;             // Region::wrap of the interior phases
+    int refresh;          // periodic ghosts refreshed before the residual
+    int nPre, nPost;
+    int xo, bo;           // offsets of x (padded) and b (interior) in LDS
+                          // (b not at the largest level)
+    TailStep pre[TAIL_STEPS], post[TAIL_STEPS];
+};
+template <typename T>
+struct TailPlan {
+    int nl;               // levels, the coarsest included
+    int singular;
+    int nc;               // cells of the coarsest level
+    size_t lds;           // bytes
+    const double* inv;    // its inverse (FP32 cycles), or null
+    TailLevel<T> lv[TAIL_LEVELS];
+};
+// part 0: the whole leg (needs inv); 1: down to the coarsest right-hand side
+// (x and b of the levels left in memory); 2: up from the coarsest x.
+template <typename T>
+void launch_tail(const TailPlan<T>* plan, size_t lds, int part,
+                 hipStream_t s);
 // Two consecutive red-black phases (colour c1, then 1 - c1) over rg in one
 // launch: c1 updated in place in xR, the other colour read from xBin and
 // written to xBout (a second buffer; cells outside rg copied).  Not

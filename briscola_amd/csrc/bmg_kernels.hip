@@ -3342,6 +3342,718 @@ struct KCoarseWave
 
 
 // ---------------------------------------------------------------------------
+// The small levels of a V-cycle in one workgroup: smoothing, residual,
+// restriction, coarse solve, prolongation and smoothing of every level from
+// at most TAIL_CELLS cells down.  As launches these levels are
+// bound by launch latency (3-4 us each, some 25 of them); here x of every
+// level stays in LDS (plain padded layout, K fastest) and a step costs its
+// LDS latency and a barrier.  Thread pair h owns the 2x2x2 block h of a
+// level, thread a of the pair its plane I = 2bi+1+a: two cells of each
+// colour, their coefficients and b in registers for the level's whole leg,
+// and the block's eight residuals, which are the restriction's, in the pair.
+// Per-cell arithmetic is that of the launches (gs_update, pair_Ax's sum,
+// restrict_impl, prolong8_impl, coarse_inv_body), so results keep their
+// bits.  Measured at 16^3, 8^3, 4^3 in FP32: 41 us, of which the phases 13,
+// the first loads of coefficients 6, the coarse product 3, against about
+// 110 us of launches and gaps; in FP64, whose 16^3 phases one compute unit
+// runs no faster than a launch does, 35 + 16 + 33 us (down, coarse, up)
+// against 125 us.  Pitches that put the lanes of a half wavefront into
+// different banks, masks in place of index tests and the kernel's plan in
+// scalar loads took the FP32 leg from 61 to 41 us.
+constexpr int TAIL_NT = 1024;   // threads, one half each
+
+template <typename T>
+struct TailOwn
+{
+    T a[2][2][7];     // [colour][j]
+    T b[2][2];
+};
+
+// Position of this thread's half; false past the level's blocks.
+struct TailPos
+{
+    int I, J0, K0;        // plane, first row and cell
+    int bi, bj, bk;
+};
+
+__device__ __forceinline__ bool tail_pos(const TailDims& L, TailPos& q)
+{
+    const int t = int(threadIdx.x);
+    const int h = t >> 1;
+    const int n1 = L.N[1] >> 1, n2 = L.N[2] >> 1;
+    q.bk = h % n2;
+    const int r = h/n2;
+    q.bj = r % n1;
+    q.bi = r/n1;
+    q.I = 2*q.bi + 1 + (t & 1);
+    q.J0 = 2*q.bj + 1;
+    q.K0 = 2*q.bk + 1;
+    return q.bi < (L.N[0] >> 1);
+}
+
+// Cell of colour c in row J0 + j of a half.
+__device__ __forceinline__ int tail_k(const TailPos& q, int c, int j)
+{
+    return q.K0 + ((c - q.I - q.J0 - j - q.K0) & 1);
+}
+
+__device__ __forceinline__ int tail_x(const TailDims& L, int I, int J, int K)
+{
+    return I*L.pI + J*L.pJ + K;
+}
+
+// A thread's cells for a leg's steps, computed once: every step runs in all
+// 16 wavefronts, so its integer work counts (an instruction is about 7 ns of
+// the workgroup).  mask: bits e = 2c + j of the interior region, then of the
+// planes 1 and N of each axis (4 + 4(2d + side) + e).
+struct TailCells
+{
+    int i;            // LDS index of (I, J0, K0)
+    int par;          // its colour
+    unsigned mask;
+    int on;           // the half exists
+};
+
+__device__ __forceinline__ void tail_cells_of(const TailDims& L, int wrap,
+                                              TailCells& q)
+{
+    TailPos p;
+    const bool on = tail_pos(L, p);
+    q.i = tail_x(L, p.I, p.J0, p.K0);
+    q.par = (p.I + p.J0 + p.K0) & 1;
+    unsigned m = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+    {
+        const int g[3] = {p.I, p.J0 + (e & 1), tail_k(p, e >> 1, e & 1)};
+        bool in = true;
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+        {
+            // padded on periodic faces unless they wrap
+            const int pad = !wrap && L.bc[2*d] == PER ? 1 : 0;
+            in = in && g[d] >= 1 + pad && g[d] <= L.N[d] - pad;
+            if (g[d] == 1) m |= 1u << (4 + 8*d + e);
+            if (g[d] == L.N[d]) m |= 1u << (8 + 8*d + e);
+        }
+        if (in) m |= 1u << e;
+    }
+    q.mask = on ? m : 0u;
+    q.on = on;
+}
+
+// LDS index of the thread's cell of colour c in row j.
+__device__ __forceinline__ int tail_i(const TailDims& L,
+                                      const TailCells& q, int c,
+                                      int j)
+{
+    return q.i + j*L.pJ + ((c ^ q.par ^ j) & 1);
+}
+
+template <typename T>
+__device__ __forceinline__ void tail_load(const TailDims& L,
+                                          const TailLevel<T>& lv, const T* bl,
+                                          TailOwn<T>& o)
+{
+    TailPos q;
+    if (!tail_pos(L, q)) return;
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+    {
+        const int K = tail_k(q, c, j);
+        const unsigned i = unsigned(cidx(L, q.I, q.J0 + j, K));
+#pragma unroll
+        for (int s = 0; s < 7; s++)
+            o.a[c][j][s] = ld(lv.a7[c], unsigned(s*nci(L)) + i);
+        o.b[c][j] = bl ? bl[((q.I - 1)*L.N[1] + q.J0 + j - 1)*L.N[2] +
+                               K - 1]
+                          : ld(static_cast<const T*>(lv.b[c]), i);
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void tail_nb(const TailDims& L, const T* X, int i,
+                                        T nb[6])
+{
+    const int sJ = L.pJ, sI = L.pI;
+    nb[0] = X[i - sI];
+    nb[1] = X[i + sI];
+    nb[2] = X[i - sJ];
+    nb[3] = X[i + sJ];
+    nb[4] = X[i - 1];
+    nb[5] = X[i + 1];
+}
+
+// Copies of a boundary cell's value into the periodic face ghosts of the
+// axes in `axes` that mirror it (m: the thread's mask, e: the cell).
+template <typename T>
+__device__ __forceinline__ void tail_images(const TailDims& L, T* X, int i,
+                                            unsigned m, int e, int axes, T v)
+{
+    const int st[3] = {L.pI, L.pJ, 1};
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+        if (axes & (1 << d))
+        {
+            if (m & (1u << (4 + 8*d + e))) X[i + L.N[d]*st[d]] = v;
+            if (m & (1u << (8 + 8*d + e))) X[i - L.N[d]*st[d]] = v;
+        }
+}
+
+// Updates this thread's cells of colour C among `bits` (2 per half: rows).
+template <typename T, int C>
+__device__ __forceinline__ void tail_update(const TailDims& L, T* X,
+                                            const TailOwn<T>& o,
+                                            const TailCells& q,
+                                            unsigned bits,
+                                            int wrap)
+{
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+    {
+        if (!(bits & (1u << (2*C + j)))) continue;
+        int i = tail_i(L, q, C, j);
+        // the neighbours' addresses formed here, not kept across the steps:
+        // with the coefficients they exceed 128 registers
+        asm volatile("" : "+v"(i));
+        T nb[6];
+        tail_nb(L, X, i, nb);
+        const T v = gs_update<T>(o.a[C][j], nb, o.b[C][j]);
+        X[i] = v;
+        if (wrap) tail_images(L, X, i, q.mask, 2*C + j, wrap, v);
+    }
+}
+
+// Every ghost of x in LDS (ghost_cell's rules of mode 1 without boundary
+// values, which only level 0 has).
+template <typename T>
+__device__ __forceinline__ void tail_ghosts(const TailDims& L, T* X)
+{
+    const unsigned mP2 = L.mP2, mN1 = L.mN1;
+    const int P0 = L.P[0], P1 = L.P[1], P2 = L.P[2];
+    const int nA = 2*P1*P2, nB = 2*(P0 - 2)*P2, nC = 2*(P0 - 2)*(P1 - 2);
+    for (int t = int(threadIdx.x); t < nA + nB + nC; t += TAIL_NT)
+    {
+        int g[3];
+        if (t < nA)
+        {
+            const int side = t >= P1*P2;
+            const int v = t - (side ? P1*P2 : 0);
+            g[0] = side ? P0 - 1 : 0;
+            g[1] = int(__umulhi(unsigned(v), mP2));
+            g[2] = v - g[1]*P2;
+        }
+        else if (t < nA + nB)
+        {
+            const int w = t - nA, half = (P0 - 2)*P2;
+            const int side = w >= half;
+            const int v = w - (side ? half : 0);
+            const int i = int(__umulhi(unsigned(v), mP2));
+            g[0] = 1 + i;
+            g[1] = side ? P1 - 1 : 0;
+            g[2] = v - i*P2;
+        }
+        else
+        {
+            const int w = t - nA - nB, half = (P0 - 2)*(P1 - 2);
+            const int side = w >= half;
+            const int v = w - (side ? half : 0);
+            const int i = int(__umulhi(unsigned(v), mN1));
+            g[0] = 1 + i;
+            g[1] = 1 + v - i*(P1 - 2);
+            g[2] = side ? P2 - 1 : 0;
+        }
+        int nout = 0;
+        bool allPer = true, neu = true;
+        int s[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+        {
+            const int bo = g[d] == 0 ? -1 : (g[d] == L.P[d] - 1 ? 1 : 0);
+            const int bcf = bo > 0 ? L.bc[2*d + 1] : L.bc[2*d];
+            if (bo != 0)
+            {
+                nout++;
+                if (bcf != PER) allPer = false;
+                if (bcf != NEU) neu = false;
+            }
+            s[d] = bo;
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            s[d] = g[d] - (allPer ? s[d]*L.N[d] : s[d]);
+        const T xi = X[tail_x(L, s[0], s[1], s[2])];
+        T v = xi;
+        if (nout == 1 && !allPer) v = neu ? xi + T(0) : T(0) - xi;
+        X[tail_x(L, g[0], g[1], g[2])] = v;
+    }
+}
+
+// The steps of a smoothing call, one per lane (loaded with the leg's other
+// data, read back by lane so that no step waits for memory).
+__device__ __forceinline__ int tail_program(const TailStep* st)
+{
+    static_assert(sizeof(TailStep) == 4 && TAIL_STEPS == 64, "");
+    return reinterpret_cast<const int*>(st)[threadIdx.x & 63];
+}
+
+// The periodic face ghosts, each written by the owner of its cell.
+template <typename T>
+__device__ __forceinline__ void tail_periodic(const TailDims& L, T* X,
+                                              const TailCells& q)
+{
+    const int axes = (L.bc[0] == PER ? 1 : 0) | (L.bc[2] == PER ? 2 : 0) |
+                     (L.bc[4] == PER ? 4 : 0);
+    if (q.mask >> 4)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+        {
+            const int i = tail_i(L, q, e >> 1, e & 1);
+            tail_images(L, X, i, q.mask, e, axes, X[i]);
+        }
+}
+
+template <typename T>
+__device__ __forceinline__ void tail_steps(const TailDims& L, int wrap,
+                                           int program, int n, T* X,
+                                           const TailOwn<T>& o,
+                                           const TailCells& q)
+{
+    for (int k = 0; k < n; k++)
+    {
+        const int w = __builtin_amdgcn_readlane(program, k);
+        const int type = w & 0xff, axis = (w >> 8) & 0xff;
+        const int c0 = (w << 8) >> 24, c1 = w >> 24;
+        if (type == TAIL_GHOSTS)
+            tail_periodic<T>(L, X, q);
+        else
+        {
+            // the cells of the step: of the interior, or of one colour on
+            // each of the two boundary planes
+            const unsigned lo = c0 < 0 ? 0u : 3u << (2*c0);
+            const unsigned hi = c1 < 0 ? 0u : 3u << (2*c1);
+            const unsigned bits = type == TAIL_PHASE
+                                      ? q.mask & lo
+                                      : ((q.mask >> (4 + 8*axis)) & lo) |
+                                            ((q.mask >> (8 + 8*axis)) & hi);
+            const int wr = type == TAIL_PHASE ? wrap : 0;
+            if (c0 == 0 || c1 == 0)
+                tail_update<T, 0>(L, X, o, q, bits, wr);
+            if (c0 == 1 || c1 == 1)
+                tail_update<T, 1>(L, X, o, q, bits, wr);
+        }
+        __syncthreads();
+    }
+}
+
+// Transfer data of a thread's blocks.
+template <typename T>
+struct TailDown
+{
+    T vf[3][2], u[3], cw[3];
+};
+
+template <typename T>
+__device__ __forceinline__ void tail_weights(const TailDims& L,
+                                             const TransferView<T>& tv,
+                                             TailDown<T>& w)
+{
+    TailPos q;
+    if (!tail_pos(L, q)) return;
+    const int c[3] = {q.bi + 1, q.bj + 1, q.bk + 1};
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+    {
+        w.vf[d][0] = tv.fw[d][2*c[d] - 1];
+        w.vf[d][1] = tv.fw[d][2*c[d]];
+        w.u[d] = tv.ru[d][c[d]];
+        w.cw[d] = tv.cw[d][c[d]];
+    }
+}
+
+template <typename T>
+struct TailUp
+{
+    T x, y[2], z[2];
+};
+
+template <typename T>
+__device__ __forceinline__ void tail_fractions(const TailDims& L,
+                                               const TransferView<T>& tv,
+                                               TailUp<T>& w)
+{
+    TailPos q;
+    if (!tail_pos(L, q)) return;
+    w.x = tv.pu[0][q.I];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+    {
+        w.y[k] = tv.pu[1][q.J0 + k];
+        w.z[k] = tv.pu[2][q.K0 + k];
+    }
+}
+
+// Residual of the level and its restriction: b of the next level into LDS
+// (and memory when gb is set).
+template <typename T>
+__device__ __forceinline__ void tail_restrict(const TailDims& L,
+                                              const TailLevel<T>& lc,
+                                              const T* X, T* bl, bool gb,
+                                              const TailOwn<T>& o,
+                                              const TailCells& q,
+                                              const TailDown<T>& wt)
+{
+    const TailDims C = lc.L;
+    const bool on = q.on != 0;
+    T r[2][2] = {{T(0), T(0)}, {T(0), T(0)}};   // [colour][j]
+    if (on)
+    {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+        {
+            const int i = tail_i(L, q, c, j);
+            const T* a = o.a[c][j];
+            T nb[6];
+            tail_nb(L, X, i, nb);
+            const T ax = a[0]*X[i] + a[1]*nb[0] + a[2]*nb[1] + a[3]*nb[2]
+                       + a[4]*nb[3] + a[5]*nb[4] + a[6]*nb[5];
+            r[c][j] = o.b[c][j] - ax;
+        }
+    }
+    // rr[cz][cy][cx]: own plane and the other thread's
+    const int me = int(threadIdx.x) & 1;
+    T rr[2][2][2];
+#pragma unroll
+    for (int cy = 0; cy < 2; cy++)
+    {
+        const int c0 = (q.par ^ cy) & 1;   // colour at cz = 0
+        const T z0 = c0 ? r[1][cy] : r[0][cy];
+        const T z1 = c0 ? r[0][cy] : r[1][cy];
+        const T w0 = __shfl_xor(z0, 1, 64), w1 = __shfl_xor(z1, 1, 64);
+        rr[0][cy][0] = me ? w0 : z0;
+        rr[0][cy][1] = me ? z0 : w0;
+        rr[1][cy][0] = me ? w1 : z1;
+        rr[1][cy][1] = me ? z1 : w1;
+    }
+    if (!on || me) return;
+    TailPos p;
+    tail_pos(L, p);
+    const int I = p.bi + 1, J = p.bj + 1, K = p.bk + 1;
+    const T ux = wt.u[0], uy = wt.u[1], uz = wt.u[2];
+    const T fx[2] = {T(1.0) - ux, ux};
+    const T fy[2] = {T(1.0) - uy, uy};
+    const T fz[2] = {T(1.0) - uz, uz};
+    T sum = T(0);
+#pragma unroll
+    for (int cz = 0; cz < 2; cz++)
+#pragma unroll
+    for (int cy = 0; cy < 2; cy++)
+#pragma unroll
+    for (int cx = 0; cx < 2; cx++)
+    {
+        T w = fx[cx]*fy[cy];
+        w = w*fz[cz];
+        if (w <= T(1e-12)) w = T(0);
+        T cvf = wt.vf[0][cx]*wt.vf[1][cy];
+        cvf = cvf*wt.vf[2][cz];
+        cvf = cvf > T(1e-16) ? cvf : T(1e-16);
+        const T icvf = recip(cvf);
+        const T t = w*rr[cz][cy][cx];
+        const T next = madd(t, icvf, sum);
+        sum = w != T(0) ? next : sum;
+    }
+    T cvc = wt.cw[0]*wt.cw[1];
+    cvc = cvc*wt.cw[2];
+    cvc = cvc > T(1e-16) ? cvc : T(1e-16);
+    const T out = sum*cvc;
+    bl[((I - 1)*C.N[1] + J - 1)*C.N[2] + K - 1] = out;
+    if (gb)
+    {
+        const int c = (I + J + K) & 1;
+        st(lc.b[c], unsigned(cidx(C, I, J, K)), out);
+    }
+}
+
+// x += the prolongation of the next level's x (its ghosts current).
+template <typename T>
+__device__ __forceinline__ void tail_prolong(const TailDims& L,
+                                             const TailDims& C, T* X,
+                                             const T* Xc,
+                                             const TailUp<T>& w)
+{
+    TailPos q;
+    if (!tail_pos(L, q)) return;
+    const int a = q.I & 1 ? 0 : 1;
+    const int ci = q.bi + 1, cj = q.bj + 1, ck = q.bk + 1;
+    const int cx[2] = {ci, ci + (a ? 1 : -1)};   // parent, neighbour
+    T cv[2][3][3];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+    for (int y = 0; y < 3; y++)
+#pragma unroll
+    for (int z = 0; z < 3; z++)
+        cv[x][y][z] = Xc[tail_x(C, cx[x], cj - 1 + y, ck - 1 + z)];
+#pragma unroll
+    for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+    {
+        const int sy[2] = {1, b ? 2 : 0};
+        const int sz[2] = {1, c ? 2 : 0};
+        T u0 = w.x, u1 = w.y[b], u2 = w.z[c];
+        const bool inside = !(u0 < T(0) || u0 >= T(1) || u1 < T(0) ||
+                              u1 >= T(1) || u2 < T(0) || u2 >= T(1));
+        if (!inside) { u0 = T(0.5); u1 = T(0.5); u2 = T(0.5); }
+        T value = T(0);
+        if constexpr (std::is_same<T, float>::value)
+        {
+            float ry[2];
+#pragma unroll
+            for (int cz = 0; cz < 2; cz++)
+            {
+                float rx[2];
+#pragma unroll
+                for (int cy = 0; cy < 2; cy++)
+                {
+                    const float v0 = cv[0][sy[cy]][sz[cz]];
+                    const float v1 = cv[1][sy[cy]][sz[cz]];
+                    rx[cy] = __builtin_fmaf(u0, v1 - v0, v0);
+                }
+                ry[cz] = __builtin_fmaf(u1, rx[1] - rx[0], rx[0]);
+            }
+            value = __builtin_fmaf(u2, ry[1] - ry[0], ry[0]);
+        }
+        else
+        {
+            const T gx[2] = {T(1.0) - u0, u0};
+            const T gy[2] = {T(1.0) - u1, u1};
+            const T gz[2] = {T(1.0) - u2, u2};
+#pragma unroll
+            for (int cz = 0; cz < 2; cz++)
+#pragma unroll
+            for (int cy = 0; cy < 2; cy++)
+#pragma unroll
+            for (int cxx = 0; cxx < 2; cxx++)
+            {
+                T g = gx[cxx]*gy[cy];
+                g = g*gz[cz];
+                const T t = g*cv[cxx][sy[cy]][sz[cz]];
+                value = value + t;
+            }
+        }
+        const int i = tail_x(L, q.I, q.J0 + b, q.K0 + c);
+        X[i] = X[i] + value;
+    }
+}
+
+// x of a level between LDS and memory: the padded block out, the interior in
+// (its ghosts 0, as every smoothing call reads none it has not refreshed,
+// but through zero couplings).
+template <typename T>
+__device__ __forceinline__ void tail_store(const TailDims& L,
+                                           const TailLevel<T>& lv, const T* X)
+{
+    const int n = L.P[0]*L.P[1]*L.P[2], P1 = L.P[1], P2 = L.P[2];
+    const unsigned mP2 = L.mP2, mP1 = L.mP1;
+    T* const x0 = lv.x[0];
+    T* const x1 = lv.x[1];
+    for (int t = int(threadIdx.x); t < n; t += TAIL_NT)
+    {
+        const int row = int(__umulhi(unsigned(t), mP2));   // I*P1 + J
+        const int I = int(__umulhi(unsigned(row), mP1));
+        const int J = row - I*P1, K = t - row*P2;
+        st((I + J + K) & 1 ? x1 : x0, unsigned(row*L.Hz + (K >> 1)),
+           X[tail_x(L, I, J, K)]);
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ void tail_fetch(const TailDims& L,
+                                           const TailLevel<T>& lv, T* X)
+{
+    const int n = L.P[0]*L.P[1]*L.P[2], P1 = L.P[1], P2 = L.P[2];
+    const unsigned mP2 = L.mP2, mP1 = L.mP1;
+    const T* const x0 = lv.x[0];
+    const T* const x1 = lv.x[1];
+    for (int t = int(threadIdx.x); t < n; t += TAIL_NT)
+    {
+        const int row = int(__umulhi(unsigned(t), mP2));
+        const int I = int(__umulhi(unsigned(row), mP1));
+        const int J = row - I*P1, K = t - row*P2;
+        const bool in = I >= 1 && I <= L.N[0] && J >= 1 && J <= L.N[1] &&
+                        K >= 1 && K <= L.N[2];
+        X[tail_x(L, I, J, K)] =
+            in ? ld((I + J + K) & 1 ? x1 : x0,
+                       unsigned(row*L.Hz + (K >> 1)))
+                  : T(0);
+    }
+}
+
+template <typename T, int PART>
+__device__ __forceinline__ void tail_body(const TailPlan<T>* __restrict__ plan,
+                                          T* lds)
+{
+    const TailPlan<T>& P = *plan;
+    const int tid = int(threadIdx.x);
+    const int lc = P.nl - 1;
+    const TailLevel<T>& Cl = P.lv[lc];
+    const TailDims C = Cl.L;
+    T* Xc = lds + Cl.xo;
+    // the restriction's weights held through the smoothing steps where
+    // registers allow
+    constexpr bool EARLY = sizeof(T) == 4;
+    // the largest level's coefficients, kept for its way up
+    TailOwn<T> top;
+    if constexpr (PART != 2)
+    {
+        for (int l = 0; l < lc; l++)
+        {
+            const TailLevel<T>& lv = P.lv[l];
+            const TailDims L = lv.L;
+            T* X = lds + lv.xo;
+            const int n = L.P[0]*L.pI;
+            const int program = tail_program(lv.pre), steps = lv.nPre;
+            const int wrap = lv.wrap, refresh = lv.refresh;
+            TailOwn<T> o;
+            TailDown<T> w;
+            TailCells q;
+            tail_load<T>(L, lv, l > 0 ? lds + lv.bo : nullptr, o);
+            if (PART == 0 && l == 0) top = o;
+            if constexpr (EARLY) tail_weights<T>(L, lv.tv, w);
+            tail_cells_of(L, wrap, q);
+            for (int t = tid; t < n; t += TAIL_NT) X[t] = T(0);
+            __syncthreads();
+            tail_steps<T>(L, wrap, program, steps, X, o, q);
+            if constexpr (!EARLY) tail_weights<T>(L, lv.tv, w);
+            if (refresh)
+            {
+                tail_periodic<T>(L, X, q);
+                __syncthreads();
+            }
+            tail_restrict<T>(L, P.lv[l + 1], X, lds + P.lv[l + 1].bo,
+                                 PART == 1, o, q, w);
+            if constexpr (PART == 1) tail_store<T>(L, lv, X);
+            __syncthreads();
+        }
+    }
+    if constexpr (PART == 1)
+    {
+        if (P.singular && tid == 0)
+            st(Cl.b[1], unsigned(cidx(C, 1, 1, 1)), T(0));
+        // the coarse solve reads ghosts of x, through zero couplings
+        const int n = C.P[0]*C.pI;
+        for (int t = tid; t < n; t += TAIL_NT) Xc[t] = T(0);
+        __syncthreads();
+        tail_store<T>(C, Cl, Xc);
+        return;
+    }
+    if constexpr (PART == 0)
+    {
+        // the coarse system by its inverse, as coarse_inv_body; four rows of
+        // a wavefront in flight
+        const T* bl = lds + Cl.bo;
+        const int lane = tid & 63;
+        const int N1 = C.N[1], N2 = C.N[2];
+        const int nc = P.nc;
+        const bool pin = P.singular != 0;
+        const double* inv = P.inv;
+        constexpr int NW = TAIL_NT/64;
+        for (int r0 = tid >> 6; r0 < nc; r0 += 4*NW)
+        {
+            double y[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int q = lane; q < nc; q += 64)
+            {
+                const double v = double(pin && q == 0 ? T(0) : bl[q]);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                {
+                    const int row = min(r0 + NW*k, nc - 1);
+                    y[k] = __builtin_fma(inv[size_t(row)*nc + q], v, y[k]);
+                }
+            }
+            for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+                for (int k = 0; k < 4; k++) y[k] += __shfl_xor(y[k], o, 64);
+            // lane k writes row k of the four
+            const double out = lane == 0 ? y[0] : (lane == 1 ? y[1]
+                                           : (lane == 2 ? y[2] : y[3]));
+            const int row = r0 + NW*lane;
+            if (lane < 4 && row < nc)
+                Xc[tail_x(C, 1 + row/(N1*N2), 1 + (row/N2) % N1,
+                          1 + row % N2)] = T(out);
+        }
+    }
+    else
+    {
+        for (int l = 0; l <= lc; l++)
+            tail_fetch<T>(P.lv[l].L, P.lv[l], lds + P.lv[l].xo);
+    }
+    __syncthreads();
+    for (int l = lc - 1; l >= 0; l--)
+    {
+        const TailLevel<T>& lv = P.lv[l];
+        const TailLevel<T>& ln = P.lv[l + 1];
+        const TailDims L = lv.L, Ln = ln.L;
+        T* X = lds + lv.xo;
+        T* Xn = lds + ln.xo;
+        const int program = tail_program(lv.post), steps = lv.nPost;
+        const int wrap = lv.wrap;
+        TailOwn<T> o;
+        TailUp<T> w;
+        TailCells q;
+        if (PART == 0 && l == 0)
+            o = top;
+        else
+            tail_load<T>(L, lv, PART == 0 ? lds + lv.bo : nullptr, o);
+        tail_fractions<T>(L, lv.tv, w);
+        tail_ghosts<T>(Ln, Xn);
+        tail_cells_of(L, wrap, q);
+        __syncthreads();
+        tail_prolong<T>(L, Ln, X, Xn, w);
+        __syncthreads();
+        tail_steps<T>(L, wrap, program, steps, X, o, q);
+    }
+    const TailLevel<T>& lv = P.lv[0];
+    const TailDims L = lv.L;
+    tail_ghosts<T>(L, lds + lv.xo);
+    __syncthreads();
+    tail_store<T>(L, lv, lds + lv.xo);
+}
+
+template <typename T, int PART>
+__global__ __launch_bounds__(TAIL_NT) void k_tail(
+    const TailPlan<T>* __restrict__ plan)
+{
+    extern __shared__ __align__(16) unsigned char tail_lds[];
+    tail_body<T, PART>(plan, reinterpret_cast<T*>(tail_lds));
+}
+
+template <typename T, int PART>
+struct KTail
+{
+    static constexpr int bx = TAIL_NT, by = 1;
+    static constexpr bool lds = true;
+    struct Args
+    {
+        const TailPlan<T>* plan;
+    };
+    __device__ static void run(const Bid, const Args& a)
+    {
+        extern __shared__ __align__(16) unsigned char tail_lds[];
+        tail_body<T, PART>(a.plan, reinterpret_cast<T*>(tail_lds));
+    }
+    static void launch(dim3 g, size_t shm, hipStream_t s, const Args& a)
+    {
+        hipLaunchKernelGGL((k_tail<T, PART>), g, dim3(bx), shm, s, a.plan);
+    }
+};
+
+// ---------------------------------------------------------------------------
 // Reductions over interior cells (per-block partials, fixed order).
 template <typename T, int MODE>
 __device__ __forceinline__ void reduce_field_body(const Bid bid,
@@ -5506,6 +6218,21 @@ void launch_coarse_inv(const LevelDims& L, const OpView<T>& op, Pair<T> x,
                             {L, op, x, b, inv, n, level0, bcvals(bcval)});
 }
 
+template <typename T>
+void launch_tail(const TailPlan<T>* plan, size_t lds, int part, hipStream_t s)
+{
+    if constexpr (sizeof(T) == 4)
+        if (part == 0)
+        {
+            dispatch<KTail<T, 0>>(dim3(1), lds, s, {plan});
+            return;
+        }
+    if (part == 1)
+        dispatch<KTail<T, 1>>(dim3(1), lds, s, {plan});
+    else
+        dispatch<KTail<T, 2>>(dim3(1), lds, s, {plan});
+}
+
 void launch_lu_inverse(const double* lu, const int* perm, int n, double* inv,
                        hipStream_t s)
 {
@@ -5860,6 +6587,8 @@ void launch_set_cell(Pair<T> f, long idx, int colour, T v, hipStream_t s)
     template void launch_zero_phase<T>(const LevelDims&, const OpView<T>&,    \
                                        Pair<T>, Pair<const T>, int,           \
                                        const Region&, hipStream_t);           \
+    template void launch_tail<T>(const TailPlan<T>*, size_t, int,             \
+                                 hipStream_t);                                \
     template void launch_coarse_inv<T>(const LevelDims&, const OpView<T>&,    \
                                        Pair<T>, Pair<const T>, const double*, \
                                        int, int, const BcData*, hipStream_t); \

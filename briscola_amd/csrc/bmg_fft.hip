@@ -5,25 +5,38 @@
 //
 // Steps (one stream, no host synchronisation inside a solve):
 //   1. right-hand side -b minus the boundary terms of the boundary cells
-//      (FFTPoissonSolver.C:123-180), scattered into a complex array E[s][a][c]
-//      (s the tridiagonal axis, a and c the transformed axes); a Neumann or
-//      Dirichlet transformed axis is extended to 2N by even or odd
-//      reflection, so that one complex FFT of the extension gives the
-//      DCT-II / DST-II (FFTW REDFT10 / RODFT10) after a twiddle, and a
-//      Dirichlet-Neumann or Neumann-Dirichlet axis to 4N by the quarter-wave
-//      reflections, whose FFT gives the DST-IV / DCT-IV (RODFT11 / REDFT11)
-//      at the odd positions;
+//      (FFTPoissonSolver.C:123-180), two neighbouring planes of the
+//      tridiagonal axis s as the real and imaginary part of one complex
+//      plane E[s/2][a][c] (a and c the transformed axes).  Every transform
+//      is real-linear, so the pair costs one complex FFT:
+//        periodic axis: DFT;
+//        Neumann or Dirichlet pair: DCT-II (FFTW REDFT10) of the values, or
+//          DST-II (RODFT10) as the DCT-II of the values with alternating
+//          signs and the modes reversed, from the N-point FFT of the values
+//          reordered even ascending, odd descending (Makhoul 1980);
+//        Neumann-Dirichlet: DCT-IV (REDFT11) from the 2N-point FFT of the
+//          values times e^{-i pi n/2N}, zero-padded; Dirichlet-Neumann:
+//          DST-IV (RODFT11), the DCT-IV of the reversed values with
+//          alternating signs of the modes;
 //   2. one batched 2-D complex FFT over (a, c) (rocFFT);
-//   3. per wave-number pair, the twiddle and the tridiagonal solve along s
-//      with the reference's coefficients, boundary rows, pinned zero mode
-//      and, for a periodic s, its cyclic two-solve variant
-//      (tridiagonalSolver.C:14-475), into a compact mode array;
-//   4. the modes expanded back to the extended spectrum (inverse twiddle,
-//      the reflection symmetries) and one batched inverse 2-D FFT;
-//   5. the real part scaled by 1/(L_a L_c) (the reference's N or 2N per
-//      transformed axis) into x, then every ghost of x refreshed
-//      (x.correctBoundaryConditions(), FFTPoissonSolver.C:437-440).
+//   3. the modes from the spectrum (a mode and its mirror images share one
+//      thread, so every element is read once): two real numbers per complex
+//      one, X[s][k1][k2] real -- a conjugate pair of periodic modes is held
+//      as its real and its imaginary part;
+//   4. per real mode the tridiagonal solve along s with the reference's
+//      coefficients, boundary rows, pinned zero mode and, for a periodic s,
+//      its cyclic two-solve variant (tridiagonalSolver.C:14-475);
+//   5. the spectrum from the modes and one batched inverse 2-D FFT;
+//   6. its real and imaginary parts into the two planes of x, then every
+//      ghost of x refreshed (x.correctBoundaryConditions(),
+//      FFTPoissonSolver.C:437-440).
 // Every boundary pair is taken on every axis.
+//
+// All steps are bound by memory: 8 bytes per cell and array.  Against a
+// complex array per plane, extended to 2N or 4N along Neumann and Dirichlet
+// axes and solved as complex lines, the 256^3 channel went from 1660 us to
+// 592 us and a 125x90x154 box with cosine, quarter-wave and sine axes from
+// 590 us to 154 us.
 #include "bmg_context.h"
 
 #include <rocfft/rocfft.h>
@@ -45,19 +58,6 @@ int axisCode(int lo, int hi)
     return hi == DIR ? C_ND : C_NN;
 }
 
-struct FftGeom {
-    int N[3], P[3];
-    int s, d1, d2;          // tridiagonal axis, transformed axes
-    int n1, n2, ns;         // sizes along d1, d2, s
-    int L1, L2;             // transform lengths (N, 2N or 4N)
-    int code1, code2, codes;
-    int bc[6];
-    double bcval[6];
-    double hwall[6];        // width of the boundary cell of each face
-    double d1sqr, d2sqr;
-    double dT;              // deltaT*dtFrac of the time term; 0: none
-};
-
 struct C2 {
     double x, y;
 };
@@ -67,313 +67,616 @@ __device__ __forceinline__ C2 cmul(C2 a, C2 b)
     return C2{a.x*b.x - a.y*b.y, a.x*b.y + a.y*b.x};
 }
 
-// e^{i theta}
-__device__ __forceinline__ C2 cexpi(double th)
+// a times the conjugate of b
+__device__ __forceinline__ C2 cmulc(C2 a, C2 b)
 {
-    double sn, cs;
-    sincos(th, &sn, &cs);
-    return C2{cs, sn};
+    return C2{a.x*b.x + a.y*b.y, a.y*b.x - a.x*b.y};
 }
 
-__device__ __forceinline__ long refIndex(const FftGeom& g, int i, int j,
-                                         int k)
+__device__ __forceinline__ C2 cadd(C2 a, C2 b)
 {
-    return ((long)(i + 1)*g.P[1] + (j + 1))*g.P[2] + (k + 1);
+    return C2{a.x + b.x, a.y + b.y};
 }
 
-// The positions of value a of a transformed axis in its extension and their
-// signs: periodic a; Neumann-Neumann (even about -1/2 and N-1/2, period 2N)
-// a, 2N-1-a; Dirichlet-Dirichlet (odd about both) a, -(2N-1-a);
-// Neumann-Dirichlet (DCT-IV: even about -1/2, odd about N-1/2, period 4N)
-// a, -(2N-1-a), -(2N+a), 4N-1-a; Dirichlet-Neumann (DST-IV: odd about -1/2,
-// even about N-1/2) a, 2N-1-a, -(2N+a), -(4N-1-a).
-__device__ __forceinline__ int extension(int code, int n, int a, int p[4],
-                                         double w[4])
+__device__ __forceinline__ C2 csub(C2 a, C2 b)
 {
-    p[0] = a;
-    w[0] = 1.0;
-    if (code == C_PER) return 1;
-    p[1] = 2*n - 1 - a;
-    if (code == C_NN || code == C_DD)
+    return C2{a.x - b.x, a.y - b.y};
+}
+
+__device__ __forceinline__ C2 chalf(C2 a) { return C2{0.5*a.x, 0.5*a.y}; }
+
+// i a
+__device__ __forceinline__ C2 cmuli(C2 a) { return C2{-a.y, a.x}; }
+
+// A transformed axis: n values, FFT length L, and its tables (device):
+// tw[j] = e^{-i pi j/2n} (Neumann and Dirichlet pairs, j <= n/2),
+// e^{-i pi (2j+1)/4n} (quarter wave, j < n); pad[j] = e^{-i pi j/2n} (quarter
+// wave, j < n); lam[k] the eigenvalue of mode k over the squared width.
+struct FftAxis {
+    int n, L, code;
+    const C2* tw;
+    const C2* pad;
+    const double* lam;
+};
+
+struct FftGeom {
+    int N[3], P[3];
+    int s, d1, d2;          // tridiagonal axis, transformed axes
+    int ns, np;             // planes, plane pairs
+    FftAxis a1, a2;         // along d1 and d2
+    int codes;
+    int bc[6];
+    double bcval[6];
+    double hwall[6];        // width of the boundary cell of each face
+    double dT;              // deltaT*dtFrac of the time term; 0: none
+};
+
+__host__ __device__ inline bool halfWave(int code)
+{
+    return code == C_NN || code == C_DD;
+}
+
+__host__ __device__ inline bool quarterWave(int code)
+{
+    return code == C_ND || code == C_DN;
+}
+
+// Position of value a in the FFT's input and its factor.
+__device__ __forceinline__ int inputPos(const FftAxis& t, int a, C2& w)
+{
+    w = C2{1.0, 0.0};
+    if (t.code == C_PER) return a;
+    if (halfWave(t.code))
     {
-        w[1] = code == C_NN ? 1.0 : -1.0;
-        return 2;
+        if (t.code == C_DD && (a & 1)) w.x = -1.0;
+        return a & 1 ? t.n - 1 - (a >> 1) : a >> 1;
     }
-    p[2] = 2*n + a;
-    p[3] = 4*n - 1 - a;
-    const bool dct = code == C_ND;
-    w[1] = dct ? -1.0 : 1.0;
-    w[2] = -1.0;
-    w[3] = dct ? 1.0 : -1.0;
-    return 4;
+    const int q = t.code == C_DN ? t.n - 1 - a : a;
+    w = t.pad[q];
+    return q;
 }
 
-// Step 1: interior cell t of the reference layout.
-__global__ void k_fft_rhs(FftGeom g, const double* b, const double* x,
-                          const double* xold, C2* E)
+// Cell (i, j, k) of plane q along axis S, position (a, c) on the others.
+template <int S>
+__device__ __forceinline__ void cellOf(int q, int a, int c, int g[3])
 {
-    const long t = (long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (t >= (long)g.N[0]*g.N[1]*g.N[2]) return;
-    int q[3];
-    q[0] = int(t/((long)g.N[1]*g.N[2]));
-    q[1] = int((t/g.N[2]) % g.N[1]);
-    q[2] = int(t % g.N[2]);
-    const long c = refIndex(g, q[0], q[1], q[2]);
+    g[0] = S == 0 ? q : a;
+    g[1] = S == 0 ? a : (S == 1 ? q : c);
+    g[2] = S == 2 ? q : c;
+}
+
+// The thread's (a, c, pair): lanes along c, or with S = 2 (c is then not
+// the contiguous axis) 16 of c by 4 pairs, so that reads along the
+// contiguous s and writes along c both fill 64-byte lines.
+template <int S>
+__device__ __forceinline__ void cellThread(int& a, int& c, int& p)
+{
+    a = blockIdx.y;
+    if (S == 2)
+    {
+        c = blockIdx.x*16 + (threadIdx.x & 15);
+        p = blockIdx.z*16 + (threadIdx.x >> 4);
+    }
+    else
+    {
+        c = blockIdx.x*256 + threadIdx.x;
+        p = blockIdx.z;
+    }
+}
+
+// Right-hand side of the interior cell g (0-based).
+__device__ __forceinline__ double rhsValue(const FftGeom& G, const int g[3],
+                                           const double* b, const double* x,
+                                           const double* xold)
+{
+    const int sI = G.P[1]*G.P[2], sJ = G.P[2];
+    const int st[3] = {sI, sJ, 1};
+    const long c = (long)(g[0] + 1)*sI + (g[1] + 1)*sJ + (g[2] + 1);
     double f = b ? -b[c] : 0.0;
     // ddt: minus x.oldTime()/(deltaT*dtFrac) (FFTPoissonSolver.C:116-131)
-    if (xold) f = f - xold[c]/g.dT;
-    const long stride[3] = {(long)g.P[1]*g.P[2], (long)g.P[2], 1};
+    if (xold) f = f - xold[c]/G.dT;
+#pragma unroll
     for (int face = 0; face < 6; face++)
     {
         const int d = face >> 1, side = face & 1;
-        if (g.bc[face] == PER) continue;
-        if (q[d] != (side ? g.N[d] - 1 : 0)) continue;
-        const double h = g.hwall[face];
+        if (G.bc[face] == PER || g[d] != (side ? G.N[d] - 1 : 0)) continue;
+        const double h = G.hwall[face];
         const double sq = h*h;
-        const double xg = x[c + (side ? stride[d] : -stride[d])];
+        const double xg = x[c + (side ? st[d] : -st[d])];
         const double xc = x[c];
-        const double term = g.bc[face] == DIR ? (xg + xc)/sq : (xg - xc)/sq;
+        const double term = G.bc[face] == DIR ? (xg + xc)/sq : (xg - xc)/sq;
         f -= term;
     }
-    const int s = q[g.s], a = q[g.d1], cc = q[g.d2];
-    int p1[4], p2[4];
-    double w1[4], w2[4];
-    const int c1 = extension(g.code1, g.n1, a, p1, w1);
-    const int c2 = extension(g.code2, g.n2, cc, p2, w2);
-    const long base = (long)s*g.L1*g.L2;
-    for (int u = 0; u < c1; u++)
-        for (int v = 0; v < c2; v++)
-            E[base + (long)p1[u]*g.L2 + p2[v]] = C2{w1[u]*w2[v]*f, 0.0};
+    return f;
 }
 
-// Mode k of a transformed axis: its position m in the spectrum of the
-// (extended) FFT and the factor turning that FFT into the transform:
-// periodic X_k = Y_k; DCT-II X_k = e^{-i pi k/2N} Y_k; DST-II X_k =
-// i e^{-i pi (k+1)/2N} Y_{k+1}; DCT-IV X_k = 1/2 e^{-i phi} Y_{2k+1} and
-// DST-IV X_k = i/2 e^{-i phi} Y_{2k+1} with phi = pi (2k+1)/4N (the sum of
-// the four reflected copies is twice the transform).
-__device__ __forceinline__ void fwdMode(int code, int n, int k, int& m,
-                                        C2& w)
+// Step 1; the second half of a quarter-wave axis (zero) included.
+template <int S>
+__global__ __launch_bounds__(256) void k_fft_rhs(FftGeom G, const double* b,
+                                                 const double* x,
+                                                 const double* xold, C2* E)
 {
-    if (code == C_PER) { m = k; w = C2{1.0, 0.0}; return; }
-    const double pi = 3.14159265358979323846;
-    if (code == C_NN)
+    int a, c, p;
+    cellThread<S>(a, c, p);
+    if (c >= G.a2.L || p >= G.np) return;
+    C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
+    if (a >= G.a1.n || c >= G.a2.n)
     {
-        m = k;
-        w = cexpi(-pi*k/(2.0*n));
+        // only quarter-wave axes have L > n; their padding keeps its place
+        // whatever the other axis' reordering
+        Ep[(size_t)a*G.a2.L + c] = C2{0.0, 0.0};
         return;
     }
-    if (code == C_ND || code == C_DN)
+    int g[3];
+    cellOf<S>(2*p, a, c, g);
+    const double f0 = rhsValue(G, g, b, x, xold);
+    double f1 = 0.0;
+    if (2*p + 1 < G.ns)
     {
-        m = 2*k + 1;
-        const C2 e = cexpi(-pi*m/(4.0*n));
-        w = code == C_ND ? C2{0.5*e.x, 0.5*e.y} : C2{-0.5*e.y, 0.5*e.x};
+        cellOf<S>(2*p + 1, a, c, g);
+        f1 = rhsValue(G, g, b, x, xold);
+    }
+    C2 w1, w2;
+    const int p1 = inputPos(G.a1, a, w1), p2 = inputPos(G.a2, c, w2);
+    Ep[(size_t)p1*G.a2.L + p2] = cmul(cmul(w1, w2), C2{f0, f1});
+}
+
+// The elements a thread of steps 3 and 5 owns along one axis: index j and
+// its mirror image m (-1: none), and the modes they give: j itself and, for
+// a Neumann or Dirichlet pair or a periodic axis, the image.
+struct Orbit {
+    int j, m;
+};
+
+__host__ __device__ inline int orbits(const FftAxis& t)
+{
+    return quarterWave(t.code) ? t.n : t.n/2 + 1;
+}
+
+__device__ __forceinline__ Orbit orbit(const FftAxis& t, int j)
+{
+    if (quarterWave(t.code)) return Orbit{j, 2*t.n - 1 - j};
+    const int m = j == 0 ? 0 : t.n - j;
+    return Orbit{j, m == j ? -1 : m};
+}
+
+// Output index of transform index m (a Dirichlet pair's DST-II modes are
+// the DCT-II's in reverse).
+__device__ __forceinline__ int modeIndex(const FftAxis& t, int m)
+{
+    return t.code == C_DD ? t.n - 1 - m : m;
+}
+
+// Transform values of an orbit from its spectrum elements u (index j) and v
+// (index m), in place: (X_j, X_m).  j == m: u alone.
+__device__ __forceinline__ void fromSpectrum(const FftAxis& t, const Orbit& o,
+                                             C2& u, C2& v)
+{
+    if (t.code == C_PER) return;
+    if (quarterWave(t.code))
+    {
+        const C2 w = t.tw[o.j];
+        u = chalf(cadd(cmul(w, u), cmulc(v, w)));
+        if (t.code == C_DN && (o.j & 1)) u = C2{-u.x, -u.y};
         return;
     }
-    m = k + 1;
-    const C2 e = cexpi(-pi*m/(2.0*n));
-    w = C2{-e.y, e.x};   // i*e
+    const C2 w = t.tw[o.j];
+    if (o.m < 0) v = u;
+    const C2 a = cmul(w, u), b = cmulc(v, w);
+    u = chalf(cadd(a, b));
+    v = cmuli(chalf(csub(a, b)));
+}
+
+// Spectrum elements (index j, index m) of the inverse FFT's input from the
+// transform values; quarter wave: u at j, nothing at the image (the padding).
+__device__ __forceinline__ void toSpectrum(const FftAxis& t, const Orbit& o,
+                                           C2& u, C2& v)
+{
+    if (t.code == C_PER) return;
+    if (quarterWave(t.code))
+    {
+        if (t.code == C_DN && (o.j & 1)) u = C2{-u.x, -u.y};
+        u = cmulc(u, t.pad[o.j]);
+        v = C2{0.0, 0.0};
+        return;
+    }
+    if (o.j == 0) return;
+    const C2 w = t.tw[o.j];
+    if (o.m < 0) v = u;
+    const C2 iv = cmuli(v);
+    const C2 a = csub(u, iv), b = cadd(u, iv);
+    u = cmulc(a, w);
+    v = cmul(b, w);
+}
+
+// Where the two planes' values of a transform value go in X: with a periodic
+// axis the value at (k1, k2) and at its conjugate partner (the periodic
+// indices negated) are Z = A + iB and Z' = conj A + i conj B of the planes'
+// modes A and B, held as Re at one and Im at the other.
+__device__ __forceinline__ void storeModes(const FftGeom& G, double* X, int p,
+                                           int i1, int i2, double v0, double v1)
+{
+    const size_t nm = (size_t)G.a1.n*G.a2.n;
+    const size_t at = (size_t)(2*p)*nm + (size_t)i1*G.a2.n + i2;
+    X[at] = v0;
+    if (2*p + 1 < G.ns) X[at + nm] = v1;
+}
+
+__device__ __forceinline__ C2 loadModes(const FftGeom& G, const double* X,
+                                        int p, int i1, int i2)
+{
+    const size_t nm = (size_t)G.a1.n*G.a2.n;
+    const size_t at = (size_t)(2*p)*nm + (size_t)i1*G.a2.n + i2;
+    return C2{X[at], 2*p + 1 < G.ns ? X[at + nm] : 0.0};
+}
+
+// The orbits a thread owns: along axis 1 and 2 the pairs (j, image), and the
+// four combinations (j1,j2), (m1,j2), (j1,m2), (m1,m2), here e0 to e3 (held
+// one by one: an array ends up in scratch memory).
+struct OrbitPair {
+    Orbit o1, o2;
+    bool m1, m2;     // the images exist and are no repetitions
+};
+
+__device__ __forceinline__ bool orbitThread(const FftGeom& G, OrbitPair& q,
+                                            int& p)
+{
+    const int n2 = orbits(G.a2);
+    const int t = blockIdx.x*256 + threadIdx.x;
+    const int j1 = t/n2, j2 = t - j1*n2;
+    p = blockIdx.y;
+    if (j1 >= orbits(G.a1)) return false;
+    q.o1 = orbit(G.a1, j1);
+    q.o2 = orbit(G.a2, j2);
+    // index 0 is its own image
+    q.m1 = q.o1.m > 0;
+    q.m2 = q.o2.m > 0;
+    return true;
+}
+
+// A complex value and its conjugate partner -> the planes' modes, two real
+// numbers each (self: the value is its own partner).
+__device__ __forceinline__ void splitPlanes(const FftGeom& G, double* X, int p,
+                                            C2 z, int i1, int i2, C2 zp,
+                                            int k1, int k2, bool self)
+{
+    if (self)
+    {
+        storeModes(G, X, p, i1, i2, z.x, z.y);
+        return;
+    }
+    // A = (Z + conj Z')/2, B = (Z - conj Z')/2i
+    storeModes(G, X, p, i1, i2, 0.5*(z.x + zp.x), 0.5*(z.y + zp.y));
+    storeModes(G, X, p, k1, k2, 0.5*(z.y - zp.y), 0.5*(zp.x - z.x));
+}
+
+// The inverse: Z and its partner Z' from the two real numbers r and m at
+// their indices, Z = A + iB, Z' = conj A + i conj B, A = r.x + i m.x,
+// B = r.y + i m.y (self: Z alone, both real).
+__device__ __forceinline__ C2 joinFirst(C2 r, C2 m, bool self)
+{
+    return C2{self ? r.x : r.x - m.y, self ? r.y : m.x + r.y};
+}
+
+__device__ __forceinline__ C2 joinSecond(C2 r, C2 m)
+{
+    return C2{r.x + m.y, r.y - m.x};
+}
+
+// Step 3.
+__global__ __launch_bounds__(256) void k_fft_modes(FftGeom G, const C2* E,
+                                                   double* X)
+{
+    OrbitPair q;
+    int p;
+    if (!orbitThread(G, q, p)) return;
+    const C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
+    // an index without an image repeats its element
+    const int r1 = q.o1.j*G.a2.L, r1m = (q.m1 ? q.o1.m : q.o1.j)*G.a2.L;
+    const int c2 = q.o2.j, c2m = q.m2 ? q.o2.m : q.o2.j;
+    C2 e0 = Ep[r1 + c2], e1 = Ep[r1m + c2], e2 = Ep[r1 + c2m],
+       e3 = Ep[r1m + c2m];
+    fromSpectrum(G.a1, q.o1, e0, e1);
+    fromSpectrum(G.a1, q.o1, e2, e3);
+    if (halfWave(G.a2.code) && q.o2.m == 0) { e2 = e0; e3 = e1; }
+    fromSpectrum(G.a2, q.o2, e0, e2);
+    fromSpectrum(G.a2, q.o2, e1, e3);
+    const bool per1 = G.a1.code == C_PER, per2 = G.a2.code == C_PER;
+    const bool q1 = quarterWave(G.a1.code), q2 = quarterWave(G.a2.code);
+    // modes along each axis: j always; the image unless it is none, a
+    // repetition, or a quarter-wave image
+    const bool h1 = q.m1 && !q1, h2 = q.m2 && !q2;
+    const int i1 = modeIndex(G.a1, q.o1.j), i2 = modeIndex(G.a2, q.o2.j);
+    const int k1 = h1 ? modeIndex(G.a1, q.o1.m) : i1;
+    const int k2 = h2 ? modeIndex(G.a2, q.o2.m) : i2;
+    if (per1 && per2)
+    {
+        splitPlanes(G, X, p, e0, i1, i2, h1 ? (h2 ? e3 : e1) : e2, k1,
+                    k2, !h1 && !h2);
+        if (h1 && h2) splitPlanes(G, X, p, e1, k1, i2, e2, i1, k2, false);
+    }
+    else if (per1)
+    {
+        splitPlanes(G, X, p, e0, i1, i2, e1, k1, i2, !h1);
+        if (h2) splitPlanes(G, X, p, e2, i1, k2, e3, k1, k2, !h1);
+    }
+    else if (per2)
+    {
+        splitPlanes(G, X, p, e0, i1, i2, e2, i1, k2, !h2);
+        if (h1) splitPlanes(G, X, p, e1, k1, i2, e3, k1, k2, !h2);
+    }
+    else
+    {
+        storeModes(G, X, p, i1, i2, e0.x, e0.y);
+        if (h1) storeModes(G, X, p, k1, i2, e1.x, e1.y);
+        if (h2) storeModes(G, X, p, i1, k2, e2.x, e2.y);
+        if (h1 && h2) storeModes(G, X, p, k1, k2, e3.x, e3.y);
+    }
+}
+
+// Step 5; the whole extended spectrum is written.
+__global__ __launch_bounds__(256) void k_fft_spectrum(FftGeom G,
+                                                      const double* X, C2* E)
+{
+    OrbitPair q;
+    int p;
+    if (!orbitThread(G, q, p)) return;
+    C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
+    const bool per1 = G.a1.code == C_PER, per2 = G.a2.code == C_PER;
+    const bool q1 = quarterWave(G.a1.code), q2 = quarterWave(G.a2.code);
+    const bool h1 = q.m1 && !q1, h2 = q.m2 && !q2;
+    const int i1 = modeIndex(G.a1, q.o1.j), i2 = modeIndex(G.a2, q.o2.j);
+    const int k1 = h1 ? modeIndex(G.a1, q.o1.m) : i1;
+    const int k2 = h2 ? modeIndex(G.a2, q.o2.m) : i2;
+    // all four modes loaded before any branch (an index without an image
+    // repeats)
+    const C2 ii = loadModes(G, X, p, i1, i2), ki = loadModes(G, X, p, k1, i2);
+    const C2 ik = loadModes(G, X, p, i1, k2), kk = loadModes(G, X, p, k1, k2);
+    // no periodic axis: the values themselves
+    C2 e0 = ii, e1 = ki, e2 = ik, e3 = kk;
+    if (per1 && per2)
+    {
+        // partners (j1,j2)-(m1,m2) and (m1,j2)-(j1,m2); with one image
+        // missing the first alone, at whichever index has one
+        const C2 zp = joinSecond(ii, kk);
+        const bool both = h1 && h2;
+        e0 = joinFirst(ii, kk, !h1 && !h2);
+        e1 = both ? joinFirst(ki, ik, false) : zp;
+        e2 = both ? joinSecond(ki, ik) : zp;
+        e3 = zp;
+    }
+    else if (per1)
+    {
+        e0 = joinFirst(ii, ki, !h1);
+        e1 = joinSecond(ii, ki);
+        e2 = joinFirst(ik, kk, !h1);
+        e3 = joinSecond(ik, kk);
+    }
+    else if (per2)
+    {
+        e0 = joinFirst(ii, ik, !h2);
+        e2 = joinSecond(ii, ik);
+        e1 = joinFirst(ki, kk, !h2);
+        e3 = joinSecond(ki, kk);
+    }
+    toSpectrum(G.a1, q.o1, e0, e1);
+    toSpectrum(G.a1, q.o1, e2, e3);
+    toSpectrum(G.a2, q.o2, e0, e2);
+    toSpectrum(G.a2, q.o2, e1, e3);
+    const int r1 = q.o1.j*G.a2.L, r1m = q.o1.m*G.a2.L;
+    Ep[r1 + q.o2.j] = e0;
+    if (q.m1) Ep[r1m + q.o2.j] = e1;
+    if (q.m2) Ep[r1 + q.o2.m] = e2;
+    if (q.m1 && q.m2) Ep[r1m + q.o2.m] = e3;
+}
+
+// A row of the tridiagonal systems along s: couplings to the rows above and
+// below, and what its diagonal takes off the modes' eigenvalue (the boundary
+// rows as tridiagonalSolver.C:107-250).
+struct FftRow {
+    double up, down, east, west;
+};
+
+// Step 4: one thread per real mode, lanes along k2.  X: the transformed
+// right-hand side in, the solution out; R: reciprocals of the eliminated
+// diagonal; V: the cyclic auxiliary solution.  One division per row serves
+// its elimination and its back substitution.  Few wavefronts are in flight
+// (one per 64 modes), so each loads the next eight rows while it eliminates
+// eight: 256^3 256 us without that, 164 us with it (six arrays of 134 MB).
+template <bool CYC>
+__global__ __launch_bounds__(64) void k_fft_tridiag(
+    FftGeom G, double* __restrict__ X, double* __restrict__ R,
+    double* __restrict__ V, const FftRow* __restrict__ row, double pin)
+{
+    const int k2 = blockIdx.x*64 + threadIdx.x;
+    const int k1 = blockIdx.y;
+    if (k2 >= G.a2.n) return;
+    const size_t nm = (size_t)G.a1.n*G.a2.n;
+    const size_t t = (size_t)k1*G.a2.n + k2;
+    const double l1 = G.a1.lam[k1], l2 = G.a2.lam[k2];
+    const double Lm = l1 + l2;
+    // zero mode of a singular system: the first row pinned
+    const bool pinned = l1 == 0.0 && l2 == 0.0 &&
+                        (G.codes == C_NN || G.codes == C_PER);
+    const int ns = G.ns, last = ns - 1;
+    // ddt: every diagonal minus 1/(deltaT*dtFrac) (:352, :430), the pinned
+    // row included
+    const double idT = G.dT != 0.0 ? 1.0/G.dT : 0.0;
+    auto diag = [&](int k, const FftRow& w) -> double
+    {
+        const double d = pinned && k == 0 ? pin : Lm - w.east - w.west;
+        return d - idT;
+    };
+    constexpr int AH = 8;
+    constexpr int start = CYC ? 1 : 0;
+    // forward elimination (tridiagonalSolver.C:340-346)
+    double f = 0.0, r = 0.0, v = 0.0, up = 0.0;
+    double nxt[AH], cur[AH];
+    auto ahead = [&](int k0, double (&d)[AH])
+    {
+#pragma unroll
+        for (int u = 0; u < AH; u++)
+            d[u] = X[(size_t)min(k0 + u, last)*nm + t];
+    };
+    ahead(start, nxt);
+    for (int k0 = start; k0 < ns; k0 += AH)
+    {
+#pragma unroll
+        for (int u = 0; u < AH; u++) cur[u] = nxt[u];
+        if (k0 + AH < ns) ahead(k0 + AH, nxt);
+#pragma unroll
+        for (int u = 0; u < AH; u++)
+        {
+            const int k = k0 + u;
+            if (k >= ns) break;
+            const FftRow w = row[k];
+            double d = diag(k, w);
+            double fk = cur[u];
+            double vk = 0.0;
+            if (CYC) vk = k == 1 ? -w.down : (k == last ? -w.up : 0.0);
+            if (k > start)
+            {
+                const double m = w.down*r;
+                d = d - m*up;
+                fk = fk - m*f;
+                if (CYC) vk = vk - m*v;
+            }
+            r = 1.0/d;
+            f = fk;
+            v = vk;
+            up = w.up;
+            if (k < last)
+            {
+                X[(size_t)k*nm + t] = f;
+                R[(size_t)k*nm + t] = r;
+                if (CYC) V[(size_t)k*nm + t] = v;
+            }
+        }
+    }
+    // back substitution (:348-354)
+    f = f*r;
+    v = v*r;
+    X[(size_t)last*nm + t] = f;
+    if (CYC) V[(size_t)last*nm + t] = v;
+    const double uN = f, vN = v;
+    double fn[AH], rn[AH], vn[AH];
+    auto behind = [&](int k0)
+    {
+#pragma unroll
+        for (int u = 0; u < AH; u++)
+        {
+            const size_t at = (size_t)max(k0 - u, start)*nm + t;
+            fn[u] = X[at];
+            rn[u] = R[at];
+            vn[u] = CYC ? V[at] : 0.0;
+        }
+    };
+    if (ns - 2 >= start) behind(ns - 2);
+    for (int k0 = ns - 2; k0 >= start; k0 -= AH)
+    {
+        double fi[AH], ri[AH], vi[AH];
+#pragma unroll
+        for (int u = 0; u < AH; u++)
+        {
+            fi[u] = fn[u];
+            ri[u] = rn[u];
+            vi[u] = vn[u];
+        }
+        if (k0 - AH >= start) behind(k0 - AH);
+#pragma unroll
+        for (int u = 0; u < AH; u++)
+        {
+            const int k = k0 - u;
+            if (k < start) break;
+            const double c = row[k].up;
+            f = (fi[u] - c*f)*ri[u];
+            X[(size_t)k*nm + t] = f;
+            if (CYC)
+            {
+                v = (vi[u] - c*v)*ri[u];
+                V[(size_t)k*nm + t] = v;
+            }
+        }
+    }
+    if constexpr (CYC)
+    {
+        // reconstruction (tridiagonalSolver.C:418-450); f, v: row 1
+        const FftRow w = row[0];
+        const double den = (diag(0, w) + w.down*vN) + w.up*v;
+        const double p0 = ((X[t] - w.down*uN) - w.up*f)/den;
+        X[t] = p0;
+#pragma unroll 8
+        for (int k = 1; k < ns; k++)
+        {
+            const size_t at = (size_t)k*nm + t;
+            X[at] = X[at] + p0*V[at];
+        }
+    }
+}
+
+// Value (a, c) of a plane pair from the inverse FFT, unscaled: quarter-wave
+// axes sum an element and its image, e^{i phi} D_n + e^{-i phi} D_(2N-1-n).
+__device__ __forceinline__ C2 outputLine(const FftAxis& t, const C2* line,
+                                         int c)
+{
+    if (t.code == C_PER) return line[c];
+    if (halfWave(t.code))
+    {
+        const C2 v = line[c & 1 ? t.n - 1 - (c >> 1) : c >> 1];
+        return t.code == C_DD && (c & 1) ? C2{-v.x, -v.y} : v;
+    }
+    const int q = t.code == C_DN ? t.n - 1 - c : c;
+    const C2 w = t.tw[q];
+    return cadd(cmulc(line[q], w), cmul(line[2*t.n - 1 - q], w));
+}
+
+// Step 6: the two planes of x.
+template <int S>
+__global__ __launch_bounds__(256) void k_fft_out(FftGeom G, const C2* E,
+                                                 double* x, double scale)
+{
+    int a, c, p;
+    cellThread<S>(a, c, p);
+    if (c >= G.a2.n || p >= G.np) return;
+    const C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
+    const FftAxis& t = G.a1;
+    C2 v;
+    if (quarterWave(t.code))
+    {
+        const int q = t.code == C_DN ? t.n - 1 - a : a;
+        const C2 w = t.tw[q];
+        v = cadd(cmulc(outputLine(G.a2, Ep + (size_t)q*G.a2.L, c), w),
+                 cmul(outputLine(G.a2, Ep + (size_t)(2*t.n - 1 - q)*G.a2.L, c),
+                      w));
+    }
+    else
+    {
+        int q = a;
+        if (halfWave(t.code)) q = a & 1 ? t.n - 1 - (a >> 1) : a >> 1;
+        v = outputLine(G.a2, Ep + (size_t)q*G.a2.L, c);
+        if (t.code == C_DD && (a & 1)) v = C2{-v.x, -v.y};
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+    {
+        if (2*p + h >= G.ns) break;
+        int g[3];
+        cellOf<S>(2*p + h, a, c, g);
+        x[((size_t)(g[0] + 1)*G.P[1] + (g[1] + 1))*G.P[2] + (g[2] + 1)] =
+            (h ? v.y : v.x)*scale;
+    }
 }
 
 // Eigenvalue of mode k (tridiagonalSolver.C:31-98).
-__device__ __forceinline__ double eigen(int code, int n, int k)
+double eigen(int code, int n, int k)
 {
     const double pi = 3.14159265358979323846;
     double sn;
-    if (code == C_DD) sn = sin((k + 1)*pi/(2.0*n));
-    else if (code == C_NN) sn = sin(k*pi/(2.0*n));
-    else if (code == C_PER) sn = sin(k*pi/n);
-    else sn = sin((2.0*(k + 1) - 1.0)*pi/(4.0*n));
+    if (code == C_DD) sn = std::sin((k + 1)*pi/(2.0*n));
+    else if (code == C_NN) sn = std::sin(k*pi/(2.0*n));
+    else if (code == C_PER) sn = std::sin(std::min(k, n - k)*pi/n);
+    else sn = std::sin((2.0*(k + 1) - 1.0)*pi/(4.0*n));
     return -4.0*(sn*sn);
-}
-
-// Step 3: one thread per wave-number pair (k1, k2); the modes of all s are
-// read from E, solved, and written to X[s][k1][k2].  Dh and V are scratch
-// of the same shape (eliminated diagonal, cyclic auxiliary solution).
-__global__ void k_fft_tridiag(FftGeom g, const C2* E, C2* X, double* Dh,
-                              double* V, const double* h, const double* de,
-                              const double* dw)
-{
-    const long t = (long)blockIdx.x*blockDim.x + threadIdx.x;
-    const long nm = (long)g.n1*g.n2;
-    if (t >= nm) return;
-    const int k1 = int(t/g.n2), k2 = int(t % g.n2);
-    int m1, m2;
-    C2 w1, w2;
-    fwdMode(g.code1, g.n1, k1, m1, w1);
-    fwdMode(g.code2, g.n2, k2, m2, w2);
-    const C2 w = cmul(w1, w2);
-    const double lam1 = eigen(g.code1, g.n1, k1);
-    const double lam2 = eigen(g.code2, g.n2, k2);
-    const double Lm = lam1/g.d1sqr + lam2/g.d2sqr;
-    const int ns = g.ns, last = ns - 1;
-    const bool zero = lam1 == 0.0 && lam2 == 0.0;
-    // main diagonal of row k (tridiagonalSolver.C:107-250)
-    auto diag = [&](int k) -> double {
-        const double east = 1.0/(de[k]*h[k]);
-        const double west = 1.0/(h[k]*dw[k]);
-        if (k > 0 && k < last) return Lm - east - west;
-        const double pin = -1.0/(de[0]*h[0]) - 2.0/(h[0]*dw[0]);
-        switch (g.codes)
-        {
-        case C_DD:
-            return k == 0 ? Lm - east - 2.0/(h[0]*dw[0])
-                          : Lm - 2.0/(de[last]*h[last]) - west;
-        case C_NN:
-            if (k == 0) return zero ? pin : Lm - east;
-            return Lm - west;
-        case C_DN:
-            return k == 0 ? Lm - east - 2.0/(h[0]*dw[0]) : Lm - west;
-        case C_ND:
-            return k == 0 ? Lm - east
-                          : Lm - 2.0/(de[last]*h[last]) - west;
-        default:
-            if (k == 0) return zero ? pin : Lm - east - west;
-            return Lm - east - west;
-        }
-    };
-    // ddt: every diagonal minus 1/(deltaT*dtFrac) (tridiagonalSolver.C:352,
-    // :430), the pinned zero-mode row included
-    auto diagT = [&](int k) -> double {
-        const double d = diag(k);
-        return g.dT != 0.0 ? d - 1.0/g.dT : d;
-    };
-    auto DU = [&](int k) { return 1.0/(h[k]*de[k]); };
-    auto DL = [&](int k) { return 1.0/(h[k]*dw[k]); };
-    const long plane = (long)g.L1*g.L2;
-    const long off = (long)m1*g.L2 + m2;
-    const bool cyc = g.codes == C_PER;
-    const int start = cyc ? 1 : 0;
-    // right-hand sides: the transformed modes
-    for (int k = 0; k < ns; k++)
-    {
-        const C2 y = E[k*plane + off];
-        X[k*nm + t] = cmul(w, y);
-        Dh[k*nm + t] = diagT(k);
-        if (cyc) V[k*nm + t] = k == 1 ? -DL(1) : (k == last ? -DU(last) : 0.0);
-    }
-    // forward elimination (tridiagonalSolver.C:340-346)
-    for (int k = 1 + start; k < ns; k++)
-    {
-        const double dp = Dh[(k - 1)*nm + t];
-        const double m = DL(k)/dp;
-        Dh[k*nm + t] = Dh[k*nm + t] - m*DU(k - 1);
-        C2 f = X[k*nm + t];
-        const C2 fp = X[(k - 1)*nm + t];
-        f.x = f.x - m*fp.x;
-        f.y = f.y - m*fp.y;
-        X[k*nm + t] = f;
-        if (cyc) V[k*nm + t] = V[k*nm + t] - m*V[(k - 1)*nm + t];
-    }
-    // back substitution (:348-354)
-    {
-        const double d = Dh[last*nm + t];
-        C2 p = X[last*nm + t];
-        p.x = p.x/d;
-        p.y = p.y/d;
-        X[last*nm + t] = p;
-        if (cyc) V[last*nm + t] = V[last*nm + t]/d;
-    }
-    for (int k = ns - 2; k >= start; k--)
-    {
-        const double d = Dh[k*nm + t];
-        const C2 pn = X[(k + 1)*nm + t];
-        C2 f = X[k*nm + t];
-        f.x = (f.x - DU(k)*pn.x)/d;
-        f.y = (f.y - DU(k)*pn.y)/d;
-        X[k*nm + t] = f;
-        if (cyc) V[k*nm + t] = (V[k*nm + t] - DU(k)*V[(k + 1)*nm + t])/d;
-    }
-    if (cyc)
-    {
-        // reconstruction (tridiagonalSolver.C:418-450)
-        const C2 f0 = cmul(w, E[off]);
-        const C2 uN = X[last*nm + t], u1 = X[nm + t];
-        const double vN = V[last*nm + t], v1 = V[nm + t];
-        const double den = (diagT(0) + DL(0)*vN) + DU(0)*v1;
-        C2 p0;
-        p0.x = ((f0.x - DL(0)*uN.x) - DU(0)*u1.x)/den;
-        p0.y = ((f0.y - DL(0)*uN.y) - DU(0)*u1.y)/den;
-        X[t] = p0;
-        for (int k = 1; k < ns; k++)
-        {
-            C2 u = X[k*nm + t];
-            const double v = V[k*nm + t];
-            u.x = u.x + p0.x*v;
-            u.y = u.y + p0.y*v;
-            X[k*nm + t] = u;
-        }
-    }
-}
-
-// Spectrum position m of a transformed axis from the modes: the mode index
-// (or -1 for a zero) and the factor (inverse of fwdMode, with the
-// reflection symmetries X_{2N-m} = -X_m (DCT-II), S_{2N-m} = S_m (DST-II)).
-// Quarter-wave axes (L = 4N): x_a = 1/2N * 2 sum_k X_k cos or sin(phi_k
-// (2a+1)) is the real inverse FFT, scaled by 1/4N, of the spectrum with
-// 2 e^{i phi_k} X_k (DCT-IV; -2i e^{i phi_k} X_k for DST-IV) at 2k+1 and
-// its conjugate factor (2 e^{-i phi_k}; +2i e^{-i phi_k}) at 4N-1-2k.
-__device__ __forceinline__ void bwdMode(int code, int n, int m, int& k, C2& w)
-{
-    if (code == C_PER) { k = m; w = C2{1.0, 0.0}; return; }
-    const double pi = 3.14159265358979323846;
-    if (code == C_ND || code == C_DN)
-    {
-        if ((m & 1) == 0) { k = -1; return; }
-        const bool lower = m < 2*n;
-        k = lower ? (m - 1)/2 : (4*n - 1 - m)/2;
-        const double phi = pi*(2*k + 1)/(4.0*n);
-        const C2 e = cexpi(lower ? phi : -phi);
-        if (code == C_ND)
-            w = C2{2.0*e.x, 2.0*e.y};
-        else
-            w = lower ? C2{2.0*e.y, -2.0*e.x} : C2{-2.0*e.y, 2.0*e.x};
-        return;
-    }
-    const C2 e = cexpi(pi*m/(2.0*n));
-    if (code == C_NN)
-    {
-        if (m == n) { k = -1; return; }
-        k = m < n ? m : 2*n - m;
-        w = m < n ? e : C2{-e.x, -e.y};
-        return;
-    }
-    if (m == 0) { k = -1; return; }
-    k = m <= n ? m - 1 : 2*n - m - 1;
-    w = C2{e.y, -e.x};   // -i*e
-}
-
-// Step 4: every position of the extended spectrum.
-__global__ void k_fft_expand(FftGeom g, const C2* X, C2* E)
-{
-    const long t = (long)blockIdx.x*blockDim.x + threadIdx.x;
-    const long plane = (long)g.L1*g.L2;
-    if (t >= plane*g.ns) return;
-    const int s = int(t/plane);
-    const long r = t - (long)s*plane;
-    const int m1 = int(r/g.L2), m2 = int(r % g.L2);
-    int k1, k2;
-    C2 w1, w2;
-    bwdMode(g.code1, g.n1, m1, k1, w1);
-    bwdMode(g.code2, g.n2, m2, k2, w2);
-    C2 v{0.0, 0.0};
-    if (k1 >= 0 && k2 >= 0)
-        v = cmul(cmul(w1, w2),
-                 X[((long)s*g.n1 + k1)*g.n2 + k2]);
-    E[t] = v;
-}
-
-// Step 5: scaled real part into the interior of x.
-__global__ void k_fft_out(FftGeom g, const C2* E, double* x, double scale)
-{
-    const long t = (long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (t >= (long)g.N[0]*g.N[1]*g.N[2]) return;
-    int q[3];
-    q[0] = int(t/((long)g.N[1]*g.N[2]));
-    q[1] = int((t/g.N[2]) % g.N[1]);
-    q[2] = int(t % g.N[2]);
-    const long e = ((long)q[g.s]*g.L1 + q[g.d1])*g.L2 + q[g.d2];
-    x[refIndex(g, q[0], q[1], q[2])] = E[e].x*scale;
 }
 
 // Every ghost of x (meshLevel::correctBoundaryConditions on level 0): face
@@ -381,14 +684,20 @@ __global__ void k_fft_out(FftGeom g, const C2* E, double* x, double scale)
 // delta = 1/h of the mirrored boundary cell, Dirichlet 2v - x_P -- and edge
 // and corner ghosts by periodic image when every face they border is
 // periodic, else a copy of the adjacent interior cell.
-__global__ void k_fft_ghosts(FftGeom g, double* x)
+__global__ __launch_bounds__(256) void k_fft_ghosts(FftGeom g, double* x)
 {
-    const long t = (long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (t >= (long)g.P[0]*g.P[1]*g.P[2]) return;
+    // blockIdx.z: the two faces normal to an axis (whole, the lower axis'
+    // edges included); blockIdx.y a row, lanes along its last axis
+    const int d = blockIdx.z >> 1, side = blockIdx.z & 1;
+    const int a1 = d == 0 ? 1 : 0, a2 = d == 2 ? 1 : 2;
+    const int u = blockIdx.x*256 + threadIdx.x;
+    if (int(blockIdx.y) >= g.P[a1] || u >= g.P[a2]) return;
+    const int w = side ? g.P[d] - 1 : 0;
     int q[3];
-    q[0] = int(t/((long)g.P[1]*g.P[2]));
-    q[1] = int((t/g.P[2]) % g.P[1]);
-    q[2] = int(t % g.P[2]);
+    q[0] = d == 0 ? w : int(blockIdx.y);
+    q[1] = d == 0 ? int(blockIdx.y) : (d == 1 ? w : u);
+    q[2] = d == 2 ? w : u;
+    const long t = ((long)q[0]*g.P[1] + q[1])*g.P[2] + q[2];
     int bo[3], nout = 0;
     bool allPer = true;
     for (int d = 0; d < 3; d++)
@@ -438,13 +747,13 @@ struct bmg_fft
     int device = 0;
     hipStream_t stream = nullptr;
     FftGeom g{};
-    C2* E = nullptr;       // extended spectrum, ns x L1 x L2
-    C2* X = nullptr;       // modes, ns x n1 x n2
-    double* Dh = nullptr;
-    double* V = nullptr;
-    double* h = nullptr;   // widths along s, and their east/west means
-    double* de = nullptr;
-    double* dw = nullptr;
+    C2* E = nullptr;       // plane pairs, np x L1 x L2
+    double* X = nullptr;   // modes, ns x n1 x n2
+    double* R = nullptr;   // reciprocal eliminated diagonals
+    double* V = nullptr;   // cyclic auxiliary solution
+    double* tables = nullptr;      // twiddles, eigenvalues and rows
+    const FftRow* row = nullptr;   // the rows along s
+    double pin = 0.0;              // diagonal of the zero mode's pinned row
     void* work = nullptr;
     rocfft_plan fwd = nullptr, bwd = nullptr;
     rocfft_execution_info info = nullptr;
@@ -454,8 +763,8 @@ struct bmg_fft
         if (fwd) rocfft_plan_destroy(fwd);
         if (bwd) rocfft_plan_destroy(bwd);
         if (info) rocfft_execution_info_destroy(info);
-        for (void* p : {(void*)E, (void*)X, (void*)Dh, (void*)V, (void*)h,
-                        (void*)de, (void*)dw, work})
+        for (void* p : {(void*)E, (void*)X, (void*)R, (void*)V,
+                        (void*)tables, work})
             if (p) (void)hipFree(p);
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -506,23 +815,45 @@ void fft_create(bmg_fft** out, const bmg_grid* grid)
         throw Error(BMG_ERR_ARG, "at least two mesh directions must be "
                                  "uniform for the FFT solver");
     if (g.s < 0) g.s = g.N[0] > 1 ? 0 : 2;
-    g.d1 = g.s == 0 ? 2 : 0;
-    g.d2 = g.s == 2 ? 1 : (g.s == 0 ? 1 : 2);
-    g.n1 = g.N[g.d1];
-    g.n2 = g.N[g.d2];
+    g.d1 = g.s == 0 ? 1 : 0;
+    g.d2 = g.s == 2 ? 1 : 2;
     g.ns = g.N[g.s];
-    g.code1 = axisCode(g.bc[2*g.d1], g.bc[2*g.d1 + 1]);
-    g.code2 = axisCode(g.bc[2*g.d2], g.bc[2*g.d2 + 1]);
+    g.np = (g.ns + 1)/2;
     g.codes = axisCode(g.bc[2*g.s], g.bc[2*g.s + 1]);
     if (g.ns < 2 || (g.codes == C_PER && g.ns < 3))
         throw Error(BMG_ERR_ARG, "too few cells along the tridiagonal axis");
-    auto extLen = [](int code, int n) {
-        return code == C_PER ? n : (code == C_ND || code == C_DN ? 4*n : 2*n);
-    };
-    g.L1 = extLen(g.code1, g.n1);
-    g.L2 = extLen(g.code2, g.n2);
-    g.d1sqr = w[g.d1][0]*w[g.d1][0];
-    g.d2sqr = w[g.d2][0]*w[g.d2][0];
+    FftAxis* ax[2] = {&g.a1, &g.a2};
+    const int dd[2] = {g.d1, g.d2};
+    std::vector<double> tables;
+    size_t at[2][3];
+    for (int t = 0; t < 2; t++)
+    {
+        FftAxis& A = *ax[t];
+        const int d = dd[t];
+        A.n = g.N[d];
+        A.code = axisCode(g.bc[2*d], g.bc[2*d + 1]);
+        A.L = quarterWave(A.code) ? 2*A.n : A.n;
+        const long double pi = 3.14159265358979323846264338327950288L;
+        // tables collected for one upload, in doubles
+        auto unit = [&](long double th)
+        {
+            tables.push_back(double(std::cos(th)));
+            tables.push_back(double(std::sin(th)));
+        };
+        at[t][0] = tables.size();
+        if (halfWave(A.code))
+            for (int j = 0; j <= A.n/2; j++) unit(-pi*j/(2.0L*A.n));
+        if (quarterWave(A.code))
+            for (int j = 0; j < A.n; j++) unit(-pi*(2*j + 1)/(4.0L*A.n));
+        at[t][1] = tables.size();
+        if (quarterWave(A.code))
+            for (int j = 0; j < A.n; j++) unit(-pi*j/(2.0L*A.n));
+        at[t][2] = tables.size();
+        const double sq = w[d][0]*w[d][0];
+        for (int k = 0; k < A.n; k++)
+            tables.push_back(eigen(A.code, A.n, k)/sq);
+        if (tables.size() & 1) tables.push_back(0.0);
+    }
     // widths along s with the ghost widths (mirrored, or the periodic
     // images) and their means (tridiagonalSolver.C:112-130)
     const std::vector<double>& ws = w[g.s];
@@ -540,25 +871,58 @@ void fft_create(bmg_fft** out, const bmg_grid* grid)
     }
     HIPCK(hipGetDevice(&F->device));
     HIPCK(hipStreamCreateWithFlags(&F->stream, hipStreamNonBlocking));
-    const size_t nE = size_t(ns)*g.L1*g.L2;
-    const size_t nX = size_t(ns)*g.n1*g.n2;
+    const size_t nE = size_t(g.np)*g.a1.L*g.a2.L;
+    const size_t nX = size_t(ns)*g.a1.n*g.a2.n;
     F->E = devAlloc<C2>(nE);
-    F->X = devAlloc<C2>(nX);
-    F->Dh = devAlloc<double>(nX);
+    F->X = devAlloc<double>(nX);
+    F->R = devAlloc<double>(nX);
     F->V = devAlloc<double>(per ? nX : 1);
-    F->h = devUpload(h);
-    F->de = devUpload(de);
-    F->dw = devUpload(dw);
+    std::vector<FftRow> rows(ns);
+    for (int k = 0; k < ns; k++)
+    {
+        FftRow& q = rows[k];
+        q.up = 1.0/(h[k]*de[k]);
+        q.down = 1.0/(h[k]*dw[k]);
+        q.east = q.up;
+        q.west = q.down;
+        if (per) continue;
+        if (k == 0)
+            q.west = g.codes == C_DD || g.codes == C_DN ? 2.0/(h[0]*dw[0])
+                                                        : 0.0;
+        if (k == ns - 1)
+            q.east = g.codes == C_DD || g.codes == C_ND ? 2.0/(de[k]*h[k])
+                                                        : 0.0;
+    }
+    F->pin = -1.0/(de[0]*h[0]) - 2.0/(h[0]*dw[0]);
+    const size_t atRows = tables.size();
+    for (const FftRow& q : rows)
+        tables.insert(tables.end(), {q.up, q.down, q.east, q.west});
+    F->tables = devUpload(tables);
+    for (int t = 0; t < 2; t++)
+    {
+        ax[t]->tw = reinterpret_cast<const C2*>(F->tables + at[t][0]);
+        ax[t]->pad = reinterpret_cast<const C2*>(F->tables + at[t][1]);
+        ax[t]->lam = F->tables + at[t][2];
+    }
+    F->row = reinterpret_cast<const FftRow*>(F->tables + atRows);
     std::call_once(g_rocfftSetup, [] { rocfftCheck(rocfft_setup(), "setup"); });
-    const size_t lengths[2] = {size_t(g.L2), size_t(g.L1)};
+    // an axis of one point needs no FFT (and two leave none)
+    size_t lengths[2], dims = 0;
+    for (const FftAxis* A : {&g.a2, &g.a1})
+        if (A->L > 1) lengths[dims++] = size_t(A->L);
+    if (dims == 0)
+    {
+        *out = F.release();
+        return;
+    }
     rocfftCheck(rocfft_plan_create(&F->fwd, rocfft_placement_inplace,
                                    rocfft_transform_type_complex_forward,
-                                   rocfft_precision_double, 2, lengths,
-                                   size_t(ns), nullptr), "plan");
+                                   rocfft_precision_double, dims, lengths,
+                                   size_t(g.np), nullptr), "plan");
     rocfftCheck(rocfft_plan_create(&F->bwd, rocfft_placement_inplace,
                                    rocfft_transform_type_complex_inverse,
-                                   rocfft_precision_double, 2, lengths,
-                                   size_t(ns), nullptr), "plan");
+                                   rocfft_precision_double, dims, lengths,
+                                   size_t(g.np), nullptr), "plan");
     size_t w1 = 0, w2 = 0;
     rocfftCheck(rocfft_plan_get_work_buffer_size(F->fwd, &w1), "work size");
     rocfftCheck(rocfft_plan_get_work_buffer_size(F->bwd, &w2), "work size");
@@ -589,27 +953,55 @@ void fft_solve_device(bmg_fft* F, const double* db, double* dx,
         throw Error(BMG_ERR_ARG, "time term needs deltaT*dtFrac > 0");
     FftGeom g = F->g;
     g.dT = dxold ? dT : 0.0;
-    const long cells = long(g.N[0])*g.N[1]*g.N[2];
-    const long padded = long(g.P[0])*g.P[1]*g.P[2];
-    const long nE = long(g.ns)*g.L1*g.L2;
-    const long nm = long(g.n1)*g.n2;
     hipStream_t s = F->stream;
-    auto blocks = [](long n) { return dim3(unsigned((n + 255)/256)); };
-    hipLaunchKernelGGL(k_fft_rhs, blocks(cells), dim3(256), 0, s, g, db, dx,
-                       dxold, F->E);
+    auto blocks = [](int n, int b) { return unsigned((n + b - 1)/b); };
+    // steps 1 and 6: a thread per plane pair and position
+    auto cells = [&](int L1, int L2)
+    {
+        return g.s == 2 ? dim3(blocks(L2, 16), L1, blocks(g.np, 16))
+                        : dim3(blocks(L2, 256), L1, g.np);
+    };
+    const dim3 gin = cells(g.a1.L, g.a2.L), gout = cells(g.a1.n, g.a2.n);
+    if (g.s == 0)
+        hipLaunchKernelGGL(k_fft_rhs<0>, gin, dim3(256), 0, s, g, db, dx,
+                           dxold, F->E);
+    else if (g.s == 1)
+        hipLaunchKernelGGL(k_fft_rhs<1>, gin, dim3(256), 0, s, g, db, dx,
+                           dxold, F->E);
+    else
+        hipLaunchKernelGGL(k_fft_rhs<2>, gin, dim3(256), 0, s, g, db, dx,
+                           dxold, F->E);
     HIPCK(hipGetLastError());
     void* buf[1] = {F->E};
-    rocfftCheck(rocfft_execute(F->fwd, buf, nullptr, F->info), "forward");
-    hipLaunchKernelGGL(k_fft_tridiag, blocks(nm), dim3(256), 0, s, g, F->E,
-                       F->X, F->Dh, F->V, F->h, F->de, F->dw);
-    hipLaunchKernelGGL(k_fft_expand, blocks(nE), dim3(256), 0, s, g, F->X,
-                       F->E);
+    if (F->fwd)
+        rocfftCheck(rocfft_execute(F->fwd, buf, nullptr, F->info), "forward");
+    const dim3 gorb(blocks(orbits(g.a1)*orbits(g.a2), 256), g.np);
+    hipLaunchKernelGGL(k_fft_modes, gorb, dim3(256), 0, s, g, F->E, F->X);
+    const dim3 gtri(blocks(g.a2.n, 64), g.a1.n);
+    if (g.codes == C_PER)
+        hipLaunchKernelGGL(k_fft_tridiag<true>, gtri, dim3(64), 0, s, g, F->X,
+                           F->R, F->V, F->row, F->pin);
+    else
+        hipLaunchKernelGGL(k_fft_tridiag<false>, gtri, dim3(64), 0, s, g, F->X,
+                           F->R, F->V, F->row, F->pin);
+    hipLaunchKernelGGL(k_fft_spectrum, gorb, dim3(256), 0, s, g, F->X, F->E);
     HIPCK(hipGetLastError());
-    rocfftCheck(rocfft_execute(F->bwd, buf, nullptr, F->info), "inverse");
-    const double scale = 1.0/(double(g.L1)*double(g.L2));
-    hipLaunchKernelGGL(k_fft_out, blocks(cells), dim3(256), 0, s, g, F->E,
-                       dx, scale);
-    hipLaunchKernelGGL(k_fft_ghosts, blocks(padded), dim3(256), 0, s, g, dx);
+    if (F->bwd)
+        rocfftCheck(rocfft_execute(F->bwd, buf, nullptr, F->info), "inverse");
+    const double scale = 1.0/(double(g.a1.n)*double(g.a2.n));
+    if (g.s == 0)
+        hipLaunchKernelGGL(k_fft_out<0>, gout, dim3(256), 0, s, g, F->E, dx,
+                           scale);
+    else if (g.s == 1)
+        hipLaunchKernelGGL(k_fft_out<1>, gout, dim3(256), 0, s, g, F->E, dx,
+                           scale);
+    else
+        hipLaunchKernelGGL(k_fft_out<2>, gout, dim3(256), 0, s, g, F->E, dx,
+                           scale);
+    const int pmax = std::max(g.P[0], g.P[1]);
+    hipLaunchKernelGGL(k_fft_ghosts,
+                       dim3(blocks(std::max(g.P[1], g.P[2]), 256), pmax, 6),
+                       dim3(256), 0, s, g, dx);
     HIPCK(hipGetLastError());
     HIPCK(hipStreamSynchronize(s));
 }

@@ -1,0 +1,50 @@
+"""The FFT solver's plane pairs, mirror-image orbits and transform lengths at
+the sizes where they can go wrong: odd and even, one and two cells along a
+transformed axis, odd and even plane counts along every tridiagonal axis, more
+than one block of modes, against the oracle (1e-11 of the solution, as the
+solver's other tests)."""
+import itertools
+
+import numpy as np
+import pytest
+
+from briscola_amd import bmg
+from oracle import fft_ref as F
+
+pytestmark = pytest.mark.gpu
+
+PAIRS = {"N": (F.NEU, F.NEU), "D": (F.DIR, F.DIR), "P": (F.PER, F.PER),
+         "Q": (F.DIR, F.NEU), "R": (F.NEU, F.DIR)}
+
+
+@pytest.mark.parametrize("kinds", ["NDP", "PPN", "QRD", "PQP", "DNR", "PPP",
+                                   "NNN", "RPQ"])
+@pytest.mark.parametrize("stretch", [0, 1, 2, None])
+@pytest.mark.parametrize("n", [(7, 9, 11), (6, 5, 8), (3, 2, 1), (2, 1, 3),
+                               (5, 70, 67)])
+def test_odd_and_small_sizes(gpu, n, stretch, kinds):
+    if stretch is not None and kinds[stretch] == "P":
+        pytest.skip("periodic axes are uniform")
+    verts = [np.linspace(0.0, 1.0 + d, q + 1) for d, q in enumerate(n)]
+    if stretch is not None and n[stretch] > 1:
+        t = np.linspace(-1.0, 1.0, n[stretch] + 1)
+        verts[stretch] = np.tanh(1.5 * t) / np.tanh(1.5)
+    s = F.plan(verts)[0]
+    if n[s] < (3 if kinds[s] == "P" else 2):
+        pytest.skip("too few cells along the tridiagonal axis")
+    bc = [k for a in kinds for k in PAIRS[a]]
+    print(f"[fft shapes] n={n} kinds={kinds} stretch={stretch}", flush=True)
+    rng = np.random.default_rng(4)
+    b = np.zeros(tuple(q + 2 for q in n))
+    b[1:-1, 1:-1, 1:-1] = rng.standard_normal(n)
+    if F.DIR not in bc:
+        # a compatible source: the pinned row of the zero mode else amplifies
+        # rounding by the condition of the singular operator
+        w = [np.diff(v) for v in verts]
+        vol = w[0][:, None, None] * w[1][None, :, None] * w[2][None, None, :]
+        b[1:-1, 1:-1, 1:-1] -= (vol * b[1:-1, 1:-1, 1:-1]).sum() / vol.sum()
+    x0 = np.zeros_like(b)
+    ref = np.asarray(F.solve(b, x0, bc, verts))
+    x = bmg.FFT(verts, bc).solve(b.copy(), x0.copy())
+    got = x[1:-1, 1:-1, 1:-1]
+    assert np.abs(got - ref).max() <= 1e-11 * np.abs(ref).max()

@@ -95,6 +95,7 @@ struct Acts {
     bf16* dyd[3] = {nullptr, nullptr, nullptr};
     float* gout = nullptr;
     float* partial = nullptr;
+    float* wgrad = nullptr;    // workspace of the weight gradients
     float* scal = nullptr;     // [0] shift, [1] loss
     bool train = false;
 
@@ -106,6 +107,7 @@ struct Acts {
         dfree(dy3);
         dfree(gout);
         dfree(partial);
+        dfree(wgrad);
         dfree(scal);
         for (int i = 0; i < 3; i++)
         {
@@ -188,11 +190,16 @@ struct Net {
         if (stream) (void)hipStreamDestroy(stream);
     }
 
-    void refreshBF16()
+    WeightViews views() const
     {
+        WeightViews v;
         for (int i = 0; i < 7; i++)
-            to_bf16(P + woff[i], WB[i], long(kConvs[i].cout)*kp[i], stream);
+            v.l[i] = WeightView{int(woff[i]), kConvs[i].cin, kConvs[i].cout,
+                                kp[i], kpt[i], WB[i], WT[i]};
+        return v;
     }
+
+    void refreshBF16() { refresh_weights(views(), P, int(nparam), stream); }
 
     void ensureActs(int D, int H, int W, bool train)
     {
@@ -232,6 +239,11 @@ struct Net {
                 a.dpin[l] = dalloc<bf16>(size_t(a.M[l])*kPinC[l]);
             a.dy3 = dalloc<bf16>(size_t(a.M[3])*128);
             a.gout = dalloc<float>(a.M[0]);
+            size_t need = 0;
+            for (int i = 0; i < 7; i++)
+                need = std::max(need, wgrad_workspace(wgrad(i, nullptr, 8,
+                                                            nullptr, 8)));
+            a.wgrad = dalloc<float>(need);
         }
     }
 
@@ -274,16 +286,12 @@ struct Net {
         head_fwd(a.yd[0], 16, a.M[0], P + hoff, a.out, s);
     }
 
-    // gradient of one convolution: dz (post-ReLU mask applied) -> weight
-    // and bias gradients, and optionally the input gradient dx
-    void convBackward(int i, const bf16* x, int ldx, const bf16* dz, int lddz,
-                      bf16* dx, int lddx, hipStream_t s)
+    WgradArgs wgrad(int i, const bf16* x, int ldx, const bf16* dz,
+                    int lddz) const
     {
         const ConvSpec& c = kConvs[i];
-        const Grid3 g = acts.g[c.level];
-        const int M = g.D*g.H*g.W;
         WgradArgs w;
-        w.g = g;
+        w.g = acts.g[c.level];
         w.x = x;
         w.ldx = ldx;
         w.cin = c.cin;
@@ -293,14 +301,20 @@ struct Net {
         w.taps = 27;
         w.kp = kp[i];
         w.dw = G + woff[i];
-        w.chunk = std::max(256, (M + 255)/256/32*32);
-        conv_wgrad(w, s);
-        // bias gradient: column sums of dz through a 1x1x1 weight gradient
-        // against a constant-one input is avoided; sum dz directly
-        biasGrad(dz, lddz, M, c.cout, G + boff[i], s);
+        w.chunk = 256;
+        return w;
+    }
+
+    // gradient of one convolution: dz (post-ReLU mask applied) -> weight
+    // and bias gradients, and optionally the input gradient dx
+    void convBackward(int i, const bf16* x, int ldx, const bf16* dz, int lddz,
+                      bf16* dx, int lddx, hipStream_t s)
+    {
+        const ConvSpec& c = kConvs[i];
+        const Grid3 g = acts.g[c.level];
+        conv_wgrad(wgrad(i, x, ldx, dz, lddz), acts.wgrad, G + boff[i], s);
         if (dx)
         {
-            flip_weights(WB[i], c.cin, c.cout, kp[i], 27, WT[i], kpt[i], s);
             ConvArgs d;
             d.g = g;
             d.x = dz;
@@ -318,9 +332,6 @@ struct Net {
         }
     }
 
-    void biasGrad(const bf16* dz, int lddz, int M, int C, float* out,
-                  hipStream_t s);
-
     // backward from acts.gout (dL/d out) to G
     void backward(hipStream_t s)
     {
@@ -330,64 +341,31 @@ struct Net {
         const int nb = head_bwd(a.yd[0], 16, a.M[0], P + hoff, a.gout, a.dyd[0],
                                 16, a.partial, s);
         col_sum(a.partial, nb, 17, 1.0f, G + hoff, s);
-        // D0
-        relu_bwd(a.dyd[0], 16, a.yd[0], 16, a.M[0], 16, s);
+        // D0 (the head's gradient carries its ReLU mask, as do the ones below)
         convBackward(6, a.cat[0], 48, a.dyd[0], 16, a.dcat[0], 48, s);
-        up_bwd(a.dcat[0], 48, a.g[0], 32, a.dyd[1], 32, s);
         // D1
-        relu_bwd(a.dyd[1], 32, a.yd[1], 32, a.M[1], 32, s);
+        up_relu_bwd(a.dcat[0], 48, a.g[0], 32, a.yd[1], 32, a.dyd[1], 32, s);
         convBackward(5, a.cat[1], 96, a.dyd[1], 32, a.dcat[1], 96, s);
-        up_bwd(a.dcat[1], 96, a.g[1], 64, a.dyd[2], 64, s);
         // D2
-        relu_bwd(a.dyd[2], 64, a.yd[2], 64, a.M[2], 64, s);
+        up_relu_bwd(a.dcat[1], 96, a.g[1], 64, a.yd[2], 64, a.dyd[2], 64, s);
         convBackward(4, a.cat[2], 192, a.dyd[2], 64, a.dcat[2], 192, s);
-        up_bwd(a.dcat[2], 192, a.g[2], 128, a.dy3, 128, s);
         // E3
-        relu_bwd(a.dy3, 128, a.y3, 128, a.M[3], 128, s);
+        up_relu_bwd(a.dcat[2], 192, a.g[2], 128, a.y3, 128, a.dy3, 128, s);
         convBackward(3, a.pin[3], 64, a.dy3, 128, a.dpin[3], 64, s);
         // E2: skip gradient + pooled gradient
-        pool_bwd(a.dpin[3], 64, a.g[2], 64, a.dcat[2] + 128, 192, s);
-        relu_bwd(a.dcat[2] + 128, 192, a.cat[2] + 128, 192, a.M[2], 64, s);
+        pool_relu_bwd(a.dpin[3], 64, a.g[2], 64, a.cat[2] + 128, 192,
+                      a.dcat[2] + 128, 192, s);
         convBackward(2, a.pin[2], 32, a.dcat[2] + 128, 192, a.dpin[2], 32, s);
         // E1
-        pool_bwd(a.dpin[2], 32, a.g[1], 32, a.dcat[1] + 64, 96, s);
-        relu_bwd(a.dcat[1] + 64, 96, a.cat[1] + 64, 96, a.M[1], 32, s);
+        pool_relu_bwd(a.dpin[2], 32, a.g[1], 32, a.cat[1] + 64, 96,
+                      a.dcat[1] + 64, 96, s);
         convBackward(1, a.pin[1], 16, a.dcat[1] + 64, 96, a.dpin[1], 16, s);
         // E0
-        pool_bwd(a.dpin[1], 16, a.g[0], 16, a.dcat[0] + 32, 48, s);
-        relu_bwd(a.dcat[0] + 32, 48, a.cat[0] + 32, 48, a.M[0], 16, s);
+        pool_relu_bwd(a.dpin[1], 16, a.g[0], 16, a.cat[0] + 32, 48,
+                      a.dcat[0] + 32, 48, s);
         convBackward(0, a.xin, 8, a.dcat[0] + 32, 48, nullptr, 0, s);
     }
 };
-
-namespace {
-
-// per-block partial column sums of a BF16 slice (C <= 256 channels)
-__global__ __launch_bounds__(256) void k_bias_partial(const bf16* dz, int ld,
-                                                      int M, int C, int rows,
-                                                      float* partial)
-{
-    const int c = threadIdx.x;
-    if (c >= C) return;
-    const int m0 = blockIdx.x*rows;
-    const int m1 = min(M, m0 + rows);
-    float s = 0.0f;
-    for (int m = m0; m < m1; m++) s += float(dz[size_t(m)*ld + c]);
-    partial[size_t(blockIdx.x)*C + c] = s;
-}
-
-}  // namespace
-
-void Net::biasGrad(const bf16* dz, int lddz, int M, int C, float* out,
-                   hipStream_t s)
-{
-    const int rows = 1024;
-    const int nb = (M + rows - 1)/rows;
-    // acts.partial holds at least 17*M/256 floats >= C*M/1024 for C <= 128
-    hipLaunchKernelGGL(k_bias_partial, dim3(nb), dim3(256), 0, s, dz, lddz, M,
-                       C, rows, acts.partial);
-    col_sum(acts.partial, nb, C, 1.0f, out, s);
-}
 
 }  // namespace unet
 }  // namespace bmg
@@ -522,9 +500,8 @@ int bmg_unet_train_step(bmg_unet* u, int D, int H, int W, const float* f,
         bmg::unet::col_sum(a.partial, nb2, 1, 1.0f/float(a.M[0]), a.scal + 1, s);
         n.backward(s);
         n.step++;
-        bmg::unet::adam(n.P, n.Mo, n.Ve, n.G, int(n.nparam), lr, 0.9f, 0.999f,
-                        1e-8f, n.step, nullptr, s);
-        n.refreshBF16();
+        bmg::unet::adam(n.views(), n.P, n.Mo, n.Ve, n.G, int(n.nparam), lr,
+                        0.9f, 0.999f, 1e-8f, n.step, s);
         float h = 0.0f;
         UCK(hipMemcpyAsync(&h, a.scal + 1, sizeof(float), hipMemcpyDeviceToHost,
                            s));
@@ -621,9 +598,21 @@ int bmg_unet_op_conv_wgrad(int D, int H, int W, const uint16_t* x, int ldx,
         a.kp = kp;
         a.dw = dw;
         a.chunk = chunk;
-        bmg::unet::conv_wgrad(a, nullptr);
-        UCK(hipGetLastError());
-        UCK(hipDeviceSynchronize());
+        float* work = nullptr;
+        try
+        {
+            const size_t need = bmg::unet::wgrad_workspace(a);
+            if (need) work = bmg::unet::dalloc<float>(need);
+            bmg::unet::conv_wgrad(a, work, nullptr, nullptr);
+            UCK(hipGetLastError());
+            UCK(hipDeviceSynchronize());
+        }
+        catch (...)
+        {
+            bmg::unet::dfree(work);
+            throw;
+        }
+        bmg::unet::dfree(work);
     });
 }
 

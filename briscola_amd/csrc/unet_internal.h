@@ -56,20 +56,27 @@ struct WgradArgs {
 inline int round32(int k) { return (k + 31)/32*32; }
 
 void conv_fwd(const ConvArgs& a, hipStream_t s);
-void conv_wgrad(const WgradArgs& a, hipStream_t s);
+// Floats of workspace the tiled weight gradient of these arguments needs (0:
+// the general kernel takes them, without workspace).
+size_t wgrad_workspace(const WgradArgs& a);
+// dbias (tiled kernel only): cout column sums of dz, added at the end of dw's
+// cout*kp weights.
+void conv_wgrad(const WgradArgs& a, float* workspace, float* dbias,
+                hipStream_t s);
 // weights of the data gradient: wt[c][t'*cout + n] = w[n][(26-t')*cin + c]
 void flip_weights(const bf16* w, int cin, int cout, int kp, int taps, bf16* wt,
                   int kpt, hipStream_t s);
-void relu_bwd(bf16* dy, int lddy, const bf16* y, int ldy, int M, int C,
-              hipStream_t s);
 void pool(const bf16* x, int ldx, Grid3 fine, int C, bf16* y, int ldy,
           hipStream_t s);
-void pool_bwd(const bf16* dy, int lddy, Grid3 fine, int C, bf16* dx, int lddx,
-              hipStream_t s);
+// dx = (dx + dy/8 of the parent) where y > 0 (C, strides and bases multiples
+// of 8 channels, likewise up_relu_bwd)
+void pool_relu_bwd(const bf16* dy, int lddy, Grid3 fine, int C, const bf16* y,
+                   int ldy, bf16* dx, int lddx, hipStream_t s);
 void up(const bf16* x, int ldx, Grid3 fine, int C, bf16* y, int ldy,
         hipStream_t s);
-void up_bwd(const bf16* dy, int lddy, Grid3 fine, int C, bf16* dx, int lddx,
-            hipStream_t s);
+// dx = the sum of the eight children's dy where y > 0
+void up_relu_bwd(const bf16* dy, int lddy, Grid3 fine, int C, const bf16* y,
+                 int ldy, bf16* dx, int lddx, hipStream_t s);
 // w[0..15] weights, w[16] bias
 void head_fwd(const bf16* x, int ldx, int M, const float* w, float* out,
               hipStream_t s);
@@ -81,9 +88,21 @@ int diff_sum(const float* a, const float* b, int M, float* partial,
              hipStream_t s);
 void col_sum(const float* in, int rows, int cols, float scale, float* out,
              hipStream_t s);
-void adam(float* w, float* m, float* v, const float* g, int n, float lr,
-          float b1, float b2, float eps, int step, bf16* wb, hipStream_t s);
-void to_bf16(const float* a, bf16* b, long n, hipStream_t s);
+// The BF16 copies of a layer's weights: parameters [off, off + cout*kp).
+struct WeightView {
+    int off, cin, cout, kp, kpt;
+    bf16* w;
+    bf16* wt;    // flipped, for the data gradient; null: none
+};
+struct WeightViews {
+    enum { LAYERS = 7 };
+    WeightView l[LAYERS];
+};
+void adam(const WeightViews& views, float* w, float* m, float* v,
+          const float* g, int n, float lr, float b1, float b2, float eps,
+          int step, hipStream_t s);
+void refresh_weights(const WeightViews& views, const float* w, int n,
+                     hipStream_t s);
 void pack_input(const float* f, const float* lam, int M, bf16* x,
                 hipStream_t s);
 

@@ -15,6 +15,8 @@
 // l%16, k = 8*(l/16)..+7), D (lane l: column l%16, rows 4*(l/16)..+3).
 #include "unet_internal.h"
 
+#include <algorithm>
+
 namespace bmg {
 namespace unet {
 
@@ -134,14 +136,13 @@ struct ConvTile {
 // CIN > 0: all CIN channels staged at once, the k loop unrolled with each
 // step's tap and channel known at compile time per lane group; CIN = 0:
 // 32-channel chunks of a runtime channel count (a multiple of 32), the 27
-// taps unrolled.  Consecutive k steps alternate between two accumulator
-// sets (AS = 2 when the tiles leave registers for it) so that dependent
-// MFMAs do not follow each other.
-template <int NT, int MT, int CIN>
+// taps unrolled.  Consecutive k steps alternate between AS accumulator
+// sets (2 when the tiles leave registers for it) so that dependent MFMAs do
+// not follow each other.
+template <int NT, int MT, int CIN, int AS>
 __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
 {
     using Tl = ConvTile<MT>;
-    constexpr int AS = NT*MT <= 8 ? 2 : 1;
     constexpr int CH = CIN > 0 ? CIN : 32;
     // LDS voxel stride in elements (padded by 8: 16-byte reads of 16
     // consecutive voxels spread over the banks), known at compile time so
@@ -161,6 +162,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
     const int y0 = ((b/ntx) % nty)*Tl::TY;
     const int z0 = (b/(ntx*nty))*Tl::TZ;
     const int nchunk = a.cin/CH;
+    const int nb0 = blockIdx.y*NT*16;   // first output channel
     constexpr int parts = CH/8;
     floatx4 acc[AS][MT][NT];
 #pragma unroll
@@ -181,7 +183,8 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
     }
     const bf16* wrow[NT];
 #pragma unroll
-    for (int j = 0; j < NT; j++) wrow[j] = a.w + size_t(j*16 + row)*a.kp + kq;
+    for (int j = 0; j < NT; j++)
+        wrow[j] = a.w + size_t(nb0 + j*16 + row)*a.kp + kq;
     // halo-tile offset of tap t, in voxels
     auto tap_off = [](int t)
     {
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
 #pragma unroll
         for (int j = 0; j < NT; j++)
         {
-            const int n = j*16 + row;
+            const int n = nb0 + j*16 + row;
             const float bias = a.bias ? a.bias[n] : 0.0f;
 #pragma unroll
             for (int q = 0; q < 4; q++)
@@ -289,11 +292,11 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
                 tb[(4*g + q)*16 + row] = bf16(v);
             }
             __syncthreads();
-            // lanes 0..31: voxel x0 + lane/2, channels j*16 + 8*(lane&1)
+            // lanes 0..31: voxel x0 + lane/2, channels nb0 + j*16 + 8*(lane&1)
             if (lane < 32 && yy < H && zz < D)
             {
                 const int xx = x0 + (lane >> 1);
-                const int n0 = j*16 + 8*(lane & 1);
+                const int n0 = nb0 + j*16 + 8*(lane & 1);
                 if (xx < W && n0 < a.cout)
                     *reinterpret_cast<bf16x8*>(
                         a.y + size_t((zz*H + yy)*W + xx)*a.ldy + n0) =
@@ -360,6 +363,213 @@ __global__ __launch_bounds__(64) void k_conv_wgrad(WgradArgs a)
     }
 }
 
+// Weight gradient of a 3x3x3 convolution from LDS (and the bias gradient,
+// the column sums of dZ).  The product reduces over voxels, so its fragments
+// hold 8 voxels of one channel, while memory holds the channels of a voxel:
+// a tile of X (one voxel of halo) and of dZ is transposed 8x8 in registers on
+// its way into LDS.  Along x the tile's 8S positions are grouped by residue
+// mod S, x = x0 + r + S e, and a unit is the 16 bytes e = 0..7 of one
+// (z, y, r, channel): a tap's shift by +-1 in x is then another residue, and
+// residues -1 and S are kept too, so that every fragment is one aligned
+// 16-byte read.  A K step of the matrix instruction takes 32 voxels: S
+// residues of 4/S planes at one y (S = 4, 2, 1 for rows of at least 17, 9
+// and 1 voxels, so that short rows do not multiply zeros).
+// A workgroup owns 16 input channels (all 8 of the first layer, two taps per
+// 16 columns) and 16 NT output channels for all 27 taps, its four wavefronts
+// a quarter of the taps each, the accumulators in registers over all tiles
+// of its share; shares are summed by k_wgrad_sum in a fixed order.  Units are
+// placed at channel ^ (position & 7), without which the transposed stores hit
+// one bank.
+// 64^3 training step: one 16x16 tile per wavefront, its fragments gathered
+// value by value from memory and added atomically, took 1.5 ms in 7 launches;
+// 0.15 ms in this form.
+template <int S, int NT, int CC>
+struct WgradTile {
+    static constexpr int ZG = 4/S;
+    static constexpr int YT = NT <= 2 ? 8 : 4;
+    static constexpr int XU = (ZG + 2)*(YT + 2)*(S + 2);   // positions of X
+    static constexpr int ZU = ZG*YT*S;                     // and dZ
+    static constexpr int NN = 16*NT;
+    static constexpr int LDS = (XU*CC + ZU*NN)*16;
+    static constexpr int BLOCKS = CC == 8 ? 14 : 27;       // of 16 columns
+    static constexpr int SLOTS = (BLOCKS + 1 + 3)/4;       // with the bias
+};
+
+// Transposes 8 voxels x 8 channels into the units of the 8 channels.
+__device__ __forceinline__ void store_units(bf16* lds, int unit0, int sw,
+                                            const bf16x8 (&v)[8])
+{
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+    {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = v[e][c];
+        *reinterpret_cast<bf16x8*>(lds + 8*(unit0 + (c ^ sw))) = o;
+    }
+}
+
+template <int S, int NT, int CC>
+__global__ __launch_bounds__(256) void k_wgrad_lds(WgradArgs a, int nsplit,
+                                                   float* partial)
+{
+    using Tl = WgradTile<S, NT, CC>;
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    bf16* lx = reinterpret_cast<bf16*>(lds_raw);
+    bf16* lz = lx + 8*Tl::XU*CC;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 15, g = lane >> 4;
+    const int gs = g % S, gz = g/S;
+    const int c0 = CC == 8 ? 0 : blockIdx.x*16;
+    const int n0 = blockIdx.y*Tl::NN;
+    const int W = a.g.W, H = a.g.H, D = a.g.D;
+    const int ntx = (W + 8*S - 1)/(8*S), nty = (H + Tl::YT - 1)/Tl::YT;
+    const int ntz = (D + Tl::ZG - 1)/Tl::ZG;
+    floatx4 acc[Tl::SLOTS][NT];
+#pragma unroll
+    for (int i = 0; i < Tl::SLOTS; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 ones;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ones[i] = __bf16(1.0f);
+    // position offset of this lane's tap in each slot, and its channel
+    int off[Tl::SLOTS];
+#pragma unroll
+    for (int i = 0; i < Tl::SLOTS; i++)
+    {
+        const int blk = wave + 4*i;
+        const int t = min(CC == 8 ? 2*blk + (row >> 3) : blk, 26);
+        off[i] = ((t/9)*(Tl::YT + 2) + (t/3) % 3)*(S + 2) + t % 3;
+    }
+    const int ch = CC == 8 ? row & 7 : row;
+    const int ntiles = ntx*nty*ntz;
+    for (int tile = blockIdx.z; tile < ntiles; tile += nsplit)
+    {
+        const int x0 = (tile % ntx)*8*S;
+        const int y0 = ((tile/ntx) % nty)*Tl::YT;
+        const int z0 = (tile/(ntx*nty))*Tl::ZG;
+        if (tile != int(blockIdx.z)) __syncthreads();
+        constexpr int CP = CC/8, NP = Tl::NN/8;
+        for (int u = tid; u < Tl::XU*CP; u += 256)
+        {
+            const int part = u % CP, pos = u/CP;
+            const int ss = pos % (S + 2), r = pos/(S + 2);
+            const int gy = y0 - 1 + r % (Tl::YT + 2);
+            const int gz_ = z0 - 1 + r/(Tl::YT + 2);
+            const bool in = gy >= 0 && gy < H && gz_ >= 0 && gz_ < D;
+            const bf16* src = a.x + size_t((gz_*H + gy)*W)*a.ldx + c0 + 8*part;
+            bf16x8 v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+            {
+                const int gx = x0 - 1 + ss + S*e;
+                v[e] = in && gx >= 0 && gx < W
+                           ? *reinterpret_cast<const bf16x8*>(
+                                 src + ptrdiff_t(gx)*a.ldx)
+                           : zero8();
+            }
+            store_units(lx, pos*CC + 8*part, pos & 7, v);
+        }
+        for (int u = tid; u < Tl::ZU*NP; u += 256)
+        {
+            const int part = u % NP, pos = u/NP;
+            const int ss = pos % S, r = pos/S;
+            const int gy = y0 + r % Tl::YT, gz_ = z0 + r/Tl::YT;
+            const bool in = gy < H && gz_ < D;
+            const bf16* src = a.dz + size_t((gz_*H + gy)*W)*a.lddz + n0 +
+                              8*part;
+            bf16x8 v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+            {
+                const int gx = x0 + ss + S*e;
+                v[e] = in && gx < W ? *reinterpret_cast<const bf16x8*>(
+                                          src + ptrdiff_t(gx)*a.lddz)
+                                    : zero8();
+            }
+            store_units(lz, pos*Tl::NN + 8*part, pos & 7, v);
+        }
+        __syncthreads();
+#pragma unroll 1
+        for (int y = 0; y < Tl::YT; y++)
+        {
+            const int pz = (gz*Tl::YT + y)*S + gs;
+            bf16x8 av[NT];
+#pragma unroll
+            for (int j = 0; j < NT; j++)
+                av[j] = *reinterpret_cast<const bf16x8*>(
+                    lz + 8*(pz*Tl::NN + ((16*j + row) ^ (pz & 7))));
+            const int px = (gz*(Tl::YT + 2) + y)*(S + 2) + gs;
+#pragma unroll
+            for (int i = 0; i < Tl::SLOTS; i++)
+            {
+                const int blk = wave + 4*i;
+                if (blk > Tl::BLOCKS) continue;
+                bf16x8 bv = ones;
+                if (blk < Tl::BLOCKS)
+                {
+                    const int p = px + off[i];
+                    bv = *reinterpret_cast<const bf16x8*>(
+                        lx + 8*(p*CC + (ch ^ (p & 7))));
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        av[j], bv, acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+    // lane: column blk*16 + row, rows n = 4*(lane/16) + r of tile j
+    float* out = partial + size_t(blockIdx.z)*a.cout*(a.kp + 1);
+#pragma unroll
+    for (int i = 0; i < Tl::SLOTS; i++)
+    {
+        const int blk = wave + 4*i;
+        if (blk > Tl::BLOCKS) continue;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+            {
+                const int n = n0 + 16*j + 4*g + r;
+                if (blk < Tl::BLOCKS)
+                {
+                    const int k = CC == 8 ? blk*16 + row
+                                          : blk*a.cin + c0 + row;
+                    if (k < 27*a.cin) out[size_t(n)*a.kp + k] = acc[i][j][r];
+                }
+                else if (row == 0 && blockIdx.x == 0)
+                    out[size_t(a.cout)*a.kp + n] = acc[i][j][r];
+            }
+    }
+}
+
+// dw[i] += sum of the shares' partials (the bias gradients follow the
+// weights'; padding columns are left alone).  64 values per workgroup, four
+// groups of shares, summed in a fixed order.
+__global__ __launch_bounds__(256) void k_wgrad_sum(const float* partial,
+                                                   int nsplit, int cout,
+                                                   int kp, int used, int n,
+                                                   float* dw)
+{
+    __shared__ float sm[4][64];
+    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int i = blockIdx.x*64 + lane;
+    const size_t stride = size_t(cout)*(kp + 1);
+    const bool on = i < n && (i >= cout*kp || i % kp < used);
+    float s = 0.0f;
+    if (on)
+    {
+#pragma unroll 8
+        for (int k = q; k < nsplit; k += 4) s += partial[k*stride + i];
+    }
+    sm[q][lane] = s;
+    __syncthreads();
+    if (q == 0 && on)
+        dw[i] += (sm[0][lane] + sm[1][lane]) + (sm[2][lane] + sm[3][lane]);
+}
+
 // W'[c][t'*Cout + n] = W[n][(26 - t')*Cin + c]: the weights of the data
 // gradient, a forward convolution of dZ with flipped taps and swapped
 // channels.
@@ -378,17 +588,6 @@ __global__ void k_flip_weights(const bf16* w, int cin, int cout, int kp,
         v = w[size_t(n)*kp + tsrc*cin + c];
     }
     wt[i] = v;
-}
-
-// dZ = dY where Y > 0 (ReLU), in place on a channel slice.
-__global__ void k_relu_bwd(bf16* dy, int lddy, const bf16* y, int ldy, int M,
-                           int C)
-{
-    const long i = long(blockIdx.x)*blockDim.x + threadIdx.x;
-    if (i >= long(M)*C) return;
-    const int m = int(i/C), c = int(i - long(m)*C);
-    if (!(bf2f(y[size_t(m)*ldy + c]) > 0.0f))
-        dy[size_t(m)*lddy + c] = bf16(0.0f);
 }
 
 // 2x2x2 average pooling of a channel slice (fine grid g) into a coarse one.
@@ -412,19 +611,30 @@ __global__ void k_pool(const bf16* x, int ldx, Grid3 g, int C, bf16* y,
 }
 
 // Gradient of the pooling: every fine voxel receives dY/8 of its parent,
-// added to dX (which already holds the skip-connection gradient).
-__global__ void k_pool_bwd(const bf16* dy, int lddy, Grid3 g, int C, bf16* dx,
-                           int lddx)
+// added to dX (which already holds the skip-connection gradient), times the
+// ReLU mask of the fine activation y; 8 channels per thread.
+__global__ void k_pool_relu_bwd8(const bf16* dy, int lddy, Grid3 g, int C,
+                                 const bf16* y, int ldy, bf16* dx, int lddx)
 {
+    const int C8 = C/8;
     const long i = long(blockIdx.x)*blockDim.x + threadIdx.x;
-    if (i >= long(g.D)*g.H*g.W*C) return;
-    const int c = int(i % C);
-    const int m = int(i/C);
-    const int x = m % g.W, y = (m/g.W) % g.H, z = m/(g.W*g.H);
-    const int mc = ((z/2)*(g.H/2) + y/2)*(g.W/2) + x/2;
-    const float v = bf2f(dx[size_t(m)*lddx + c]) +
-                    0.125f*bf2f(dy[size_t(mc)*lddy + c]);
-    dx[size_t(m)*lddx + c] = bf16(v);
+    if (i >= long(g.D)*g.H*g.W*C8) return;
+    const int c = int(i % C8)*8;
+    const int m = int(i/C8);
+    const int x = m % g.W, yy = (m/g.W) % g.H, z = m/(g.W*g.H);
+    const int mc = ((z/2)*(g.H/2) + yy/2)*(g.W/2) + x/2;
+    bf16x8* const out = reinterpret_cast<bf16x8*>(dx + size_t(m)*lddx + c);
+    const bf16x8 act = *reinterpret_cast<const bf16x8*>(y + size_t(m)*ldy + c);
+    const bf16x8 up = *reinterpret_cast<const bf16x8*>(dy + size_t(mc)*lddy + c);
+    const bf16x8 old = *out;
+    bf16x8 o;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+    {
+        const float v = float(old[q]) + 0.125f*float(up[q]);
+        o[q] = float(act[q]) > 0.0f ? bf16(v) : bf16(0.0f);
+    }
+    *out = o;
 }
 
 // Nearest-neighbour upsampling by 2 of a coarse channel slice into a fine
@@ -485,24 +695,37 @@ __global__ void k_pool8(const bf16* x, int ldx, Grid3 g, int C, bf16* y,
     *reinterpret_cast<bf16x8*>(y + size_t(mc)*ldy + c) = o;
 }
 
-// Gradient of the upsampling: the coarse voxel sums its 8 children.
-__global__ void k_up_bwd(const bf16* dy, int lddy, Grid3 g, int C, bf16* dx,
-                         int lddx)
+// Gradient of the upsampling, the coarse voxel summing its 8 children, times
+// the ReLU mask of the coarse activation y, on 8 channels per thread (16-byte
+// loads and stores).
+__global__ void k_up_relu_bwd8(const bf16* dy, int lddy, Grid3 g, int C,
+                               const bf16* y, int ldy, bf16* dx, int lddx)
 {
-    const int Dc = g.D/2, Hc = g.H/2, Wc = g.W/2;
+    const int Dc = g.D/2, Hc = g.H/2, Wc = g.W/2, C8 = C/8;
     const long i = long(blockIdx.x)*blockDim.x + threadIdx.x;
-    if (i >= long(Dc)*Hc*Wc*C) return;
-    const int c = int(i % C);
-    const int mc = int(i/C);
+    if (i >= long(Dc)*Hc*Wc*C8) return;
+    const int c = int(i % C8)*8;
+    const int mc = int(i/C8);
     const int xc = mc % Wc, yc = (mc/Wc) % Hc, zc = mc/(Wc*Hc);
-    float s = 0.0f;
+    const bf16x8 act = *reinterpret_cast<const bf16x8*>(y + size_t(mc)*ldy + c);
+    float s[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) s[q] = 0.0f;
+#pragma unroll
     for (int d = 0; d < 8; d++)
     {
         const int zf = 2*zc + (d >> 2), yf = 2*yc + ((d >> 1) & 1),
                   xf = 2*xc + (d & 1);
-        s += bf2f(dy[size_t((zf*g.H + yf)*g.W + xf)*lddy + c]);
+        const bf16x8 v = *reinterpret_cast<const bf16x8*>(
+            dy + size_t((zf*g.H + yf)*g.W + xf)*lddy + c);
+#pragma unroll
+        for (int q = 0; q < 8; q++) s[q] += float(v[q]);
     }
-    dx[size_t(mc)*lddx + c] = bf16(s);
+    bf16x8 o;
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+        o[q] = float(act[q]) > 0.0f ? bf16(s[q]) : bf16(0.0f);
+    *reinterpret_cast<bf16x8*>(dx + size_t(mc)*lddx + c) = o;
 }
 
 // Output projection (1x1x1, 16 channels -> 1, FP32; w[16] is the bias)
@@ -518,15 +741,16 @@ __global__ void k_head_fwd(const bf16* x, int ldx, int M, const float* w,
     out[m] = s;
 }
 
-// dX[m][c] = g[m] * w[c]; per-block partial sums of g[m]*X[m][c] (16
-// channels) and of g[m] for the weight and bias gradients.
+// dX[m][c] = g[m] * w[c] where X > 0 (X is a ReLU's output); per-block
+// partial sums of g[m]*X[m][c] (16 channels) and of g[m] for the weight and
+// bias gradients.
 __global__ __launch_bounds__(256) void k_head_bwd(const bf16* x, int ldx,
                                                   int M, const float* w,
                                                   const float* gout,
                                                   bf16* dx, int lddx,
                                                   float* partial)
 {
-    __shared__ float sm[17][256];
+    __shared__ float sm[17][4];
     const int m = blockIdx.x*256 + threadIdx.x;
     float gw[17];
 #pragma unroll
@@ -535,25 +759,36 @@ __global__ __launch_bounds__(256) void k_head_bwd(const bf16* x, int ldx,
     {
         const float g = gout[m];
 #pragma unroll
-        for (int c = 0; c < 16; c++)
+        for (int h = 0; h < 2; h++)
         {
-            gw[c] = g*bf2f(x[size_t(m)*ldx + c]);
-            dx[size_t(m)*lddx + c] = bf16(g*w[c]);
+            const bf16x8 v = *reinterpret_cast<const bf16x8*>(
+                x + size_t(m)*ldx + 8*h);
+            bf16x8 o;
+#pragma unroll
+            for (int c = 0; c < 8; c++)
+            {
+                const float xv = float(v[c]);
+                gw[8*h + c] = g*xv;
+                o[c] = xv > 0.0f ? bf16(g*w[8*h + c]) : bf16(0.0f);
+            }
+            *reinterpret_cast<bf16x8*>(dx + size_t(m)*lddx + 8*h) = o;
         }
         gw[16] = g;
     }
+    // within the wavefront, then the four wavefronts in order
 #pragma unroll
-    for (int c = 0; c < 17; c++) sm[c][threadIdx.x] = gw[c];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1)
+    for (int c = 0; c < 17; c++)
     {
-        if (int(threadIdx.x) < s)
-            for (int c = 0; c < 17; c++)
-                sm[c][threadIdx.x] += sm[c][threadIdx.x + s];
-        __syncthreads();
+        for (int o = 32; o > 0; o >>= 1) gw[c] += __shfl_xor(gw[c], o, 64);
+        if ((threadIdx.x & 63) == 0) sm[c][threadIdx.x >> 6] = gw[c];
     }
-    if (threadIdx.x < 17) partial[size_t(blockIdx.x)*17 + threadIdx.x] =
-        sm[threadIdx.x][0];
+    __syncthreads();
+    if (threadIdx.x < 17)
+    {
+        const float* v = sm[threadIdx.x];
+        partial[size_t(blockIdx.x)*17 + threadIdx.x] =
+            (v[0] + v[1]) + (v[2] + v[3]);
+    }
 }
 
 // Mean-removed squared error: loss partials and the output gradient
@@ -598,22 +833,57 @@ __global__ __launch_bounds__(256) void k_diff_sum(const float* a,
     if (threadIdx.x == 0) partial[blockIdx.x] = sm[0];
 }
 
-// out[0..cols) = scale * column sums of an rows x cols FP32 array (one
-// thread per column, fixed order).
-__global__ void k_col_sum(const float* in, int rows, int cols, float scale,
-                          float* out)
+// out[c] = scale * sum of column c of a rows x cols FP32 array: one
+// workgroup per column, fixed order (one thread per column took 41 us for
+// 1024 rows, each addition waiting for its load).
+__global__ __launch_bounds__(256) void k_col_sum(const float* in, int rows,
+                                                 int cols, float scale,
+                                                 float* out)
 {
-    const int c = blockIdx.x*blockDim.x + threadIdx.x;
-    if (c >= cols) return;
+    __shared__ float sm[4];
+    const int c = blockIdx.x;
     float s = 0.0f;
-    for (int r = 0; r < rows; r++) s += in[size_t(r)*cols + c];
-    out[c] = scale*s;
+#pragma unroll 4
+    for (int r = threadIdx.x; r < rows; r += 256) s += in[size_t(r)*cols + c];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) out[c] = scale*((sm[0] + sm[1]) + (sm[2] + sm[3]));
 }
 
-// Adam on FP32 master weights, refreshing the BF16 copy.
-__global__ void k_adam(float* w, float* mo, float* ve, const float* g, int n,
-                       float lr, float b1, float b2, float eps, float c1,
-                       float c2, bf16* wb)
+// The BF16 copies of parameter i of the network: the weights [n][k] and, for
+// the data gradient, the flipped ones wt[c][t'*cout + n] = w[n][(26-t')*cin +
+// c]; biases and the head have none.
+__device__ __forceinline__ void refresh_weight(const WeightViews& v, int i,
+                                               float w)
+{
+#pragma unroll
+    for (int q = 0; q < WeightViews::LAYERS; q++)
+    {
+        const WeightView& l = v.l[q];
+        const int j = i - l.off;
+        if (j < 0 || j >= l.cout*l.kp) continue;
+        const bf16 b = bf16(w);
+        l.w[j] = b;
+        const int n = j/l.kp, k = j - n*l.kp;
+        if (l.wt && k < 27*l.cin)
+        {
+            const int t = k/l.cin, c = k - t*l.cin;
+            l.wt[size_t(c)*l.kpt + (26 - t)*l.cout + n] = b;
+        }
+    }
+}
+
+__global__ void k_refresh(WeightViews v, const float* w, int n)
+{
+    const int i = blockIdx.x*blockDim.x + threadIdx.x;
+    if (i < n) refresh_weight(v, i, w[i]);
+}
+
+// Adam on the FP32 master weights, with their BF16 copies.
+__global__ void k_adam(WeightViews views, float* w, float* mo, float* ve,
+                       const float* g, int n, float lr, float b1, float b2,
+                       float eps, float c1, float c2)
 {
     const int i = blockIdx.x*blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -624,13 +894,7 @@ __global__ void k_adam(float* w, float* mo, float* ve, const float* g, int n,
     ve[i] = v;
     const float wi = w[i] - lr*(m/c1)/(sqrtf(v/c2) + eps);
     w[i] = wi;
-    if (wb) wb[i] = bf16(wi);
-}
-
-__global__ void k_to_bf16(const float* a, bf16* b, long n)
-{
-    const long i = long(blockIdx.x)*blockDim.x + threadIdx.x;
-    if (i < n) b[i] = bf16(a[i]);
+    refresh_weight(views, i, wi);
 }
 
 // Network input from the solver's FP64 colour-split level-0 fields is built
@@ -653,8 +917,8 @@ inline unsigned nblk(long n, int b) { return unsigned((n + b - 1)/b); }
 
 namespace {
 
-template <int NT, int MT, int CIN>
-void launch_conv_lds(const ConvArgs& a, hipStream_t s)
+template <int NT, int MT, int CIN, int AS>
+void launch_conv_lds(const ConvArgs& a, hipStream_t s, int groups = 1)
 {
     using Tl = ConvTile<MT>;
     const int ch = CIN > 0 ? CIN : 32;
@@ -663,8 +927,8 @@ void launch_conv_lds(const ConvArgs& a, hipStream_t s)
     const unsigned nb = unsigned((a.g.W + 15)/16)*
                         unsigned((a.g.H + Tl::TY - 1)/Tl::TY)*
                         unsigned((a.g.D + Tl::TZ - 1)/Tl::TZ);
-    hipLaunchKernelGGL((k_conv_fwd_lds<NT, MT, CIN>), dim3(nb), dim3(256), shm,
-                       s, a);
+    hipLaunchKernelGGL((k_conv_fwd_lds<NT, MT, CIN, AS>), dim3(nb, groups),
+                       dim3(256), shm, s, a);
 }
 
 template <int NT, int CIN>
@@ -675,7 +939,23 @@ void conv_lds_mt(const ConvArgs& a, hipStream_t s)
     constexpr bool fit4 = ConvTile<4>::HV*(ch + 8)*2 <= 65536;
     constexpr bool fit2 = ConvTile<2>::HV*(ch + 8)*2 <= 65536;
     constexpr int MT = (MT0 >= 4 && fit4) ? 4 : ((MT0 >= 2 && fit2) ? 2 : 1);
-    launch_conv_lds<NT, MT, CIN>(a, s);
+    constexpr int AS = NT*MT <= 8 ? 2 : 1;
+    using Tl = ConvTile<MT>;
+    const long nb = long((a.g.W + 15)/16)*((a.g.H + Tl::TY - 1)/Tl::TY)*
+                    ((a.g.D + Tl::TZ - 1)/Tl::TZ);
+    if (nb < 256 && (MT > 1 || NT > 2))
+    {
+        // a small grid fills too few of the 256 compute units with large
+        // tiles: 64 voxels by 16 or 32 channels per workgroup, the k steps
+        // summed as the large tile sums them (192 -> 64 channels at 16^3: 16
+        // workgroups 106 us, 128 workgroups 35 us)
+        if (NT % 2 == 0)
+            launch_conv_lds<2, 1, CIN, AS>(a, s, NT/2);
+        else
+            launch_conv_lds<1, 1, CIN, AS>(a, s, NT);
+        return;
+    }
+    launch_conv_lds<NT, MT, CIN, AS>(a, s);
 }
 
 // Output tiles per wavefront: at most 16 accumulator tiles (NT x MT), and
@@ -730,8 +1010,84 @@ void conv_fwd(const ConvArgs& a, hipStream_t s)
     }
 }
 
-void conv_wgrad(const WgradArgs& a, hipStream_t s)
+namespace {
+
+template <int S, int NT, int CC>
+int wgrad_lds(const WgradArgs& a, int nsplit, float* partial, hipStream_t s)
 {
+    using Tl = WgradTile<S, NT, CC>;
+    static_assert(Tl::LDS <= 65536, "tile exceeds 64 KB of LDS");
+    const int ntiles = ((a.g.W + 8*S - 1)/(8*S))*
+                       ((a.g.H + Tl::YT - 1)/Tl::YT)*
+                       ((a.g.D + Tl::ZG - 1)/Tl::ZG);
+    const int gx = CC == 8 ? 1 : a.cin/16, gy = a.cout/Tl::NN;
+    // about two workgroups per compute unit
+    const int n = std::max(1, std::min({ntiles, nsplit, 512/(gx*gy)}));
+    hipLaunchKernelGGL((k_wgrad_lds<S, NT, CC>), dim3(gx, gy, n), dim3(256),
+                       Tl::LDS, s, a, n, partial);
+    return n;
+}
+
+template <int S, int NT>
+int wgrad_cc(const WgradArgs& a, int nsplit, float* partial, hipStream_t s)
+{
+    return a.cin == 8 ? wgrad_lds<S, NT, 8>(a, nsplit, partial, s)
+                      : wgrad_lds<S, NT, 16>(a, nsplit, partial, s);
+}
+
+template <int S>
+int wgrad_nt(const WgradArgs& a, int nsplit, float* partial, hipStream_t s)
+{
+    if (a.cout % 64 == 0) return wgrad_cc<S, 4>(a, nsplit, partial, s);
+    if (a.cout % 32 == 0) return wgrad_cc<S, 2>(a, nsplit, partial, s);
+    return wgrad_cc<S, 1>(a, nsplit, partial, s);
+}
+
+}  // namespace
+
+size_t wgrad_workspace(const WgradArgs& a)
+{
+    const bool tiled = a.taps == 27 && (a.cin == 8 || a.cin % 16 == 0) &&
+                       a.cout % 16 == 0 && a.ldx % 8 == 0 &&
+                       a.lddz % 8 == 0 &&
+                       reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
+                       reinterpret_cast<uintptr_t>(a.dz) % 16 == 0;
+    if (!tiled) return 0;
+    // at most 512 workgroups, one share each; at least two tiles a share
+    // where the grid has them
+    const int S = a.g.W > 16 ? 4 : (a.g.W > 8 ? 2 : 1);
+    const int nt = a.cout % 64 == 0 ? 4 : (a.cout % 32 == 0 ? 2 : 1);
+    const int yt = nt <= 2 ? 8 : 4, zg = 4/S;
+    const long tiles = long((a.g.W + 8*S - 1)/(8*S))*((a.g.H + yt - 1)/yt)*
+                       ((a.g.D + zg - 1)/zg);
+    const int groups = (a.cin == 8 ? 1 : a.cin/16)*(a.cout/(16*nt));
+    const long n = std::max(1L, std::min(tiles, long(512/groups)));
+    return size_t(n)*a.cout*(a.kp + 1);
+}
+
+// Shapes and alignments the tiled kernel takes (wgrad_workspace > 0) go to
+// it; any other goes to the general one (its bias gradient is then the
+// caller's).
+void conv_wgrad(const WgradArgs& a, float* workspace, float* dbias,
+                hipStream_t s)
+{
+    const size_t need = wgrad_workspace(a);
+    if (need && workspace)
+    {
+        const int S = a.g.W > 16 ? 4 : (a.g.W > 8 ? 2 : 1);
+        const int nsplit = int(need/(size_t(a.cout)*(a.kp + 1)));
+        const int n = S == 4 ? wgrad_nt<4>(a, nsplit, workspace, s)
+                    : (S == 2 ? wgrad_nt<2>(a, nsplit, workspace, s)
+                              : wgrad_nt<1>(a, nsplit, workspace, s));
+        // dbias, when asked for, follows the weights
+        const int total = a.cout*a.kp + (dbias ? a.cout : 0);
+        if (dbias && dbias != a.dw + size_t(a.cout)*a.kp)
+            throw UnetError("bias gradient must follow the weights'");
+        hipLaunchKernelGGL(k_wgrad_sum, dim3(nblk(total, 64)), dim3(256), 0, s,
+                           workspace, n, a.cout, a.kp, 27*a.cin, total, a.dw);
+        return;
+    }
+    if (dbias) throw UnetError("weight gradient shape not supported");
     const int M = a.g.D*a.g.H*a.g.W;
     const int K = a.taps*a.cin;
     const dim3 g(nblk(K, 16), nblk(a.cout, 16), nblk(M, a.chunk));
@@ -743,13 +1099,6 @@ void flip_weights(const bf16* w, int cin, int cout, int kp, int taps, bf16* wt,
 {
     hipLaunchKernelGGL(k_flip_weights, dim3(nblk(long(cin)*kpt, 256)),
                        dim3(256), 0, s, w, cin, cout, kp, taps, wt, kpt);
-}
-
-void relu_bwd(bf16* dy, int lddy, const bf16* y, int ldy, int M, int C,
-              hipStream_t s)
-{
-    hipLaunchKernelGGL(k_relu_bwd, dim3(nblk(long(M)*C, 256)), dim3(256), 0, s,
-                       dy, lddy, y, ldy, M, C);
 }
 
 void pool(const bf16* x, int ldx, Grid3 g, int C, bf16* y, int ldy,
@@ -766,12 +1115,12 @@ void pool(const bf16* x, int ldx, Grid3 g, int C, bf16* y, int ldy,
                            ldx, g, C, y, ldy);
 }
 
-void pool_bwd(const bf16* dy, int lddy, Grid3 g, int C, bf16* dx, int lddx,
-              hipStream_t s)
+void pool_relu_bwd(const bf16* dy, int lddy, Grid3 g, int C, const bf16* y,
+                   int ldy, bf16* dx, int lddx, hipStream_t s)
 {
-    const long n = long(g.D)*g.H*g.W*C;
-    hipLaunchKernelGGL(k_pool_bwd, dim3(nblk(n, 256)), dim3(256), 0, s, dy,
-                       lddy, g, C, dx, lddx);
+    const long n = long(g.D)*g.H*g.W*C/8;
+    hipLaunchKernelGGL(k_pool_relu_bwd8, dim3(nblk(n, 256)), dim3(256), 0, s,
+                       dy, lddy, g, C, y, ldy, dx, lddx);
 }
 
 void up(const bf16* x, int ldx, Grid3 g, int C, bf16* y, int ldy,
@@ -788,12 +1137,12 @@ void up(const bf16* x, int ldx, Grid3 g, int C, bf16* y, int ldy,
                            C, y, ldy);
 }
 
-void up_bwd(const bf16* dy, int lddy, Grid3 g, int C, bf16* dx, int lddx,
-            hipStream_t s)
+void up_relu_bwd(const bf16* dy, int lddy, Grid3 g, int C, const bf16* y,
+                 int ldy, bf16* dx, int lddx, hipStream_t s)
 {
-    const long n = long(g.D/2)*(g.H/2)*(g.W/2)*C;
-    hipLaunchKernelGGL(k_up_bwd, dim3(nblk(n, 256)), dim3(256), 0, s, dy, lddy,
-                       g, C, dx, lddx);
+    const long n = long(g.D/2)*(g.H/2)*(g.W/2)*C/8;
+    hipLaunchKernelGGL(k_up_relu_bwd8, dim3(nblk(n, 256)), dim3(256), 0, s, dy,
+                       lddy, g, C, y, ldy, dx, lddx);
 }
 
 void head_fwd(const bf16* x, int ldx, int M, const float* w, float* out,
@@ -832,22 +1181,25 @@ int diff_sum(const float* a, const float* b, int M, float* partial,
 void col_sum(const float* in, int rows, int cols, float scale, float* out,
              hipStream_t s)
 {
-    hipLaunchKernelGGL(k_col_sum, dim3(nblk(cols, 64)), dim3(64), 0, s, in,
-                       rows, cols, scale, out);
+    hipLaunchKernelGGL(k_col_sum, dim3(cols), dim3(256), 0, s, in, rows, cols,
+                       scale, out);
 }
 
-void adam(float* w, float* m, float* v, const float* g, int n, float lr,
-          float b1, float b2, float eps, int step, bf16* wb, hipStream_t s)
+void adam(const WeightViews& views, float* w, float* m, float* v,
+          const float* g, int n, float lr, float b1, float b2, float eps,
+          int step, hipStream_t s)
 {
     const float c1 = 1.0f - powf(b1, float(step));
     const float c2 = 1.0f - powf(b2, float(step));
-    hipLaunchKernelGGL(k_adam, dim3(nblk(n, 256)), dim3(256), 0, s, w, m, v, g,
-                       n, lr, b1, b2, eps, c1, c2, wb);
+    hipLaunchKernelGGL(k_adam, dim3(nblk(n, 256)), dim3(256), 0, s, views, w,
+                       m, v, g, n, lr, b1, b2, eps, c1, c2);
 }
 
-void to_bf16(const float* a, bf16* b, long n, hipStream_t s)
+void refresh_weights(const WeightViews& views, const float* w, int n,
+                     hipStream_t s)
 {
-    hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n, 256)), dim3(256), 0, s, a, b, n);
+    hipLaunchKernelGGL(k_refresh, dim3(nblk(n, 256)), dim3(256), 0, s, views,
+                       w, n);
 }
 
 void pack_input(const float* f, const float* lam, int M, bf16* x,

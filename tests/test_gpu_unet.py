@@ -255,3 +255,42 @@ def test_what_training_gains(gpu, capsys):
                   f"{it['fcg'][0]} without the network, "
                   f"{it['fcg_learned'][0]} with it (guess residual "
                   f"{it['fcg_learned'][1]:.3g} of the zero guess's)")
+
+
+@pytest.mark.parametrize("shape", [(3, 5, 7), (6, 9, 16), (5, 17, 33),
+                                   (4, 8, 40), (2, 4, 8)])
+@pytest.mark.parametrize("cin,cout", [(8, 16), (16, 32), (48, 16), (32, 64),
+                                      (64, 128)])
+def test_wgrad_tiles(gpu, shape, cin, cout):
+    """The tiled weight gradient at rows of every residue grouping (at most 8,
+    9 to 16, above), partial tiles on each axis and all output groupings;
+    exact BF16 products summed in FP32 (bound as above)."""
+    r = np.random.default_rng(cin + cout)
+    x = U.to_bf16(r.standard_normal(shape + (cin,)).astype(np.float32))
+    dz = U.to_bf16(r.standard_normal(shape + (cout,)).astype(np.float32))
+    kp = unet.round32(27 * cin)
+    ref = U.conv_wgrad(x, dz, kp)
+    got = unet.op_conv_wgrad(dev_bf16(x), dev_bf16(dz), kp).cpu().numpy()
+    assert np.abs(got - ref).max() < 1e-4 * np.abs(ref).max()
+    assert np.all(got[:, 27 * cin:] == 0.0)
+
+
+@pytest.mark.parametrize("shape,cin,cout", [((4, 6, 20), 192, 64),
+                                            ((8, 8, 8), 64, 128),
+                                            ((5, 3, 17), 48, 48),
+                                            ((16, 16, 16), 64, 192)])
+def test_small_grid_forward(gpu, shape, cin, cout):
+    """Grids of few tiles take output channels in groups over workgroups."""
+    r = np.random.default_rng(cin)
+    x = U.to_bf16(r.standard_normal(shape + (cin,)).astype(np.float32))
+    kp = unet.round32(27 * cin)
+    w = np.zeros((cout, kp), np.float32)
+    w[:, :27 * cin] = U.to_bf16(
+        (r.standard_normal((cout, 27 * cin)) / np.sqrt(27 * cin)).astype(
+            np.float32))
+    bias = r.standard_normal(cout).astype(np.float32)
+    ref = U.conv(x, w[:, :27 * cin], bias, relu=True)
+    y = unet.op_conv(dev_bf16(x), dev_bf16(w), torch.from_numpy(bias).cuda(),
+                     cout, True).float().cpu().numpy()
+    # one BF16 rounding of the result and FP32 sums
+    assert np.abs(y - ref).max() <= 2.0**-8 * np.abs(ref).max()

@@ -81,7 +81,11 @@ const ConvSpec kConvs[7] = {{8, 16, 2, 0},    {16, 32, 16, 1},
 struct Acts {
     Grid3 g[4];
     int M[4];
-    bf16* xin = nullptr;       // M0 x 8
+    // inference: the skip tensors E0, E1, E2 (M0x16, M1x32, M2x64); training
+    // keeps them inside cat
+    bf16* skip[3] = {nullptr, nullptr, nullptr};
+    // training: packed input (M0 x 8) and [up | skip] of each level
+    bf16* xin = nullptr;
     bf16* cat[3] = {nullptr, nullptr, nullptr};  // M0x48, M1x96, M2x192
     bf16* pin[4] = {nullptr, nullptr, nullptr, nullptr};  // pooled inputs
                                                           // of E1..E3 (1..3)
@@ -112,6 +116,7 @@ struct Acts {
         for (int i = 0; i < 3; i++)
         {
             dfree(cat[i]); dfree(yd[i]); dfree(dcat[i]); dfree(dyd[i]);
+            dfree(skip[i]);
         }
         for (int i = 0; i < 4; i++) { dfree(pin[i]); dfree(dpin[i]); }
     }
@@ -206,28 +211,36 @@ struct Net {
         if (D % 8 || H % 8 || W % 8 || D < 8 || H < 8 || W < 8)
             throw UnetError("U-Net grid extents must be multiples of 8");
         Acts& a = acts;
-        const bool same = a.xin && a.g[0].D == D && a.g[0].H == H &&
+        const bool same = a.y3 && a.g[0].D == D && a.g[0].H == H &&
                           a.g[0].W == W;
         if (same && (!train || a.train)) return;
         a.freeAll();
+        a.train = false;
         for (int l = 0; l < 4; l++)
         {
             a.g[l] = Grid3{D >> l, H >> l, W >> l};
             a.M[l] = a.g[l].D*a.g[l].H*a.g[l].W;
         }
-        a.xin = dalloc<bf16>(size_t(a.M[0])*8);
         for (int l = 0; l < 3; l++)
         {
-            a.cat[l] = dalloc<bf16>(size_t(a.M[l])*kCatC[l]);
-            a.yd[l] = dalloc<bf16>(size_t(a.M[l])*kDecC[l]);
+            if (train)
+                a.cat[l] = dalloc<bf16>(size_t(a.M[l])*kCatC[l]);
+            else
+                a.skip[l] = dalloc<bf16>(size_t(a.M[l])*kDecC[l]);
+            // the first decoder output is only kept for the backward pass
+            if (train || l > 0)
+                a.yd[l] = dalloc<bf16>(size_t(a.M[l])*kDecC[l]);
         }
         for (int l = 1; l < 4; l++)
             a.pin[l] = dalloc<bf16>(size_t(a.M[l])*kPinC[l]);
         a.y3 = dalloc<bf16>(size_t(a.M[3])*128);
-        a.out = dalloc<float>(a.M[0]);
-        a.partial = dalloc<float>(size_t((a.M[0] + 255)/256)*17 + 64);
-        a.scal = dalloc<float>(4);
-        a.train = train;
+        if (train)
+        {
+            a.xin = dalloc<bf16>(size_t(a.M[0])*8);
+            a.out = dalloc<float>(a.M[0]);
+            a.partial = dalloc<float>(size_t((a.M[0] + 255)/256)*17 + 64);
+            a.scal = dalloc<float>(4);
+        }
         if (train)
         {
             for (int l = 0; l < 3; l++)
@@ -244,6 +257,7 @@ struct Net {
                 need = std::max(need, wgrad_workspace(wgrad(i, nullptr, 8,
                                                             nullptr, 8)));
             a.wgrad = dalloc<float>(need);
+            a.train = true;
         }
     }
 
@@ -266,7 +280,54 @@ struct Net {
         return a;
     }
 
-    // forward from the packed input acts.xin to acts.out
+    // Inference pass from the FP32 inputs to out: upsampling and skip
+    // concatenation are read in place by the decoder's convolutions, the
+    // encoder's write their averages, the last one the output projection.
+    // (Training keeps every activation its backward pass reads.)
+    void infer(const float* f, const float* c, float* out, hipStream_t s)
+    {
+        Acts& a = acts;
+        const bool cat = a.cat[0] != nullptr;
+        auto skip = [&](int l) { return cat ? a.cat[l] + kUpC[l] : a.skip[l]; };
+        auto ld = [&](int l) { return cat ? kCatC[l] : kDecC[l]; };
+        conv_first(a.g[0], f, c, WB[0], kp[0], P + boff[0], skip(0), ld(0),
+                   a.pin[1], 16, s);
+        // layer i from (coarse u, fine x) to y, pooled to p
+        auto layer = [&](int i, const bf16* u, int c0, const bf16* x, int ldx,
+                         bf16* y, int ldy, bf16* p)
+        {
+            TileConvArgs t{};
+            t.g = a.g[kConvs[i].level];
+            t.up = u;
+            t.ldu = c0;
+            t.c0 = c0;
+            t.x = x;
+            t.ldx = ldx;
+            t.cin = kConvs[i].cin;
+            t.w = WB[i];
+            t.kp = kp[i];
+            t.cout = kConvs[i].cout;
+            t.bias = P + boff[i];
+            t.y = y;
+            t.ldy = ldy;
+            t.pool = p;
+            t.ldp = kConvs[i].cout;
+            if (!y)
+            {
+                t.head = P + hoff;
+                t.out = out;
+            }
+            conv_rows(t, s);
+        };
+        layer(1, nullptr, 0, a.pin[1], 16, skip(1), ld(1), a.pin[2]);
+        layer(2, nullptr, 0, a.pin[2], 32, skip(2), ld(2), a.pin[3]);
+        layer(3, nullptr, 0, a.pin[3], 64, a.y3, 128, nullptr);
+        layer(4, a.y3, 128, skip(2), ld(2), a.yd[2], 64, nullptr);
+        layer(5, a.yd[2], 64, skip(1), ld(1), a.yd[1], 32, nullptr);
+        layer(6, a.yd[1], 32, skip(0), ld(0), nullptr, 0, nullptr);
+    }
+
+    // training forward from the packed input acts.xin to acts.out
     void forward(hipStream_t s)
     {
         Acts& a = acts;
@@ -415,10 +476,8 @@ void net_forward(::bmg_unet* u, int D, int H, int W, const float* f,
 {
     Net& n = *u->net;
     n.ensureActs(D, H, W, false);
-    pack_input(f, c, n.acts.M[0], n.acts.xin, s);
-    n.forward(s);
-    UCK(hipMemcpyAsync(out, n.acts.out, size_t(n.acts.M[0])*sizeof(float),
-                       hipMemcpyDeviceToDevice, s));
+    n.infer(f, c, out, s);
+    UCK(hipGetLastError());
 }
 
 }  // namespace unet
@@ -471,10 +530,7 @@ int bmg_unet_forward(bmg_unet* u, int D, int H, int W, const float* f,
     return urun([&] {
         Net& n = *u->net;
         n.ensureActs(D, H, W, false);
-        bmg::unet::pack_input(f, c, n.acts.M[0], n.acts.xin, n.stream);
-        n.forward(n.stream);
-        UCK(hipMemcpyAsync(out, n.acts.out, size_t(n.acts.M[0])*sizeof(float),
-                           hipMemcpyDeviceToDevice, n.stream));
+        n.infer(f, c, out, n.stream);
         UCK(hipGetLastError());
         UCK(hipStreamSynchronize(n.stream));
     });

@@ -38,6 +38,28 @@ struct ConvArgs {
     int ldy;
 };
 
+// One convolution of the inference pass (with bias and ReLU): the first c0
+// input channels from a tensor of half the extents through nearest-neighbour
+// upsampling, the others from x; also the 2x2x2 averages of the output
+// (pool set) or, instead of it, the output projection (head set).
+struct TileConvArgs {
+    Grid3 g;
+    const bf16* up;    // coarse tensor (extents g/2), c0 channels; or null
+    int ldu, c0;
+    const bf16* x;     // fine tensor, the remaining channels
+    int ldx;
+    int cin;
+    const bf16* w;     // [cout][kp], k = t*cin + c
+    int kp, cout;
+    const float* bias;
+    bf16* y;
+    int ldy;
+    bf16* pool;        // POOL: coarse output, row stride ldp
+    int ldp;
+    const float* head; // HEAD: 16 weights and the bias
+    float* out;
+};
+
 // dw[n][k] += sum_m dz[m][n] * x[tap_k(m)][c_k] (FP32 accumulation).
 struct WgradArgs {
     Grid3 g;
@@ -56,6 +78,12 @@ struct WgradArgs {
 inline int round32(int k) { return (k + 31)/32*32; }
 
 void conv_fwd(const ConvArgs& a, hipStream_t s);
+void conv_rows(const TileConvArgs& a, hipStream_t s);
+// The first convolution (2 real input channels, BF16 of f and c; w as E0's
+// [16][kp]) with bias and ReLU, and its averages.
+void conv_first(const Grid3& g, const float* f, const float* c, const bf16* w,
+                int kp, const float* bias, bf16* y, int ldy, bf16* pool,
+                int ldp, hipStream_t s);
 // Floats of workspace the tiled weight gradient of these arguments needs (0:
 // the general kernel takes them, without workspace).
 size_t wgrad_workspace(const WgradArgs& a);

@@ -307,6 +307,350 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
     }
 }
 
+// Forward convolution of the inference pass, 3x3x3 with bias and ReLU, input
+// channels in chunks of 16: the first c0 of them from a coarse tensor read
+// through the nearest-neighbour upsampling, the others from a fine one (the
+// skip connection), so neither the upsampled tensor nor the concatenation is
+// ever written.  A workgroup of 4 wavefronts owns 16 x TY x TZ voxels and
+// 16 NT output channels, a wavefront MT consecutive rows (y) of one plane.
+// A chunk's input tile with its halo is staged in LDS as two planes of
+// 16-byte units (8 channels of a voxel), so the 16 lanes of a fragment read
+// 256 contiguous bytes.  A K step takes 16 channels of two taps with the same
+// dy; for a pair of (dz, dx) a wavefront reads the fragments of its MT + 2
+// rows once and uses each for the three dy: 10 LDS reads for 24 NT matrix
+// instructions (MT = 8), where one read per instruction and output tile had
+// the LDS, not the matrix cores, set the time.
+// Epilogue through LDS: 16-byte stores; POOL: the 2x2x2 averages of the
+// rounded outputs (k_pool8's order) too; HEAD: only the network's 1x1x1
+// output projection of them (k_head_fwd's order), cout = 16.
+// Summed in another order than the training pass's convolutions (FP32).
+// 256^3: 48 -> 16 channels with the upsampling 3.9 ms -> TBDA, 96 -> 32 at
+// 128^3 0.94 ms -> TBDB; the whole pass 6.8 -> TBDF ms.
+template <int MT>
+struct ConvRows {
+    static constexpr int WY = 8/MT;          // wavefronts along y
+    static constexpr int TY = 8, TZ = 4/WY;
+    static constexpr int HX = 18, HY = TY + 2, HZ = TZ + 2;
+    static constexpr int HV = HX*HY*HZ;
+    static constexpr int UNITS = 2*HV;
+    static constexpr int VOX = 16*TY*TZ;
+};
+
+template <int NT, int MT, bool POOL, bool HEAD>
+__global__ __launch_bounds__(256) void k_conv_rows(TileConvArgs a)
+{
+    using Tl = ConvRows<MT>;
+    constexpr int OUT = Tl::VOX*NT*2;        // units of the output tile
+    constexpr int LDS = Tl::UNITS > OUT ? Tl::UNITS : OUT;
+    __shared__ __align__(16) bf16 lds[LDS*8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = lane & 15, g = lane >> 4;
+    const int W = a.g.W, H = a.g.H, D = a.g.D;
+    const int ntx = (W + 15)/16, nty = (H + Tl::TY - 1)/Tl::TY;
+    const int b = blockIdx.x;
+    const int x0 = (b % ntx)*16;
+    const int y0 = ((b/ntx) % nty)*Tl::TY;
+    const int z0 = (b/(ntx*nty))*Tl::TZ;
+    const int nb0 = blockIdx.y*NT*16;
+    const int wz = wave/Tl::WY, wy = (wave % Tl::WY)*MT;
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // this lane's half of the channels, and of each tap pair
+    const int half = g & 1, second = g >> 1;
+    const int base = (half*Tl::HV + (wz*Tl::HY + wy)*Tl::HX + row)*8;
+    const bf16* wl = a.w + size_t(nb0 + row)*a.kp + half*8;
+    constexpr int PER = (Tl::UNITS + 255)/256;
+    bf16x8 pre[PER];
+    // unit u of a chunk: voxel u/2 of the halo tile, half u & 1 (16-byte
+    // pieces of one voxel in adjacent lanes)
+    auto fetch = [&](int ch0)
+    {
+        const bool coarse = ch0 < a.c0;
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+        {
+            const int u = tid + 256*k;
+            const int v = u >> 1;
+            const int hx = v % Tl::HX, r = v/Tl::HX;
+            const int gx = x0 - 1 + hx, gy = y0 - 1 + r % Tl::HY;
+            const int gz = z0 - 1 + r/Tl::HY;
+            pre[k] = zero8();
+            if (u < Tl::UNITS && gx >= 0 && gx < W && gy >= 0 && gy < H &&
+                gz >= 0 && gz < D)
+            {
+                if (coarse)
+                    pre[k] = *reinterpret_cast<const bf16x8*>(
+                        a.up + size_t(((gz >> 1)*(H >> 1) + (gy >> 1))*
+                                      (W >> 1) + (gx >> 1))*a.ldu +
+                        ch0 + 8*(u & 1));
+                else
+                    pre[k] = *reinterpret_cast<const bf16x8*>(
+                        a.x + size_t((gz*H + gy)*W + gx)*a.ldx +
+                        (ch0 - a.c0) + 8*(u & 1));
+            }
+        }
+    };
+    fetch(0);
+    for (int ch0 = 0; ch0 < a.cin; ch0 += 16)
+    {
+        if (ch0 > 0) __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+        {
+            const int u = tid + 256*k;
+            if (u < Tl::UNITS)
+                *reinterpret_cast<bf16x8*>(
+                    lds + ((u & 1)*Tl::HV + (u >> 1))*8) = pre[k];
+        }
+        __syncthreads();
+        if (ch0 + 16 < a.cin) fetch(ch0 + 16);
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+        {
+            // (dz, dx) pairs (0,1), (2,3), (4,5), (6,7), (8,-)
+            const int qa = 2*q, qb = q < 4 ? 2*q + 1 : 8;
+            const int tq = second ? qb : qa;
+            const int dz = tq/3, dx = tq - 3*dz;
+            const bool none = q == 4 && second;
+            bf16x8 bw[3][NT];
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                for (int j = 0; j < NT; j++)
+                {
+                    bw[dy][j] = *reinterpret_cast<const bf16x8*>(
+                        wl + size_t(j*16)*a.kp + (dz*9 + dy*3 + dx)*a.cin +
+                        ch0);
+                    if (q == 4 && none) bw[dy][j] = zero8();
+                }
+            const bf16* p = lds + base + (dz*Tl::HY*Tl::HX + dx)*8;
+            bf16x8 av[MT + 2];
+#pragma unroll
+            for (int r = 0; r < MT + 2; r++)
+                av[r] = *reinterpret_cast<const bf16x8*>(p + r*Tl::HX*8);
+#pragma unroll
+            for (int dy = 0; dy < 3; dy++)
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            av[i + dy], bw[dy][j], acc[i][j], 0, 0, 0);
+        }
+    }
+    // outputs rounded to BF16 into LDS, [voxel][channel]
+    __syncthreads();
+    constexpr int NC = 16*NT;
+#pragma unroll
+    for (int j = 0; j < NT; j++)
+    {
+        const float bias = a.bias[nb0 + j*16 + row];
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+            {
+                float v = acc[i][j][q] + bias;
+                if (v < 0.0f) v = 0.0f;
+                const int vox = (wz*Tl::TY + wy + i)*16 + 4*g + q;
+                lds[vox*NC + j*16 + row] = bf16(v);
+            }
+    }
+    __syncthreads();
+    if constexpr (HEAD)
+    {
+        float hw[17];
+#pragma unroll
+        for (int c = 0; c < 17; c++) hw[c] = a.head[c];
+        for (int v = tid; v < Tl::VOX; v += 256)
+        {
+            const int xx = x0 + (v & 15), yy = y0 + (v >> 4) % Tl::TY;
+            const int zz = z0 + (v >> 4)/Tl::TY;
+            const bf16x8 lo = *reinterpret_cast<const bf16x8*>(lds + v*16);
+            const bf16x8 hi = *reinterpret_cast<const bf16x8*>(lds + v*16 + 8);
+            float s = hw[16];
+#pragma unroll
+            for (int c = 0; c < 8; c++) s += hw[c]*float(lo[c]);
+#pragma unroll
+            for (int c = 0; c < 8; c++) s += hw[8 + c]*float(hi[c]);
+            if (xx < W && yy < H && zz < D)
+                a.out[size_t((zz*H + yy)*W + xx)] = s;
+        }
+    }
+    else
+    {
+        for (int u = tid; u < OUT; u += 256)
+        {
+            const int part = u % (2*NT), v = u/(2*NT);
+            const int xx = x0 + (v & 15), yy = y0 + (v >> 4) % Tl::TY;
+            const int zz = z0 + (v >> 4)/Tl::TY;
+            if (xx < W && yy < H && zz < D)
+                *reinterpret_cast<bf16x8*>(
+                    a.y + size_t((zz*H + yy)*W + xx)*a.ldy + nb0 + 8*part) =
+                    *reinterpret_cast<const bf16x8*>(lds + u*8);
+        }
+    }
+    if constexpr (POOL)
+    {
+        for (int u = tid; u < OUT/8; u += 256)
+        {
+            const int part = u % (2*NT), v = u/(2*NT);
+            const int cx = v & 7, cy = (v >> 3) % (Tl::TY/2);
+            const int cz = (v >> 3)/(Tl::TY/2);
+            float s[8];
+#pragma unroll
+            for (int q = 0; q < 8; q++) s[q] = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 8; d++)
+            {
+                const int vox = ((2*cz + (d >> 2))*Tl::TY + 2*cy +
+                                 ((d >> 1) & 1))*16 + 2*cx + (d & 1);
+                const bf16x8 t = *reinterpret_cast<const bf16x8*>(
+                    lds + vox*NC + 8*part);
+#pragma unroll
+                for (int q = 0; q < 8; q++) s[q] += float(t[q]);
+            }
+            bf16x8 o;
+#pragma unroll
+            for (int q = 0; q < 8; q++) o[q] = bf16(0.125f*s[q]);
+            const int X = x0/2 + cx, Y = y0/2 + cy, Z = z0/2 + cz;
+            if (X < W/2 && Y < H/2 && Z < D/2)
+                *reinterpret_cast<bf16x8*>(
+                    a.pool + size_t((Z*(H/2) + Y)*(W/2) + X)*a.ldp + nb0 +
+                    8*part) = o;
+        }
+    }
+}
+
+// First convolution of the inference pass from the two FP32 inputs (rounded
+// to BF16 as k_pack_input does): 2 -> 16 channels with bias and ReLU, its
+// output and the 2x2x2 averages.  K = 9 rows (dz, dy) of three taps times 2
+// channels, padded to 8: a lane's values are contiguous in LDS, three matrix
+// instructions per 16 voxels where the padding to 8 channels took seven.
+__global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
+                                                    const float* c,
+                                                    const bf16* w, int kp,
+                                                    const float* bias, bf16* y,
+                                                    int ldy, bf16* pool,
+                                                    int ldp)
+{
+    constexpr int TY = 8, TZ = 4, HX = 18, HY = TY + 2, HZ = TZ + 2;
+    constexpr int VOX = 16*TY*TZ;
+    __shared__ __align__(16) unsigned char raw[VOX*32];
+    static_assert(VOX*32 >= HX*HY*HZ*4, "");
+    unsigned* in = reinterpret_cast<unsigned*>(raw);
+    bf16* lds = reinterpret_cast<bf16*>(raw);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = lane & 15, g = lane >> 4;
+    const int W = gr.W, H = gr.H, D = gr.D;
+    const int ntx = (W + 15)/16, nty = (H + TY - 1)/TY;
+    const int b = blockIdx.x;
+    const int x0 = (b % ntx)*16;
+    const int y0 = ((b/ntx) % nty)*TY;
+    const int z0 = (b/(ntx*nty))*TZ;
+    for (int v = tid; v < HX*HY*HZ; v += 256)
+    {
+        const int hx = v % HX, r = v/HX;
+        const int gx = x0 - 1 + hx, gy = y0 - 1 + r % HY, gz = z0 - 1 + r/HY;
+        unsigned two = 0;
+        if (gx >= 0 && gx < W && gy >= 0 && gy < H && gz >= 0 && gz < D)
+        {
+            const size_t m = size_t((gz*H + gy)*W + gx);
+            const bf16 p[2] = {bf16(f[m]), bf16(c[m])};
+            two = __builtin_bit_cast(unsigned short, p[0]) |
+                  (unsigned(__builtin_bit_cast(unsigned short, p[1])) << 16);
+        }
+        in[v] = two;
+    }
+    // weights of the lane's output channel, row 4s + g of the nine
+    bf16x8 bw[3];
+    int off[3];
+#pragma unroll
+    for (int s = 0; s < 3; s++)
+    {
+        const int q = 4*s + g;
+        bw[s] = zero8();
+        if (q < 9)
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+            {
+                bw[s][2*t] = w[size_t(row)*kp + (3*q + t)*8];
+                bw[s][2*t + 1] = w[size_t(row)*kp + (3*q + t)*8 + 1];
+            }
+        const int qq = min(q, 8);
+        off[s] = ((qq/3)*HY + qq % 3)*HX;
+    }
+    __syncthreads();
+    floatx4 acc[TY];
+#pragma unroll
+    for (int i = 0; i < TY; i++)
+    {
+        acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        const unsigned* p = in + (wave*HY + i)*HX + row;
+#pragma unroll
+        for (int s = 0; s < 3; s++)
+        {
+            union { unsigned u[4]; bf16x8 v; } av;
+#pragma unroll
+            for (int k = 0; k < 3; k++) av.u[k] = p[off[s] + k];
+            av.u[3] = 0;   // not a neighbour: no value of its may enter
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av.v, bw[s],
+                                                            acc[i], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    const float bs = bias[row];
+#pragma unroll
+    for (int i = 0; i < TY; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+        {
+            float v = acc[i][q] + bs;
+            if (v < 0.0f) v = 0.0f;
+            lds[((wave*TY + i)*16 + 4*g + q)*16 + row] = bf16(v);
+        }
+    __syncthreads();
+    for (int u = tid; u < VOX*2; u += 256)
+    {
+        const int v = u >> 1;
+        const int xx = x0 + (v & 15), yy = y0 + (v >> 4) % TY;
+        const int zz = z0 + (v >> 4)/TY;
+        if (xx < W && yy < H && zz < D)
+            *reinterpret_cast<bf16x8*>(y + size_t((zz*H + yy)*W + xx)*ldy +
+                                       8*(u & 1)) =
+                *reinterpret_cast<const bf16x8*>(lds + u*8);
+    }
+    for (int u = tid; u < VOX/4; u += 256)
+    {
+        const int part = u & 1, v = u >> 1;
+        const int cx = v & 7, cy = (v >> 3) % (TY/2), cz = (v >> 3)/(TY/2);
+        float s[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s[q] = 0.0f;
+#pragma unroll
+        for (int d = 0; d < 8; d++)
+        {
+            const int vox = ((2*cz + (d >> 2))*TY + 2*cy + ((d >> 1) & 1))*16 +
+                            2*cx + (d & 1);
+            const bf16x8 t = *reinterpret_cast<const bf16x8*>(lds + vox*16 +
+                                                              8*part);
+#pragma unroll
+            for (int q = 0; q < 8; q++) s[q] += float(t[q]);
+        }
+        bf16x8 o;
+#pragma unroll
+        for (int q = 0; q < 8; q++) o[q] = bf16(0.125f*s[q]);
+        const int X = x0/2 + cx, Y = y0/2 + cy, Z = z0/2 + cz;
+        if (X < W/2 && Y < H/2 && Z < D/2)
+            *reinterpret_cast<bf16x8*>(
+                pool + size_t((Z*(H/2) + Y)*(W/2) + X)*ldp + 8*part) = o;
+    }
+}
+
 // Weight gradient dW[n][k] += sum over voxels of dZ[m][n] * X[tap(m)][c] for
 // one 16 x 16 tile of (n, k) and one chunk of voxels per wavefront; the
 // chunk partial sums are added into the FP32 gradient atomically.
@@ -1008,6 +1352,61 @@ void conv_fwd(const ConvArgs& a, hipStream_t s)
     case 12: hipLaunchKernelGGL((k_conv_fwd<12>), g, dim3(256), 0, s, a); break;
     default: throw UnetError("unsupported output channel count");
     }
+}
+
+namespace {
+
+template <int NT, int MT>
+void launch_rows(const TileConvArgs& a, hipStream_t s)
+{
+    using Tl = ConvRows<MT>;
+    const dim3 g(unsigned((a.g.W + 15)/16)*
+                     unsigned((a.g.H + Tl::TY - 1)/Tl::TY)*
+                     unsigned((a.g.D + Tl::TZ - 1)/Tl::TZ),
+                 unsigned(a.cout/(16*NT)));
+    if (a.head)
+    {
+        if constexpr (NT == 1)
+            hipLaunchKernelGGL((k_conv_rows<NT, MT, false, true>), g,
+                               dim3(256), 0, s, a);
+    }
+    else if (a.pool)
+        hipLaunchKernelGGL((k_conv_rows<NT, MT, true, false>), g, dim3(256), 0,
+                           s, a);
+    else
+        hipLaunchKernelGGL((k_conv_rows<NT, MT, false, false>), g, dim3(256),
+                           0, s, a);
+}
+
+}  // namespace
+
+void conv_rows(const TileConvArgs& a, hipStream_t s)
+{
+    if (a.cin % 16 || a.c0 % 16 || a.cout % 16 || a.ldx % 8 || a.ldu % 8 ||
+        a.ldy % 8 || a.ldp % 8 || a.kp % 8 || (a.head && a.cout != 16))
+        throw UnetError("convolution shape not supported");
+    // 512-voxel tiles by up to 32 channels (256-voxel ones by 64, whose
+    // accumulators take the registers) while they give two workgroups per
+    // compute unit; below, 256-voxel tiles by 16 channels
+    const long big = long((a.g.W + 15)/16)*((a.g.H + 7)/8)*((a.g.D + 3)/4);
+    if (a.cout % 64 == 0 && 2*big*(a.cout/64) >= 512)
+        launch_rows<4, 4>(a, s);
+    else if (a.cout % 32 == 0 && big*(a.cout/32) >= 512)
+        launch_rows<2, 8>(a, s);
+    else if (big*(a.cout/16) >= 512)
+        launch_rows<1, 8>(a, s);
+    else
+        launch_rows<1, 4>(a, s);
+}
+
+void conv_first(const Grid3& g, const float* f, const float* c, const bf16* w,
+                int kp, const float* bias, bf16* y, int ldy, bf16* pool,
+                int ldp, hipStream_t s)
+{
+    const unsigned n = unsigned((g.W + 15)/16)*unsigned((g.H + 7)/8)*
+                       unsigned((g.D + 3)/4);
+    hipLaunchKernelGGL(k_conv_first, dim3(n), dim3(256), 0, s, g, f, c, w, kp,
+                       bias, y, ldy, pool, ldp);
 }
 
 namespace {

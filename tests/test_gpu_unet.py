@@ -294,3 +294,34 @@ def test_small_grid_forward(gpu, shape, cin, cout):
                      cout, True).float().cpu().numpy()
     # one BF16 rounding of the result and FP32 sums
     assert np.abs(y - ref).max() <= 2.0**-8 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 8), (16, 24, 40), (8, 48, 16),
+                                   (32, 32, 64), (64, 64, 64)])
+def test_inference_pass(gpu, shape):
+    """The inference pass (first convolution from the FP32 inputs, upsampling
+    and skips read in place, averages and output projection in the epilogues)
+    against the float64 restatement with the same BF16 roundings; partial
+    tiles at every level, one and several tiles.  FP32 sums flip the rounding
+    of some activations, by 2^-9 of a value each; were every activation of the
+    eight layers one rounding apart, the output would be off by about
+    sqrt(8) 2^-9 = 0.0055, the bound 2^-7 (a wrong tap or row is of order
+    one).  The same after a training step, whose buffers the pass shares."""
+    r = np.random.default_rng(sum(shape))
+    f = r.standard_normal(shape).astype(np.float32)
+    c = np.where(r.uniform(size=shape) > 0.5, 1.0, -1.0).astype(np.float32)
+    net = unet.Net(seed=5)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    F, C = dev(f), dev(c)
+    for step in range(2):
+        if step:
+            if np.prod(shape) > 20000:
+                break
+            net.train_step(F, C, dev(f), 1e-3)
+        ref, _ = U.net_forward(net.params().astype(np.float64),
+                               f.astype(np.float64), c.astype(np.float64),
+                               bf16=True)
+        got = host(net.forward(F, C))
+        rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert rel < 2.0**-7, rel
+    net.close()

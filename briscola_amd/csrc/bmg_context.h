@@ -209,15 +209,14 @@ struct bmg_ctx
     int fgraphMode = -1;
     long fgraphGen = -1;
     // learned preconditioner: network (not owned), dense FP32 buffers of the
-    // level-0 interior (input, coefficient channel, output) and the host
-    // copy of the coefficient channel of the current operator
+    // level-0 interior (input, coefficient channel, output); the channel is
+    // written when an operator with face coefficients is set
     bmg_unet* unet = nullptr;
     float* uIn = nullptr;
     float* uCoef = nullptr;
     float* uOut = nullptr;
-    std::vector<float> coefChannel;
     double coefScale = 1.0;   // 10^mean(log10 lambda) of the cells
-    bool coefUploaded = false;
+    bool coefUploaded = false;   // uCoef holds the current channel
     // flexible-CG deflation (opts.deflation): face-connected sets of
     // high-coefficient level-0 cells found when the operator is assembled
     // (host labels per interior cell, -1: none), and their device data,

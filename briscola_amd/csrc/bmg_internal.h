@@ -348,6 +348,10 @@ void launch_save_ghost_coeffs(const LevelDims& L, Pair<const double> a7,
 // b[0] -= inhomogeneous boundary terms of eliminateGhosts (level 0 only)
 void launch_bc_source(const LevelDims& L, const OpView<double>& op,
                       Pair<double> b, const BcData* bcval, hipStream_t s);
+// returns the number of partial sums
+int launch_coef_channel(const LevelDims& L, const double* lx,
+                        const double* ly, const double* lz, float* out,
+                        double* partials, int npartials, hipStream_t s);
 void launch_lambda_restrict(const LevelDims& Lf, const LevelDims& Lc,
                             const double* fw0, const double* fw1,
                             const double* fw2, const double* lamf,

@@ -2581,6 +2581,38 @@ __global__ void k_lambda_restrict(LevelDims Lf, LevelDims Lc, const double* fw0,
     lamc[((long)(i + 1)*Lc.P[1] + (j + 1))*Lc.P[2] + (k + 1)] = value/area;
 }
 
+// Input channel of the learned preconditioner, (log10(mean of the six face
+// values) + 1.5)/1.5 per cell in reference cell order, and one partial sum
+// of 1.5 channel - 1.5 per workgroup.  On the host the logarithms took 5 of
+// the 7 ms of an operator update at 128x96x64.
+__global__ __launch_bounds__(256) void k_coef_channel(LevelDims L,
+                                                      const double* lx,
+                                                      const double* ly,
+                                                      const double* lz,
+                                                      float* out,
+                                                      double* partials)
+{
+    __shared__ double sm[4];
+    const int N1 = L.N[1], N2 = L.N[2];
+    const long n = long(L.N[0])*N1*N2;
+    const long sJ = L.P[2], sI = sJ*L.P[1];
+    double acc = 0.0;
+    for (long t = long(blockIdx.x)*256 + threadIdx.x; t < n;
+         t += long(gridDim.x)*256)
+    {
+        const long r = t/N2;
+        const long p = (r/N1 + 1)*sI + (r % N1 + 1)*sJ + (t - r*N2) + 1;
+        const double m = (lx[p] + lx[p + sI] + ly[p] + ly[p + sJ] + lz[p] +
+                          lz[p + 1])/6.0;
+        const double v = m > 0.0 ? log10(m) : -6.0;
+        const float ch = float((v + 1.5)/1.5);
+        out[t] = ch;
+        acc += 1.5*double(ch) - 1.5;
+    }
+    const double s = block_sum(acc, sm);
+    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
 // Face coefficient area*delta*lambda of the lower face fd of every face cell
 // (linearGaussLaplacianScheme.C:63-77), stored colour-split.
 __global__ void k_face_coeffs(LevelDims L, const double* w0, const double* w1,
@@ -6146,6 +6178,19 @@ void launch_lambda_restrict(const LevelDims& Lf, const LevelDims& Lc,
                    (Lc.N[2] + (fd == 2));
     hipLaunchKernelGGL(k_lambda_restrict, dim3((n + 255)/256), dim3(256), 0, s,
                        Lf, Lc, fw0, fw1, fw2, lamf, lamc, fd);
+}
+
+int launch_coef_channel(const LevelDims& L, const double* lx,
+                        const double* ly, const double* lz, float* out,
+                        double* partials, int npartials, hipStream_t s)
+{
+    direct_only("coefficient channel");
+    const long n = long(L.N[0])*L.N[1]*L.N[2];
+    const int nb = int(std::min<long>((n + 255)/256,
+                                      std::min(1024, npartials)));
+    hipLaunchKernelGGL(k_coef_channel, dim3(nb), dim3(256), 0, s, L, lx, ly,
+                       lz, out, partials);
+    return nb;
 }
 
 void launch_face_coeffs(const LevelDims& L, const double* w0, const double* w1,

@@ -497,12 +497,16 @@ template <typename T>
 void bmg_ctx::prolongFrom(int l, int skipColour)
 {
     // the coarse ghosts are used, so correct them first
-    // (linearProlongationScheme.C:128); the tail leaves them so
-    if (tailLevel<T>() != l + 1)
+    // (linearProlongationScheme.C:128); the tail leaves them so, and the
+    // prolongation by coarse cell forms them from the cells inside as it
+    // loads them (nothing else reads them before the level's next visit
+    // rewrites or ignores them), one launch of 4 us less per level
+    const bool stale = tailLevel<T>() != l + 1;
+    if (stale && !prolong_forms_ghosts(lv[l].L, lv[l + 1].L))
         launch_bc_fill(lv[l + 1].L, op<T>(l + 1), X<T>(l + 1), 1, (l + 1) == 0,
                    &bcval, stream);
     launch_prolong(lv[l].L, lv[l + 1].L, transfer<T>(l), cst(X<T>(l + 1)),
-                   X<T>(l), stream, skipColour);
+                   X<T>(l), stream, skipColour, stale);
 }
 
 // The first sweep of red-black smoothing on level l covers every interior
@@ -3313,6 +3317,9 @@ int bmg_op_prolong(bmg_ctx* c, int level)
         if (level + 1 >= c->nLevels()) throw Error(BMG_ERR_ARG, "no coarser level");
         if (!c->lv[level + 1].haveOp)
             throw Error(BMG_ERR_STATE, "operator not set");
+        // this entry point leaves the coarse ghosts corrected
+        launch_bc_fill(c->lv[level + 1].L, c->op<double>(level + 1),
+                       c->X<double>(level + 1), 1, 0, &c->bcval, c->stream);
         c->prolongFrom<double>(level);
         HIPCK(hipGetLastError());
         HIPCK(hipStreamSynchronize(c->stream));

@@ -275,7 +275,10 @@ template <typename T>
 // overwrites every cell of it; -1 updates all
 void launch_prolong(const LevelDims& Lf, const LevelDims& Lc,
                     const TransferView<T>& tv, Pair<const T> xc, Pair<T> xf,
-                    hipStream_t s, int skipColour = -1);
+                    hipStream_t s, int skipColour = -1, bool ghosts = false);
+// whether it can take the coarse field without its ghosts filled (ghosts
+// true: values outside are those of the homogeneous fill)
+bool prolong_forms_ghosts(const LevelDims& Lf, const LevelDims& Lc);
 // mode 0: periodic faces only (evaluate<nonEliminatedBcs,1>);
 // mode 1: full correctBoundaryConditions; mode 2: Neumann/Dirichlet faces
 // only (correct<eliminatedBcs>); level0 enables the inhomogeneous terms.

@@ -1613,7 +1613,8 @@ __device__ __forceinline__ void prolong8_impl(const Bid bid,
                                               const TransferView<T>& tv,
                                               Pair<const T> xc,
                                               Pair<T> xf,
-                                              const Tiles& tl, int skip)
+                                              const Tiles& tl, int skip,
+                                              int ghosts)
 {
     int bx, by, bz;
     if (!tile_of(tl, bid.x, bx, by, bz)) return;
@@ -1649,20 +1650,38 @@ __device__ __forceinline__ void prolong8_impl(const Bid bid,
                            ? ld(col(xf, cB ^ 1), row + unsigned(ck - 1)) : T(0);
         old[a][b][1] = cB != skip ? ld(col(xf, cB), row + unsigned(ck)) : T(0);
     }
-    // coarse block [x][y][z] = (ci-1+x, cj-1+y, ck-1+z)
+    // coarse block [x][y][z] = (ci-1+x, cj-1+y, ck-1+z); with `ghosts`, the
+    // cells outside are formed from interior ones by the rules of the
+    // homogeneous ghost fill (face_ghost, edge_ghost): one face outside, the
+    // periodic image, the adjacent cell (Neumann) or its negative
+    // (Dirichlet); an edge or corner, the image if every face is periodic,
+    // else the adjacent interior cell
     T cv[3][3][3];
 #pragma unroll
     for (int x = 0; x < 3; x++)
 #pragma unroll
     for (int y = 0; y < 3; y++)
     {
-        const int X = ci - 1 + x, Y = cj - 1 + y;
-        const int base = (X*Lc.P[1] + Y)*Lc.Hz;
+        const bool oX = ghosts && (x == 0 ? ci == 1 : x == 2 && ci == Lc.N[0]);
+        const bool oY = ghosts && (y == 0 ? cj == 1 : y == 2 && cj == Lc.N[1]);
+        const int fX = Lc.bc[x == 2], fY = Lc.bc[2 + (y == 2)];
+        const bool per = (!oX || fX == PER) && (!oY || fY == PER);
 #pragma unroll
         for (int z = 0; z < 3; z++)
         {
-            const int Z = ck - 1 + z;
-            cv[x][y][z] = ld(col(xc, (X + Y + Z) & 1), unsigned(base + (Z >> 1)));
+            const bool oZ = ghosts &&
+                            (z == 0 ? ck == 1 : z == 2 && ck == Lc.N[2]);
+            const int fZ = Lc.bc[4 + (z == 2)];
+            const bool image = per && (!oZ || fZ == PER);
+            const int X = !oX ? ci - 1 + x : !image ? ci : x ? 1 : Lc.N[0];
+            const int Y = !oY ? cj - 1 + y : !image ? cj : y ? 1 : Lc.N[1];
+            const int Z = !oZ ? ck - 1 + z : !image ? ck : z ? 1 : Lc.N[2];
+            T v = ld(col(xc, (X + Y + Z) & 1),
+                     unsigned((X*Lc.P[1] + Y)*Lc.Hz + (Z >> 1)));
+            if (int(oX) + int(oY) + int(oZ) == 1 &&
+                (oX ? fX : oY ? fY : fZ) == DIR)
+                v = T(0) - v;
+            cv[x][y][z] = v;
         }
     }
     // prolongation fractions of the children along each axis
@@ -1750,13 +1769,13 @@ __global__ __launch_bounds__(BX*BY) void k_prolong8(LevelDims Lf, LevelDims Lc,
                                                     TransferView<T> tv,
                                                     Pair<const T> xc,
                                                     Pair<T> xf, Tiles tl,
-                                                    int skip)
+                                                    int skip, int ghosts)
 {
     const Bid bid{blockIdx.x, blockIdx.y, blockIdx.z};
     if (tl.ws != 6)
-        prolong8_impl<T, true>(bid, Lf, Lc, tv, xc, xf, tl, skip);
+        prolong8_impl<T, true>(bid, Lf, Lc, tv, xc, xf, tl, skip, ghosts);
     else
-        prolong8_impl<T, false>(bid, Lf, Lc, tv, xc, xf, tl, skip);
+        prolong8_impl<T, false>(bid, Lf, Lc, tv, xc, xf, tl, skip, ghosts);
 }
 
 template <typename T>
@@ -1773,15 +1792,16 @@ struct KProlong8
         Pair<T> xf;
         Tiles tl;
         int skip;
+        int ghosts;
     };
     __device__ static void run(const Bid bid, const Args& a)
     {
         if (a.tl.ws != 6)
             prolong8_impl<T, true>(bid, a.Lf, a.Lc, a.tv, a.xc, a.xf, a.tl,
-                                   a.skip);
+                                   a.skip, a.ghosts);
         else
             prolong8_impl<T, false>(bid, a.Lf, a.Lc, a.tv, a.xc, a.xf, a.tl,
-                                    a.skip);
+                                    a.skip, a.ghosts);
     }
     static bool retile(Args& a, int ws)
     {
@@ -1791,7 +1811,8 @@ struct KProlong8
     static void launch(dim3 g, size_t shm, hipStream_t s, const Args& a)
     {
         hipLaunchKernelGGL((k_prolong8<T>), g, dim3(bx, by), shm, s, a.Lf,
-                           a.Lc, a.tv, a.xc, a.xf, a.tl, a.skip);
+                           a.Lc, a.tv, a.xc, a.xf, a.tl, a.skip,
+                           a.ghosts);
     }
 };
 
@@ -5912,12 +5933,17 @@ void launch_restrict(const LevelDims& Lf, const LevelDims& Lc,
     dispatch<KRestrict<T>>(tiles_grid(tl), 0, s, {Lf, Lc, tv, rf, bc, tl});
 }
 
+bool prolong_forms_ghosts(const LevelDims& Lf, const LevelDims& Lc)
+{
+    return Lf.N[0] == 2*Lc.N[0] && Lf.N[1] == 2*Lc.N[1] && Lf.N[2] == 2*Lc.N[2];
+}
+
 template <typename T>
 void launch_prolong(const LevelDims& Lf, const LevelDims& Lc,
                     const TransferView<T>& tv, Pair<const T> xc, Pair<T> xf,
-                    hipStream_t s, int skipColour)
+                    hipStream_t s, int skipColour, bool ghosts)
 {
-    if (Lf.N[0] == 2*Lc.N[0] && Lf.N[1] == 2*Lc.N[1] && Lf.N[2] == 2*Lc.N[2])
+    if (prolong_forms_ghosts(Lf, Lc))
     {
         // one thread per coarse cell (k_prolong8)
         const int ws = row_pack_shift(Lc.N[2]);
@@ -5926,7 +5952,8 @@ void launch_prolong(const LevelDims& Lf, const LevelDims& Lc,
                               (Lc.N[1] + rows - 1)/rows, Lc.N[0]);
         tl.ws = ws;
         dispatch<KProlong8<T>>(tiles_grid(tl), 0, s,
-                               {Lf, Lc, tv, xc, xf, tl, skipColour});
+                               {Lf, Lc, tv, xc, xf, tl, skipColour,
+                                ghosts ? 1 : 0});
         return;
     }
     const Tiles tl = pair_tiles_packed(Lf);
@@ -6621,7 +6648,7 @@ void launch_set_cell(Pair<T> f, long idx, int colour, T v, hipStream_t s)
                                      Pair<T>, hipStream_t);                   \
     template void launch_prolong<T>(const LevelDims&, const LevelDims&,       \
                                     const TransferView<T>&, Pair<const T>,    \
-                                    Pair<T>, hipStream_t, int);               \
+                                    Pair<T>, hipStream_t, int, bool);         \
     template void launch_bc_fill<T>(const LevelDims&, const OpView<T>&,       \
                                     Pair<T>, int, int, const BcData*,         \
                                     hipStream_t);                             \

@@ -82,3 +82,30 @@ def test_fp32_leg_equals_launches(gpu, n, bc, coarse_level):
     (a, ra), (b, rb) = out
     assert np.abs(a - b).max() <= 2e-6 * np.abs(a).max()
     assert abs(ra - rb) <= 1e-3 * ra
+
+
+@pytest.mark.parametrize("bc", [(N, D, D, N, N, D), (P, P, N, D, D, D),
+                                (P, P, P, P, D, N), (P,) * 6, (N,) * 6,
+                                (D, D, P, P, N, N)])
+@pytest.mark.parametrize("n,cycle", [((64, 32, 32), oracle.VCYCLE),
+                                     ((48, 64, 32), oracle.WCYCLE),
+                                     ((32, 48, 96), oracle.FCYCLE)])
+def test_ghosts_formed_by_prolongation(gpu, n, cycle, bc):
+    """Levels of more than 4096 cells, whose ghosts the prolongation forms
+    itself: faces of every kind next to each other (edges and corners of
+    mixed kinds), bit for bit."""
+    opts = dict(rel_tol=1e-9, tolerance=0.0, n_sweeps_pre=1, n_sweeps_post=1,
+                cycle=cycle, max_iter=3, coarse_mode=oracle.COARSE_DIRECT,
+                coarse_level=1)
+    verts, b0 = problem(n, bc, 7)
+    o = oracle.Oracle(verts, bc)
+    o.set_opts(**opts)
+    o.assemble(None)
+    o.set_field(oracle.B, 0, b0)
+    it, _, _ = o.solve()
+    ctx = gpu.Context(verts, bc, **opts)
+    ctx.set_laplacian(None)
+    for _ in range(2):
+        x, st = ctx.solve(b0.copy())
+        assert st.iters == it
+        assert np.array_equal(x, o.field(oracle.X, 0))

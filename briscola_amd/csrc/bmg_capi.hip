@@ -486,6 +486,18 @@ void bmg_ctx::residual(int l, bool corrBcs, bool norm, int* nblocks)
                     norm ? partials : nullptr, nblocks, stream);
 }
 
+// The same and the restriction to the coarser level in one launch.
+template <typename T>
+void bmg_ctx::restrictResidual(int l, bool corrBcs)
+{
+    Level& q = lv[l];
+    const OpView<T> o = op<T>(l);
+    if (corrBcs && anyPeriodic())
+        launch_bc_fill(q.L, o, X<T>(l), 0, l == 0, &bcval, stream);
+    launch_residual_restrict(q.L, o, lv[l + 1].L, transfer<T>(l),
+                             cst(X<T>(l)), cst(B<T>(l)), B<T>(l + 1), stream);
+}
+
 template <typename T>
 void bmg_ctx::restrictTo(int l)
 {
@@ -502,7 +514,7 @@ void bmg_ctx::prolongFrom(int l, int skipColour)
     // loads them (nothing else reads them before the level's next visit
     // rewrites or ignores them), one launch of 4 us less per level
     const bool stale = tailLevel<T>() != l + 1;
-    if (stale && !prolong_forms_ghosts(lv[l].L, lv[l + 1].L))
+    if (stale && !refined_by_two(lv[l].L, lv[l + 1].L))
         launch_bc_fill(lv[l + 1].L, op<T>(l + 1), X<T>(l + 1), 1, (l + 1) == 0,
                    &bcval, stream);
     launch_prolong(lv[l].L, lv[l + 1].L, transfer<T>(l), cst(X<T>(l + 1)),
@@ -801,9 +813,14 @@ void bmg_ctx::cycle(std::vector<int>& visits, int l, bool zeroX)
         for (int rep = 0; rep < reps; rep++)
         {
             // the phases of a wrapped level leave its periodic ghosts current
-            if (rep > 0 || l > 0)
-                residual<T>(l, wrapAxes<T>(l) == 0, false, nullptr);
-            restrictTo<T>(l);
+            if ((rep > 0 || l > 0) && refined_by_two(q.L, lv[l + 1].L))
+                restrictResidual<T>(l, wrapAxes<T>(l) == 0);
+            else
+            {
+                if (rep > 0 || l > 0)
+                    residual<T>(l, wrapAxes<T>(l) == 0, false, nullptr);
+                restrictTo<T>(l);
+            }
             cycle<T>(visits, l + 1, true);
             record_tag(cycleTag(lc - l, true));
             prolongFrom<T>(l, postPhaseColour<T>(l));

@@ -456,6 +456,8 @@ struct bmg_ctx
     template <typename T>
     void restrictTo(int l);
     template <typename T>
+    void restrictResidual(int l, bool corrBcs);
+    template <typename T>
     void prolongFrom(int l, int skipColour = -1);
     template <typename T>
     int postPhaseColour(int l) const;

@@ -270,15 +270,21 @@ void launch_restrict(const LevelDims& Lf, const LevelDims& Lc,
                      const TransferView<T>& tv, Pair<const T> rf, Pair<T> bc,
                      hipStream_t s);
 template <typename T>
+void launch_residual_restrict(const LevelDims& Lf, const OpView<T>& op,
+                              const LevelDims& Lc, const TransferView<T>& tv,
+                              Pair<const T> x, Pair<const T> b, Pair<T> bc,
+                              hipStream_t s);
+template <typename T>
 // skipColour (levels refined by 2 on every axis): the fine cells of that
 // colour are left unchanged, for a caller whose next red-black phase
 // overwrites every cell of it; -1 updates all
 void launch_prolong(const LevelDims& Lf, const LevelDims& Lc,
                     const TransferView<T>& tv, Pair<const T> xc, Pair<T> xf,
                     hipStream_t s, int skipColour = -1, bool ghosts = false);
-// whether it can take the coarse field without its ghosts filled (ghosts
-// true: values outside are those of the homogeneous fill)
-bool prolong_forms_ghosts(const LevelDims& Lf, const LevelDims& Lc);
+// Refined by 2 on every axis: the prolongation can take the coarse field
+// without its ghosts filled (ghosts true: values outside are those of the
+// homogeneous fill), and the residual can be restricted as it is formed.
+bool refined_by_two(const LevelDims& Lf, const LevelDims& Lc);
 // mode 0: periodic faces only (evaluate<nonEliminatedBcs,1>);
 // mode 1: full correctBoundaryConditions; mode 2: Neumann/Dirichlet faces
 // only (correct<eliminatedBcs>); level0 enables the inhomogeneous terms.

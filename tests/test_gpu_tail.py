@@ -109,3 +109,35 @@ def test_ghosts_formed_by_prolongation(gpu, n, cycle, bc):
         x, st = ctx.solve(b0.copy())
         assert st.iters == it
         assert np.array_equal(x, o.field(oracle.X, 0))
+
+
+@pytest.mark.parametrize("bc", [(N, D, P, P, N, N), (P, P, D, N, P, P)])
+@pytest.mark.parametrize("faces", [False, True])
+def test_residual_restricted_as_formed(gpu, faces, bc):
+    """A level of more than 32768 cells below the finest: its residual by
+    axis factors or face coefficients, restricted in the same launch, bit for
+    bit (coarse rows of 24 cells, packed; the levels below are stencils)."""
+    n = (64, 96, 96)
+    opts = dict(rel_tol=1e-9, tolerance=0.0, n_sweeps_pre=1, n_sweeps_post=1,
+                cycle=oracle.VCYCLE, max_iter=2,
+                coarse_mode=oracle.COARSE_DIRECT, coarse_level=1)
+    verts, b0 = problem(n, bc, 11)
+    lam = None
+    if faces:
+        rng = np.random.default_rng(12)
+        lam = [10.0**rng.uniform(-1, 1, b0.shape) for _ in range(3)]
+        for d in range(3):
+            if bc[2*d] == P:
+                # one coefficient for the two sides of a periodic face
+                m = np.moveaxis(lam[d], d, 0)
+                m[n[d] + 1] = m[1]
+    o = oracle.Oracle(verts, bc)
+    o.set_opts(**opts)
+    o.assemble(lam)
+    o.set_field(oracle.B, 0, b0)
+    it, _, _ = o.solve()
+    ctx = gpu.Context(verts, bc, **opts)
+    ctx.set_laplacian(lam)
+    x, st = ctx.solve(b0.copy())
+    assert st.iters == it
+    assert np.array_equal(x, o.field(oracle.X, 0))

@@ -3524,14 +3524,19 @@ static double cycleBytes(const bmg_ctx* c, int l, size_t w, bool zeroX)
     {
         const Level& qc = c->lv[l + 1];
         const double nc = double(qc.cells());
-        if (l > 0) bytes += n*cellBytesFull(q, w);
-        bytes += n*double(w) + nc*double(w);
+        // below the finest, levels refined by 2 restrict the residual as it
+        // is formed (neither written nor read again) and form the coarse
+        // ghosts in the prolongation
+        const bool by2 = refined_by_two(q.L, qc.L);
+        if (l > 0 && by2)
+            bytes += n*(cellBytesFull(q, w) - double(w));
+        else
+            bytes += (l > 0 ? n*cellBytesFull(q, w) : 0.0) + n*double(w);
+        bytes += nc*double(w);
         bytes += cycleBytes(c, l + 1, w, true);
-        bytes += 2.0*ghostCells(qc)*double(w);
+        if (!by2) bytes += 2.0*ghostCells(qc)*double(w);
         // prolongation: the fine cells read and written, half of them when
         // the first post-smoothing phase rewrites the other colour
-        const bool by2 = q.L.N[0] == 2*qc.L.N[0] && q.L.N[1] == 2*qc.L.N[1] &&
-                         q.L.N[2] == 2*qc.L.N[2];
         const int skip = w == sizeof(float) ? c->postPhaseColour<float>(l)
                                             : c->postPhaseColour<double>(l);
         bytes += (by2 && skip >= 0 ? 1.0 : 2.0)*n*double(w) + nc*double(w);

@@ -1328,13 +1328,22 @@ void bmg_ctx::prepareLearned()
                         hipMemcpyHostToDevice));
         coefUploaded = true;
     }
+    long netGen = -1;
     try
     {
-        bmg::unet::net_prepare(unet, q0.L.N[0], q0.L.N[1], q0.L.N[2]);
+        netGen = bmg::unet::net_prepare(unet, q0.L.N[0], q0.L.N[1],
+                                        q0.L.N[2]);
     }
     catch (const std::exception& e)
     {
         throw Error(BMG_ERR_HIP, e.what());
+    }
+    // the network's other users (training, another grid or context) replace
+    // the activations that the captured iteration refers to
+    if (netGen != unetGen)
+    {
+        unetGen = netGen;
+        gen++;
     }
 }
 

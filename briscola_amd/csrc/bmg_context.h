@@ -212,6 +212,7 @@ struct bmg_ctx
     // level-0 interior (input, coefficient channel, output); the channel is
     // written when an operator with face coefficients is set
     bmg_unet* unet = nullptr;
+    long unetGen = -1;   // generation of the network's buffers last seen
     float* uIn = nullptr;
     float* uCoef = nullptr;
     float* uOut = nullptr;

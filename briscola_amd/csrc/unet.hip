@@ -144,6 +144,7 @@ struct Net {
     bf16* WT[7] = {nullptr};     // flipped BF16 weights [cin][kpt]
     int step = 0;
     Acts acts;
+    long actsGen = 0;            // changes whenever acts' buffers do
 
     explicit Net(uint64_t seed)
     {
@@ -214,6 +215,7 @@ struct Net {
         const bool same = a.y3 && a.g[0].D == D && a.g[0].H == H &&
                           a.g[0].W == W;
         if (same && (!train || a.train)) return;
+        actsGen++;
         a.freeAll();
         a.train = false;
         for (int l = 0; l < 4; l++)
@@ -465,10 +467,11 @@ int urun(F&& f)
 namespace bmg {
 namespace unet {
 
-void net_prepare(::bmg_unet* u, int D, int H, int W)
+long net_prepare(::bmg_unet* u, int D, int H, int W)
 {
     if (!u) throw UnetError("no learned network attached");
     u->net->ensureActs(D, H, W, false);
+    return u->net->actsGen;
 }
 
 void net_forward(::bmg_unet* u, int D, int H, int W, const float* f,

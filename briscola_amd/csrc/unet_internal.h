@@ -136,8 +136,10 @@ void pack_input(const float* f, const float* lam, int M, bf16* x,
 
 // Solver-facing calls on a network (bmg_unet of bmg_unet.h): allocate the
 // activations of a grid (not allowed during graph capture), and run the
-// forward pass on a given stream (capturable once prepared).
-void net_prepare(struct ::bmg_unet* net, int D, int H, int W);
+// forward pass on a given stream (capturable once prepared).  net_prepare
+// returns the buffers' generation: a capture made at another one refers to
+// freed memory.
+long net_prepare(struct ::bmg_unet* net, int D, int H, int W);
 void net_forward(struct ::bmg_unet* net, int D, int H, int W, const float* f,
                  const float* c, float* out, hipStream_t s);
 

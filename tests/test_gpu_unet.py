@@ -325,3 +325,55 @@ def test_inference_pass(gpu, shape):
         rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
         assert rel < 2.0**-7, rel
     net.close()
+
+
+def jacobi_net(alpha):
+    """A network with U(f, c) = alpha f: the first convolution's centre tap
+    gives the two signs of f, the last one passes them on, the head subtracts
+    them."""
+    net = unet.Net(seed=0)
+    lay, hoff, n = U.param_layout()
+    P = np.zeros(n, np.float32)
+    wo, _, kp = lay[0]
+    P[wo + 13*8], P[wo + kp + 13*8] = 1.0, -1.0
+    wo, _, kp = lay[6]
+    P[wo + 13*48 + 32], P[wo + kp + 13*48 + 33] = 1.0, 1.0
+    P[hoff], P[hoff + 1] = alpha, -alpha
+    net.set_params(P)
+    return net
+
+
+def test_learned_solve_after_the_buffers_moved(gpu):
+    """A learned solve repeats bit for bit after its network's activations
+    were replaced: by a training step (learning rate 0) on the same grid, and
+    by a context of another size on the same network.  The solve's captured
+    iteration refers to the activations, so it has to be captured anew."""
+    net = jacobi_net(-1.0/7.0)
+    ctxs, bs = [], []
+    for n in ((16, 16, 16), (24, 16, 32)):
+        c = bmg.Context([np.arange(q + 1)/16.0 for q in n], (0, 0, 1, 1, 0, 1),
+                        rel_tol=1e-8, tolerance=0.0, n_sweeps_pre=2,
+                        n_sweeps_post=2, cycle=bmg.VCYCLE, coarse_level=1,
+                        krylov=bmg.KRYLOV_FCG_LEARNED)
+        c.set_laplacian(None)
+        net.attach(c)
+        b = np.zeros(c.padded(0))
+        b[1:-1, 1:-1, 1:-1] = np.random.default_rng(1).standard_normal(n)
+        ctxs.append(c)
+        bs.append(b)
+    first = []
+    for c, b in zip(ctxs, bs):
+        x, st = c.solve(b.copy())
+        assert st.learned_iters > 0, st.learned_guess_residual
+        first.append(x)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    for k in (0, 1, 0, 0, 1):
+        x, st = ctxs[k].solve(bs[k].copy())
+        assert st.learned_iters > 0 and np.array_equal(x, first[k])
+        f = dev(bs[k][1:-1, 1:-1, 1:-1].astype(np.float32))
+        net.train_step(f, torch.ones_like(f), f, 0.0)
+        x, st = ctxs[k].solve(bs[k].copy())
+        assert st.learned_iters > 0 and np.array_equal(x, first[k])
+    for c in ctxs:
+        c.close()
+    net.close()

@@ -670,7 +670,7 @@ void bmg_ctx::ensureTail()
         const bool stored = std::is_same<T, float>::value ? q.a7f[0] != nullptr
                                                           : q.a7[0] != nullptr;
         if (q.opkind != bmg::OP_STENCIL || !stored ||
-            q.cells() > bmg::TAIL_CELLS || need + bytes(l) > 65536 ||
+            q.cells() > bmg::TAIL_CELLS || need + bytes(l) > bmg::TAIL_LDS ||
             lc - l + 1 > bmg::TAIL_LEVELS)
             break;
         if (l < lc && (lv[l + 1].L.R[0] != 2 || lv[l + 1].L.R[1] != 2 ||
@@ -747,14 +747,22 @@ void bmg_ctx::cycle(std::vector<int>& visits, int l, bool zeroX)
     if (tailLevel<T>() == l)
     {
         // this level and the coarser ones in one workgroup: one launch with
-        // the coarse inverse, else the coarse solve between its two halves
+        // the coarse inverse, else the coarse solve between its two halves;
+        // tagged by their place around the coarse solve, whatever the number
+        // of levels, so that the legs of a batch meet
         const TailState<T>& ts = tail<T>();
         if (ts.whole)
+        {
+            record_tag(cycleTag(0, false));
             launch_tail<T>(ts.plan, ts.lds, 0, stream);
+        }
         else
         {
+            record_tag(cycleTag(1, false));
             launch_tail<T>(ts.plan, ts.lds, 1, stream);
+            record_tag(cycleTag(0, false));
             coarseSolve<T>();
+            record_tag(cycleTag(1, true));
             launch_tail<T>(ts.plan, ts.lds, 2, stream);
         }
         for (int k = l; k <= lc; k++) visits[k]++;

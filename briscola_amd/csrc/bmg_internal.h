@@ -182,6 +182,7 @@ void launch_rbgs_fill(const LevelDims& L, const OpView<T>& op, Pair<T> x,
 // device memory; a smoothing call is a list of steps.
 enum { TAIL_LEVELS = 8, TAIL_STEPS = 64 };
 constexpr long TAIL_CELLS = 4096;
+constexpr size_t TAIL_LDS = 65536;   // bytes at most
 // Steps of a smoothing call: a phase over the interior, the periodic face
 // ghosts, a phase of one or both boundary planes normal to an axis.
 enum { TAIL_PHASE = 0, TAIL_GHOSTS = 1, TAIL_SLAB = 2 };

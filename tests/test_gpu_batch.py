@@ -256,3 +256,52 @@ def test_batch_against_the_oracle(gpu):
             print(f"[batch vs oracle] {tag} system {k}: {got[2]} iterations,"
                   f" error vs FP64 direct {err:.2e}", flush=True)
             assert err < 1e-7, (tag, k, err)
+
+
+@pytest.mark.parametrize("krylov", [bmg.KRYLOV_NONE, bmg.KRYLOV_FCG],
+                         ids=["mg", "fcg"])
+@pytest.mark.parametrize("precision", [bmg.FP64, bmg.MIXED],
+                         ids=["fp64", "mixed"])
+def test_small_level_legs_are_merged(gpu, precision, krylov):
+    """The one-workgroup legs of systems of different extents and numbers of
+    levels share their launches: three orders of the same extents take
+    the launches of one of them, a system beside one of more levels none of
+    its own but the coarse solve's, and every system keeps the bits of its
+    own solve."""
+    def run(shapes):
+        probs = [W.batch_system(k, shape=s) for k, s in enumerate(shapes)]
+        for p in probs:
+            p.bc = (N, D, D, D, N, D)
+        ctxs = []
+        for p in probs:
+            c = bmg.Context(p.vertices, p.bc, p.bc_value, rel_tol=1e-8,
+                            tolerance=0.0, max_iter=200, n_sweeps_pre=2,
+                            n_sweeps_post=2, cycle=bmg.VCYCLE, coarse_level=1,
+                            precision=precision, krylov=krylov)
+            c.set_laplacian(None)
+            ctxs.append(c)
+        alone = []
+        for c, p in zip(ctxs, probs):
+            x = dev(np.zeros_like(p.b))
+            b = dev(p.b)
+            c.solve_device(b.data_ptr(), x.data_ptr())
+            alone.append(x.cpu().numpy())
+        batch = bmg.Batch(ctxs, autotune=False)
+        xs = [dev(np.zeros_like(p.b)) for p in probs]
+        bs = [dev(p.b) for p in probs]
+        batch.solve_device([b.data_ptr() for b in bs],
+                           [x.data_ptr() for x in xs], const_matrix=True)
+        n = batch.info()[0]
+        batch.close()
+        for x, a in zip(xs, alone):
+            assert same(x.cpu().numpy(), a)
+        for c in ctxs:
+            c.close()
+        return n
+
+    one = run([(16, 16, 32)])
+    assert run([(16, 16, 32), (16, 32, 16), (32, 16, 16)]) == one
+    # legs of two and of three levels; in FP64 the coarse systems of 216 and
+    # of 16 cells have kernels of their own
+    assert (run([(48, 48, 48), (16, 16, 32)])
+            == run([(48, 48, 48)]) + (precision == bmg.FP64))

@@ -109,6 +109,7 @@ struct FftGeom {
     double bcval[6];
     double hwall[6];        // width of the boundary cell of each face
     double dT;              // deltaT*dtFrac of the time term; 0: none
+    int oy, oz;             // y and z of a launch's first workgroup
 };
 
 __host__ __device__ inline bool halfWave(int code)
@@ -149,18 +150,19 @@ __device__ __forceinline__ void cellOf(int q, int a, int c, int g[3])
 // the contiguous axis) 16 of c by 4 pairs, so that reads along the
 // contiguous s and writes along c both fill 64-byte lines.
 template <int S>
-__device__ __forceinline__ void cellThread(int& a, int& c, int& p)
+__device__ __forceinline__ void cellThread(const FftGeom& G, int& a, int& c,
+                                           int& p)
 {
-    a = blockIdx.y;
+    a = G.oy + blockIdx.y;
     if (S == 2)
     {
         c = blockIdx.x*16 + (threadIdx.x & 15);
-        p = blockIdx.z*16 + (threadIdx.x >> 4);
+        p = (G.oz + blockIdx.z)*16 + (threadIdx.x >> 4);
     }
     else
     {
         c = blockIdx.x*256 + threadIdx.x;
-        p = blockIdx.z;
+        p = G.oz + blockIdx.z;
     }
 }
 
@@ -169,9 +171,9 @@ __device__ __forceinline__ double rhsValue(const FftGeom& G, const int g[3],
                                            const double* b, const double* x,
                                            const double* xold)
 {
-    const int sI = G.P[1]*G.P[2], sJ = G.P[2];
-    const int st[3] = {sI, sJ, 1};
-    const long c = (long)(g[0] + 1)*sI + (g[1] + 1)*sJ + (g[2] + 1);
+    const long sI = (long)G.P[1]*G.P[2], sJ = G.P[2];
+    const long st[3] = {sI, sJ, 1};
+    const long c = (g[0] + 1)*sI + (g[1] + 1)*sJ + (g[2] + 1);
     double f = b ? -b[c] : 0.0;
     // ddt: minus x.oldTime()/(deltaT*dtFrac) (FFTPoissonSolver.C:116-131)
     if (xold) f = f - xold[c]/G.dT;
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(256) void k_fft_rhs(FftGeom G, const double* b,
                                                  const double* xold, C2* E)
 {
     int a, c, p;
-    cellThread<S>(a, c, p);
+    cellThread<S>(G, a, c, p);
     if (c >= G.a2.L || p >= G.np) return;
     C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
     if (a >= G.a1.n || c >= G.a2.n)
@@ -322,9 +324,9 @@ __device__ __forceinline__ bool orbitThread(const FftGeom& G, OrbitPair& q,
                                             int& p)
 {
     const int n2 = orbits(G.a2);
-    const int t = blockIdx.x*256 + threadIdx.x;
-    const int j1 = t/n2, j2 = t - j1*n2;
-    p = blockIdx.y;
+    const unsigned t = blockIdx.x*256 + threadIdx.x;
+    const int j1 = int(t/unsigned(n2)), j2 = int(t - unsigned(j1)*n2);
+    p = G.oy + blockIdx.y;
     if (j1 >= orbits(G.a1)) return false;
     q.o1 = orbit(G.a1, j1);
     q.o2 = orbit(G.a2, j2);
@@ -372,7 +374,8 @@ __global__ __launch_bounds__(256) void k_fft_modes(FftGeom G, const C2* E,
     if (!orbitThread(G, q, p)) return;
     const C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
     // an index without an image repeats its element
-    const int r1 = q.o1.j*G.a2.L, r1m = (q.m1 ? q.o1.m : q.o1.j)*G.a2.L;
+    const size_t r1 = (size_t)q.o1.j*G.a2.L;
+    const size_t r1m = (size_t)(q.m1 ? q.o1.m : q.o1.j)*G.a2.L;
     const int c2 = q.o2.j, c2m = q.m2 ? q.o2.m : q.o2.j;
     C2 e0 = Ep[r1 + c2], e1 = Ep[r1m + c2], e2 = Ep[r1 + c2m],
        e3 = Ep[r1m + c2m];
@@ -463,7 +466,8 @@ __global__ __launch_bounds__(256) void k_fft_spectrum(FftGeom G,
     toSpectrum(G.a1, q.o1, e2, e3);
     toSpectrum(G.a2, q.o2, e0, e2);
     toSpectrum(G.a2, q.o2, e1, e3);
-    const int r1 = q.o1.j*G.a2.L, r1m = q.o1.m*G.a2.L;
+    const size_t r1 = (size_t)q.o1.j*G.a2.L;
+    const size_t r1m = (size_t)(q.m1 ? q.o1.m : 0)*G.a2.L;
     Ep[r1 + q.o2.j] = e0;
     if (q.m1) Ep[r1m + q.o2.j] = e1;
     if (q.m2) Ep[r1 + q.o2.m] = e2;
@@ -489,7 +493,7 @@ __global__ __launch_bounds__(64) void k_fft_tridiag(
     double* __restrict__ V, const FftRow* __restrict__ row, double pin)
 {
     const int k2 = blockIdx.x*64 + threadIdx.x;
-    const int k1 = blockIdx.y;
+    const int k1 = G.oy + blockIdx.y;
     if (k2 >= G.a2.n) return;
     const size_t nm = (size_t)G.a1.n*G.a2.n;
     const size_t t = (size_t)k1*G.a2.n + k2;
@@ -636,7 +640,7 @@ __global__ __launch_bounds__(256) void k_fft_out(FftGeom G, const C2* E,
                                                  double* x, double scale)
 {
     int a, c, p;
-    cellThread<S>(a, c, p);
+    cellThread<S>(G, a, c, p);
     if (c >= G.a2.n || p >= G.np) return;
     const C2* Ep = E + (size_t)p*G.a1.L*G.a2.L;
     const FftAxis& t = G.a1;
@@ -691,11 +695,12 @@ __global__ __launch_bounds__(256) void k_fft_ghosts(FftGeom g, double* x)
     const int d = blockIdx.z >> 1, side = blockIdx.z & 1;
     const int a1 = d == 0 ? 1 : 0, a2 = d == 2 ? 1 : 2;
     const int u = blockIdx.x*256 + threadIdx.x;
-    if (int(blockIdx.y) >= g.P[a1] || u >= g.P[a2]) return;
+    const int v1 = g.oy + blockIdx.y;
+    if (v1 >= g.P[a1] || u >= g.P[a2]) return;
     const int w = side ? g.P[d] - 1 : 0;
     int q[3];
-    q[0] = d == 0 ? w : int(blockIdx.y);
-    q[1] = d == 0 ? int(blockIdx.y) : (d == 1 ? w : u);
+    q[0] = d == 0 ? w : v1;
+    q[1] = d == 0 ? v1 : (d == 1 ? w : u);
     q[2] = d == 2 ? w : u;
     const long t = ((long)q[0]*g.P[1] + q[1])*g.P[2] + q[2];
     int bo[3], nout = 0;
@@ -954,7 +959,24 @@ void fft_solve_device(bmg_fft* F, const double* db, double* dx,
     FftGeom g = F->g;
     g.dT = dxold ? dT : 0.0;
     hipStream_t s = F->stream;
-    auto blocks = [](int n, int b) { return unsigned((n + b - 1)/b); };
+    auto blocks = [](size_t n, int b) { return unsigned((n + b - 1)/b); };
+    // launches whose y and z stay within the device's grid limit (65536),
+    // which a long axis exceeds
+    auto launch = [&](auto kernel, dim3 grid, unsigned threads, auto... args)
+    {
+        constexpr unsigned most = 65535;
+        for (unsigned z = 0; z < grid.z; z += most)
+            for (unsigned y = 0; y < grid.y; y += most)
+            {
+                g.oy = int(y);
+                g.oz = int(z);
+                hipLaunchKernelGGL(kernel,
+                                   dim3(grid.x, std::min(most, grid.y - y),
+                                        std::min(most, grid.z - z)),
+                                   dim3(threads), 0, s, g, args...);
+                HIPCK(hipGetLastError());
+            }
+    };
     // steps 1 and 6: a thread per plane pair and position
     auto cells = [&](int L1, int L2)
     {
@@ -962,47 +984,24 @@ void fft_solve_device(bmg_fft* F, const double* db, double* dx,
                         : dim3(blocks(L2, 256), L1, g.np);
     };
     const dim3 gin = cells(g.a1.L, g.a2.L), gout = cells(g.a1.n, g.a2.n);
-    if (g.s == 0)
-        hipLaunchKernelGGL(k_fft_rhs<0>, gin, dim3(256), 0, s, g, db, dx,
-                           dxold, F->E);
-    else if (g.s == 1)
-        hipLaunchKernelGGL(k_fft_rhs<1>, gin, dim3(256), 0, s, g, db, dx,
-                           dxold, F->E);
-    else
-        hipLaunchKernelGGL(k_fft_rhs<2>, gin, dim3(256), 0, s, g, db, dx,
-                           dxold, F->E);
-    HIPCK(hipGetLastError());
+    launch(g.s == 0 ? k_fft_rhs<0> : g.s == 1 ? k_fft_rhs<1> : k_fft_rhs<2>,
+           gin, 256, db, (const double*)dx, dxold, F->E);
     void* buf[1] = {F->E};
     if (F->fwd)
         rocfftCheck(rocfft_execute(F->fwd, buf, nullptr, F->info), "forward");
-    const dim3 gorb(blocks(orbits(g.a1)*orbits(g.a2), 256), g.np);
-    hipLaunchKernelGGL(k_fft_modes, gorb, dim3(256), 0, s, g, F->E, F->X);
-    const dim3 gtri(blocks(g.a2.n, 64), g.a1.n);
-    if (g.codes == C_PER)
-        hipLaunchKernelGGL(k_fft_tridiag<true>, gtri, dim3(64), 0, s, g, F->X,
-                           F->R, F->V, F->row, F->pin);
-    else
-        hipLaunchKernelGGL(k_fft_tridiag<false>, gtri, dim3(64), 0, s, g, F->X,
-                           F->R, F->V, F->row, F->pin);
-    hipLaunchKernelGGL(k_fft_spectrum, gorb, dim3(256), 0, s, g, F->X, F->E);
-    HIPCK(hipGetLastError());
+    const dim3 gorb(blocks(size_t(orbits(g.a1))*orbits(g.a2), 256), g.np);
+    launch(k_fft_modes, gorb, 256, (const C2*)F->E, F->X);
+    launch(g.codes == C_PER ? k_fft_tridiag<true> : k_fft_tridiag<false>,
+           dim3(blocks(g.a2.n, 64), g.a1.n), 64, F->X, F->R, F->V, F->row,
+           F->pin);
+    launch(k_fft_spectrum, gorb, 256, (const double*)F->X, F->E);
     if (F->bwd)
         rocfftCheck(rocfft_execute(F->bwd, buf, nullptr, F->info), "inverse");
     const double scale = 1.0/(double(g.a1.n)*double(g.a2.n));
-    if (g.s == 0)
-        hipLaunchKernelGGL(k_fft_out<0>, gout, dim3(256), 0, s, g, F->E, dx,
-                           scale);
-    else if (g.s == 1)
-        hipLaunchKernelGGL(k_fft_out<1>, gout, dim3(256), 0, s, g, F->E, dx,
-                           scale);
-    else
-        hipLaunchKernelGGL(k_fft_out<2>, gout, dim3(256), 0, s, g, F->E, dx,
-                           scale);
-    const int pmax = std::max(g.P[0], g.P[1]);
-    hipLaunchKernelGGL(k_fft_ghosts,
-                       dim3(blocks(std::max(g.P[1], g.P[2]), 256), pmax, 6),
-                       dim3(256), 0, s, g, dx);
-    HIPCK(hipGetLastError());
+    launch(g.s == 0 ? k_fft_out<0> : g.s == 1 ? k_fft_out<1> : k_fft_out<2>,
+           gout, 256, (const C2*)F->E, dx, scale);
+    launch(k_fft_ghosts, dim3(blocks(std::max(g.P[1], g.P[2]), 256),
+                              std::max(g.P[0], g.P[1]), 6), 256, dx);
     HIPCK(hipStreamSynchronize(s));
 }
 

@@ -48,3 +48,29 @@ def test_odd_and_small_sizes(gpu, n, stretch, kinds):
     x = bmg.FFT(verts, bc).solve(b.copy(), x0.copy())
     got = x[1:-1, 1:-1, 1:-1]
     assert np.abs(got - ref).max() <= 1e-11 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("kinds", ["DRP", "NPD", "PNR"])
+@pytest.mark.parametrize("n", [(4, 70000, 3), (140000, 3, 4)])
+def test_axes_beyond_the_grid_limit(gpu, n, kinds):
+    """An axis of more cells, rows or plane pairs than the 65536 workgroups
+    that a launch takes along y or z: the seven-point operator on the result
+    (its ghosts included) gives back the source.  Its rounding is that of a
+    few sums of terms of the size of x/h^2, and the transforms add log2 of
+    their length roundings, so the bound is 64 eps max|x|/h^2."""
+    h = 0.125
+    verts = [np.arange(q + 1)*h for q in n]
+    bc = [k for a in kinds for k in PAIRS[a]]
+    b = np.zeros(tuple(q + 2 for q in n))
+    b[1:-1, 1:-1, 1:-1] = np.random.default_rng(5).standard_normal(n)
+    print(f"[fft long] n={n} kinds={kinds}", flush=True)
+    x = bmg.FFT(verts, bc).solve(b.copy(), np.zeros_like(b))
+    c = (slice(1, -1),)*3
+    lap = -6.0*x[c]
+    for d in range(3):
+        for e in (slice(None, -2), slice(2, None)):
+            lap += x[c[:d] + (e,) + c[d + 1:]]
+    err = np.abs(lap/h**2 + b[c]).max()
+    bound = 64*np.finfo(float).eps*np.abs(x).max()/h**2
+    print(f"[fft long] residual {err:.2e}, bound {bound:.2e}", flush=True)
+    assert err <= bound

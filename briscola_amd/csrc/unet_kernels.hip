@@ -341,7 +341,9 @@ __global__ __launch_bounds__(256) void k_conv_rows(TileConvArgs a)
 {
     using Tl = ConvRows<MT>;
     constexpr int OUT = Tl::VOX*NT*2;        // units of the output tile
-    constexpr int LDS = Tl::UNITS > OUT ? Tl::UNITS : OUT;
+    // the input tile, and a zero unit for each row of a fragment column
+    constexpr int IN = Tl::UNITS + (MT + 1)*Tl::HX + 1;
+    constexpr int LDS = IN > OUT ? IN : OUT;
     __shared__ __align__(16) bf16 lds[LDS*8];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -395,6 +397,8 @@ __global__ __launch_bounds__(256) void k_conv_rows(TileConvArgs a)
         }
     };
     fetch(0);
+    if (tid < MT + 2)
+        *reinterpret_cast<bf16x8*>(lds + (Tl::UNITS + tid*Tl::HX)*8) = zero8();
     for (int ch0 = 0; ch0 < a.cin; ch0 += 16)
     {
         if (ch0 > 0) __syncthreads();
@@ -427,7 +431,10 @@ __global__ __launch_bounds__(256) void k_conv_rows(TileConvArgs a)
                         ch0);
                     if (q == 4 && none) bw[dy][j] = zero8();
                 }
-            const bf16* p = lds + base + (dz*Tl::HY*Tl::HX + dx)*8;
+            // the missing tap reads zeros: an infinity times a zero weight
+            // is a NaN
+            const bf16* p = lds + (none ? Tl::UNITS*8
+                                        : base + (dz*Tl::HY*Tl::HX + dx)*8);
             bf16x8 av[MT + 2];
 #pragma unroll
             for (int r = 0; r < MT + 2; r++)
@@ -596,7 +603,8 @@ __global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
         {
             union { unsigned u[4]; bf16x8 v; } av;
 #pragma unroll
-            for (int k = 0; k < 3; k++) av.u[k] = p[off[s] + k];
+            for (int k = 0; k < 3; k++)
+                av.u[k] = 4*s + g < 9 ? p[off[s] + k] : 0;
             av.u[3] = 0;   // not a neighbour: no value of its may enter
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av.v, bw[s],
                                                             acc[i], 0, 0, 0);

@@ -377,3 +377,18 @@ def test_learned_solve_after_the_buffers_moved(gpu):
     for c in ctxs:
         c.close()
     net.close()
+
+
+def test_infinite_input_stays_infinite(gpu):
+    """With positive weights throughout, one infinite input gives infinities
+    and no NaN: the matrix instructions' padding multiplies no value of the
+    tile by its zeros."""
+    shape = (16, 8, 24)
+    net = unet.Net(seed=0)
+    net.set_params(np.abs(net.params()))
+    f = np.random.default_rng(2).uniform(0.0, 1.0, shape).astype(np.float32)
+    f[5, 3, 13] = np.inf
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    got = host(net.forward(dev(f), torch.ones(shape, device="cuda:0")))
+    assert np.isinf(got[5, 3, 13]) and not np.isnan(got).any()
+    net.close()

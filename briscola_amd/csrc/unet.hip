@@ -364,7 +364,6 @@ struct Net {
         w.taps = 27;
         w.kp = kp[i];
         w.dw = G + woff[i];
-        w.chunk = 256;
         return w;
     }
 
@@ -598,6 +597,43 @@ int bmg_unet_op_conv(int D, int H, int W, const uint16_t* x, int ldx, int cin,
         a.y = reinterpret_cast<bmg::unet::bf16*>(y);
         a.ldy = ldy;
         bmg::unet::conv_fwd(a, nullptr);
+        UCK(hipGetLastError());
+        UCK(hipDeviceSynchronize());
+    });
+}
+
+int bmg_unet_op_conv_rows(int D, int H, int W, const uint16_t* up, int ldu,
+                          int c0, const uint16_t* x, int ldx, int cin,
+                          const uint16_t* w, int kp, int cout,
+                          const float* bias, int nt, int mt, uint16_t* y,
+                          int ldy, uint16_t* pool, int ldp, const float* head,
+                          float* out)
+{
+    return urun([&] {
+        using bmg::unet::bf16;
+        if (!w || !bias || (c0 > 0 && !up) || (c0 < cin && !x) || c0 < 0 ||
+            c0 > cin || kp < 27*cin || (head ? !out : !y) || (head && pool) ||
+            ((c0 > 0 || pool) && (D % 2 || H % 2 || W % 2)))
+            throw UnetError("bad argument");
+        bmg::unet::TileConvArgs a{};
+        a.g = bmg::unet::Grid3{D, H, W};
+        a.up = reinterpret_cast<const bf16*>(up);
+        a.ldu = ldu;
+        a.c0 = c0;
+        a.x = reinterpret_cast<const bf16*>(x);
+        a.ldx = ldx;
+        a.cin = cin;
+        a.w = reinterpret_cast<const bf16*>(w);
+        a.kp = kp;
+        a.cout = cout;
+        a.bias = bias;
+        a.y = reinterpret_cast<bf16*>(y);
+        a.ldy = ldy;
+        a.pool = reinterpret_cast<bf16*>(pool);
+        a.ldp = ldp;
+        a.head = head;
+        a.out = out;
+        bmg::unet::conv_rows(a, nullptr, nt, mt);
         UCK(hipGetLastError());
         UCK(hipDeviceSynchronize());
     });

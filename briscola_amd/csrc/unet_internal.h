@@ -72,13 +72,14 @@ struct WgradArgs {
     int taps;
     int kp;
     float* dw;
-    int chunk;        // voxels per workgroup
+    int chunk = 0;    // voxels per workgroup of the general kernel
 };
 
 inline int round32(int k) { return (k + 31)/32*32; }
 
 void conv_fwd(const ConvArgs& a, hipStream_t s);
-void conv_rows(const TileConvArgs& a, hipStream_t s);
+// nt, mt: tiles of 16 output channels and rows of a wavefront (0: by size).
+void conv_rows(const TileConvArgs& a, hipStream_t s, int nt = 0, int mt = 0);
 // The first convolution (2 real input channels, BF16 of f and c; w as E0's
 // [16][kp]) with bias and ReLU, and its averages.
 void conv_first(const Grid3& g, const float* f, const float* c, const bf16* w,

@@ -1388,25 +1388,44 @@ void launch_rows(const TileConvArgs& a, hipStream_t s)
 
 }  // namespace
 
-void conv_rows(const TileConvArgs& a, hipStream_t s)
+void conv_rows(const TileConvArgs& a, hipStream_t s, int nt, int mt)
 {
     if (a.cin % 16 || a.c0 % 16 || a.cout % 16 || a.ldx % 8 || a.ldu % 8 ||
         a.ldy % 8 || a.ldp % 8 || a.kp % 8 || (a.head && a.cout != 16))
         throw UnetError("convolution shape not supported");
-    // 512-voxel tiles by up to 32 channels (256-voxel ones by 64, whose
-    // accumulators take the registers) while they give two workgroups per
-    // compute unit; below, 256-voxel tiles by 16 channels
+    // the largest tile that gives two workgroups per compute unit (512):
+    // 512 voxels (mt 8) by 64 channels, 256 by 64, 512 by 32, 512 by 16;
+    // below that 256 voxels by 16 channels
     const long big = long((a.g.W + 15)/16)*((a.g.H + 7)/8)*((a.g.D + 3)/4);
-    if (a.cout % 64 == 0 && big*(a.cout/64) >= 512)
+    if (nt == 0)
+    {
+        nt = 1;
+        mt = 8;
+        if (a.cout % 64 == 0 && big*(a.cout/64) >= 512)
+            nt = 4;
+        else if (a.cout % 64 == 0 && 2*big*(a.cout/64) >= 512)
+            nt = mt = 4;
+        else if (a.cout % 32 == 0 && big*(a.cout/32) >= 512)
+            nt = 2;
+        else if (big*(a.cout/16) < 512)
+            mt = 4;
+    }
+    auto tile = [&](int n, int m)
+    {
+        return nt == n && mt == m && a.cout % (16*n) == 0;
+    };
+    if (tile(4, 8))
         launch_rows<4, 8>(a, s);
-    else if (a.cout % 64 == 0 && 2*big*(a.cout/64) >= 512)
+    else if (tile(4, 4))
         launch_rows<4, 4>(a, s);
-    else if (a.cout % 32 == 0 && big*(a.cout/32) >= 512)
+    else if (tile(2, 8))
         launch_rows<2, 8>(a, s);
-    else if (big*(a.cout/16) >= 512)
+    else if (tile(1, 8))
         launch_rows<1, 8>(a, s);
-    else
+    else if (tile(1, 4))
         launch_rows<1, 4>(a, s);
+    else
+        throw UnetError("convolution tile not supported");
 }
 
 void conv_first(const Grid3& g, const float* f, const float* c, const bf16* w,
@@ -1496,7 +1515,8 @@ void conv_wgrad(const WgradArgs& a, float* workspace, float* dbias,
                            workspace, n, a.cout, a.kp, 27*a.cin, total, a.dw);
         return;
     }
-    if (dbias) throw UnetError("weight gradient shape not supported");
+    if (dbias || a.chunk < 1)
+        throw UnetError("weight gradient shape not supported");
     const int M = a.g.D*a.g.H*a.g.W;
     const int K = a.taps*a.cin;
     const dim3 g(nblk(K, 16), nblk(a.cout, 16), nblk(M, a.chunk));

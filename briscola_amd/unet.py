@@ -23,7 +23,8 @@ EXPORTS = [
     "bmg_unet_last_error", "bmg_unet_create", "bmg_unet_destroy",
     "bmg_unet_num_params", "bmg_unet_get_params", "bmg_unet_set_params",
     "bmg_unet_get_grads", "bmg_unet_forward", "bmg_unet_train_step",
-    "bmg_unet_op_conv", "bmg_unet_op_conv_dgrad", "bmg_unet_op_conv_wgrad",
+    "bmg_unet_op_conv", "bmg_unet_op_conv_rows", "bmg_unet_op_conv_dgrad",
+    "bmg_unet_op_conv_wgrad",
     "bmg_set_learned",
 ]
 
@@ -48,6 +49,8 @@ def _lib():
         "bmg_unet_forward": (I, [P, I, I, I, P, P, P]),
         "bmg_unet_train_step": (I, [P, I, I, I, P, P, P, F, FP]),
         "bmg_unet_op_conv": (I, [I, I, I, P, I, I, P, I, I, I, P, I, P, I]),
+        "bmg_unet_op_conv_rows": (I, [I, I, I, P, I, I, P, I, I, P, I, I, P, I,
+                                      I, P, I, P, I, P, P]),
         "bmg_unet_op_conv_dgrad": (I, [I, I, I, P, I, I, P, I, I, P, I]),
         "bmg_unet_op_conv_wgrad": (I, [I, I, I, P, I, I, P, I, I, I, I, P]),
         "bmg_set_learned": (I, [P, P]),
@@ -147,6 +150,25 @@ def op_conv(x, w, bias, cout, relu, taps=27):
         D, H, W, _ptr(x), cin, cin, _ptr(w), w.shape[1], taps, cout,
         _ptr(bias) if bias is not None else None, int(relu), _ptr(y), cout))
     return y
+
+
+def op_conv_rows(up, x, w, bias, y=None, pool=None, head=None, out=None,
+                 tile=(0, 0)):
+    """The inference pass's convolution of [upsampled up | x] (either may be
+    None) with bias and ReLU into y and its averages into pool, or its output
+    projection into out; channel slices of wider tensors keep their strides."""
+    if x is not None:
+        D, H, W = x.shape[:3]
+    else:
+        D, H, W = (2*n for n in up.shape[:3])
+    c0 = up.shape[3] if up is not None else 0
+    cin = c0 + (x.shape[3] if x is not None else 0)
+    p = lambda t: _ptr(t) if t is not None else None
+    ld = lambda t: t.stride(2) if t is not None else 0
+    _check(_lib().bmg_unet_op_conv_rows(
+        D, H, W, p(up), ld(up), c0, p(x), ld(x), cin, _ptr(w), w.shape[1],
+        w.shape[0], _ptr(bias), tile[0], tile[1], p(y), ld(y), p(pool),
+        ld(pool), p(head), p(out)))
 
 
 def op_conv_dgrad(dz, w, cin):

@@ -63,10 +63,25 @@ int bmg_unet_train_step(bmg_unet* net, int D, int H, int W, const float* f,
  * rounded up to 32, zero-filled):
  *   y = act(conv3x3x3(x, w) + bias)        (taps 27) or 1x1x1 (taps 1);
  *   dx = data gradient of conv3x3x3 for output gradient dz;
- *   dw += weight gradient (FP32 [cout][kp]), voxels in chunks of `chunk`. */
+ *   the same conv3x3x3 as the inference pass runs it, with bias and ReLU:
+ *       input channels [0, c0) from `up` (extents D/2, H/2, W/2) through the
+ *       nearest-neighbour upsampling, the others from x; y and, with `pool`,
+ *       its 2x2x2 averages; with `head` (16 weights and a bias, cout = 16)
+ *       only out = head(y).  nt, mt: the tile of a wavefront, 16 nt channels
+ *       by mt rows -- (4, 8), (4, 4), (2, 8), (1, 8), (1, 4), or 0: by size;
+ *   dw += weight gradient (FP32 [cout][kp]); channel counts or strides the
+ *       tiled kernel does not take (cin 8 or a multiple of 16, cout of 16,
+ *       strides of 8, 16-byte aligned) go to a general kernel, which sums
+ *       the voxels in chunks of `chunk`. */
 int bmg_unet_op_conv(int D, int H, int W, const uint16_t* x, int ldx, int cin,
                      const uint16_t* w, int kp, int taps, int cout,
                      const float* bias, int relu, uint16_t* y, int ldy);
+int bmg_unet_op_conv_rows(int D, int H, int W, const uint16_t* up, int ldu,
+                          int c0, const uint16_t* x, int ldx, int cin,
+                          const uint16_t* w, int kp, int cout,
+                          const float* bias, int nt, int mt, uint16_t* y,
+                          int ldy, uint16_t* pool, int ldp, const float* head,
+                          float* out);
 int bmg_unet_op_conv_dgrad(int D, int H, int W, const uint16_t* dz, int lddz,
                            int cout, const uint16_t* w, int kp, int cin,
                            uint16_t* dx, int lddx);

@@ -392,3 +392,84 @@ def test_infinite_input_stays_infinite(gpu):
     got = host(net.forward(dev(f), torch.ones(shape, device="cuda:0")))
     assert np.isinf(got[5, 3, 13]) and not np.isnan(got).any()
     net.close()
+
+
+@pytest.mark.parametrize("shape", [(6, 10, 20), (4, 16, 32)])
+@pytest.mark.parametrize("c0,c1", [(0, 16), (32, 16), (64, 32)])
+@pytest.mark.parametrize("tile", [(4, 8), (4, 4), (2, 8), (1, 8), (1, 4)])
+def test_inference_convolution_tiles(gpu, tile, c0, c1, shape):
+    """Every tile of the inference pass's convolution, with and without the
+    averages and (16 channels) the output projection, from a tensor of half
+    the extents and a slice of a wider one, into a slice: partial and whole
+    tiles, one group of output channels and two.  y against float64 sums of
+    the BF16 products (one BF16 rounding, 2^-8 of the largest value, as
+    above); the averages and the projection bit for bit from y, in the order
+    of the training pass."""
+    r = np.random.default_rng(c0 + tile[0])
+    cin, cout = c0 + c1, 16*tile[0]*(2 if tile[0] < 4 else 1)
+    coarse = tuple(n // 2 for n in shape)
+    rnd = lambda s: U.to_bf16(r.standard_normal(s).astype(np.float32))
+    u, x = rnd(coarse + (c0,)), rnd(shape + (c1,))
+    w = np.zeros((cout, unet.round32(27*cin)), np.float32)
+    w[:, :27*cin] = U.to_bf16((r.standard_normal((cout, 27*cin))
+                               / np.sqrt(27*cin)).astype(np.float32))
+    bias = r.standard_normal(cout).astype(np.float32)
+    cat = np.concatenate([U.up(u), x], axis=3)
+    ref = U.conv(cat, w[:, :27*cin], bias, relu=True)
+    # the fine tensor and the output as slices of wider ones
+    wide = dev_bf16(np.concatenate([np.zeros_like(x), x], axis=3))
+    y = torch.full(shape + (cout + 16,), 7.0, dtype=torch.bfloat16,
+                   device="cuda:0")
+    pool = torch.zeros(coarse + (cout,), dtype=torch.bfloat16, device="cuda:0")
+    args = (dev_bf16(u) if c0 else None, wide[..., c1:], dev_bf16(w),
+            torch.from_numpy(bias).to("cuda:0"))
+    unet.op_conv_rows(*args, y=y[..., 16:], tile=tile)
+    got = host(y[..., 16:])
+    assert np.abs(got - ref).max() <= 2.0**-8*np.abs(ref).max()
+    assert bool((y[..., :16] == 7.0).all())
+    y2 = torch.zeros_like(y)
+    unet.op_conv_rows(*args, y=y2[..., 16:], pool=pool, tile=tile)
+    assert np.array_equal(host(y2[..., 16:]), got)
+    s = np.zeros(coarse + (cout,), np.float32)
+    for d in range(8):
+        s += got[d >> 2::2, (d >> 1) & 1::2, d & 1::2]
+    assert np.array_equal(host(pool), U.to_bf16(np.float32(0.125)*s))
+    if tile[0] > 1:
+        return
+    # the output projection: the first 16 channels' convolution
+    h = r.standard_normal(17).astype(np.float32)
+    out = torch.zeros(shape, device="cuda:0")
+    unet.op_conv_rows(args[0], args[1], args[2][:16].contiguous(), args[3][:16],
+                      head=torch.from_numpy(h).to("cuda:0"), out=out, tile=tile)
+    e = np.full(shape, h[16])
+    for c in range(16):
+        e = e + h[c]*got[..., c]
+    assert e.dtype == np.float32 and np.array_equal(host(out), e)
+
+
+def test_inference_convolution_refuses_other_tiles(gpu):
+    x = torch.zeros((2, 8, 16, 16), dtype=torch.bfloat16, device="cuda:0")
+    w = torch.zeros((32, 448), dtype=torch.bfloat16, device="cuda:0")
+    y = torch.zeros((2, 8, 16, 32), dtype=torch.bfloat16, device="cuda:0")
+    b = torch.zeros(32, device="cuda:0")
+    for tile in ((4, 8), (3, 8), (2, 4), (1, 2)):
+        with pytest.raises(bmg.BmgError):
+            unet.op_conv_rows(None, x, w, b, y=y, tile=tile)
+
+
+@pytest.mark.parametrize("cin,cout,chunk", [(24, 16, 32), (24, 40, 100),
+                                            (40, 16, 1000), (16, 24, 7),
+                                            (8, 20, 4096)])
+def test_general_weight_gradient(gpu, cin, cout, chunk):
+    """Channel counts the tiled weight gradient does not take, in chunks that
+    do not divide the 315 voxels, larger ones and ones below a K step; exact
+    BF16 products summed in FP32, bound as above."""
+    r = np.random.default_rng(cin + chunk)
+    shape = (5, 7, 9)
+    x = U.to_bf16(r.standard_normal(shape + (cin,)).astype(np.float32))
+    dz = U.to_bf16(r.standard_normal(shape + (cout,)).astype(np.float32))
+    kp = unet.round32(27 * cin)
+    ref = U.conv_wgrad(x, dz, kp)
+    got = unet.op_conv_wgrad(dev_bf16(x), dev_bf16(dz), kp, chunk).cpu().numpy()
+    assert np.abs(got - ref).max() < 1e-4 * np.abs(ref).max()
+    assert np.all(got[:, 27 * cin:] == 0.0)

@@ -224,7 +224,8 @@ __global__ __launch_bounds__(256) void k_fft_rhs(FftGeom G, const double* b,
 }
 
 // The elements a thread of steps 3 and 5 owns along one axis: index j and
-// its mirror image m (-1: none), and the modes they give: j itself and, for
+// its mirror image m (-1: none, as index 0 and the middle of an even length
+// have), and the modes they give: j itself and, for
 // a Neumann or Dirichlet pair or a periodic axis, the image.
 struct Orbit {
     int j, m;
@@ -238,8 +239,8 @@ __host__ __device__ inline int orbits(const FftAxis& t)
 __device__ __forceinline__ Orbit orbit(const FftAxis& t, int j)
 {
     if (quarterWave(t.code)) return Orbit{j, 2*t.n - 1 - j};
-    const int m = j == 0 ? 0 : t.n - j;
-    return Orbit{j, m == j ? -1 : m};
+    const int m = t.n - j;
+    return Orbit{j, j == 0 || m == j ? -1 : m};
 }
 
 // Output index of transform index m (a Dirichlet pair's DST-II modes are
@@ -317,7 +318,7 @@ __device__ __forceinline__ C2 loadModes(const FftGeom& G, const double* X,
 // one by one: an array ends up in scratch memory).
 struct OrbitPair {
     Orbit o1, o2;
-    bool m1, m2;     // the images exist and are no repetitions
+    bool m1, m2;     // the images exist
 };
 
 __device__ __forceinline__ bool orbitThread(const FftGeom& G, OrbitPair& q,
@@ -330,9 +331,8 @@ __device__ __forceinline__ bool orbitThread(const FftGeom& G, OrbitPair& q,
     if (j1 >= orbits(G.a1)) return false;
     q.o1 = orbit(G.a1, j1);
     q.o2 = orbit(G.a2, j2);
-    // index 0 is its own image
-    q.m1 = q.o1.m > 0;
-    q.m2 = q.o2.m > 0;
+    q.m1 = q.o1.m >= 0;
+    q.m2 = q.o2.m >= 0;
     return true;
 }
 
@@ -381,13 +381,12 @@ __global__ __launch_bounds__(256) void k_fft_modes(FftGeom G, const C2* E,
        e3 = Ep[r1m + c2m];
     fromSpectrum(G.a1, q.o1, e0, e1);
     fromSpectrum(G.a1, q.o1, e2, e3);
-    if (halfWave(G.a2.code) && q.o2.m == 0) { e2 = e0; e3 = e1; }
     fromSpectrum(G.a2, q.o2, e0, e2);
     fromSpectrum(G.a2, q.o2, e1, e3);
     const bool per1 = G.a1.code == C_PER, per2 = G.a2.code == C_PER;
     const bool q1 = quarterWave(G.a1.code), q2 = quarterWave(G.a2.code);
-    // modes along each axis: j always; the image unless it is none, a
-    // repetition, or a quarter-wave image
+    // modes along each axis: j always; the image where there is one, but a
+    // quarter wave's
     const bool h1 = q.m1 && !q1, h2 = q.m2 && !q2;
     const int i1 = modeIndex(G.a1, q.o1.j), i2 = modeIndex(G.a2, q.o2.j);
     const int k1 = h1 ? modeIndex(G.a1, q.o1.m) : i1;

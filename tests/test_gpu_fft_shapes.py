@@ -17,21 +17,33 @@ PAIRS = {"N": (F.NEU, F.NEU), "D": (F.DIR, F.DIR), "P": (F.PER, F.PER),
          "Q": (F.DIR, F.NEU), "R": (F.NEU, F.DIR)}
 
 
-@pytest.mark.parametrize("kinds", ["NDP", "PPN", "QRD", "PQP", "DNR", "PPP",
-                                   "NNN", "RPQ"])
-@pytest.mark.parametrize("stretch", [0, 1, 2, None])
-@pytest.mark.parametrize("n", [(7, 9, 11), (6, 5, 8), (3, 2, 1), (2, 1, 3),
-                               (5, 70, 67)])
-def test_odd_and_small_sizes(gpu, n, stretch, kinds):
-    if stretch is not None and kinds[stretch] == "P":
-        pytest.skip("periodic axes are uniform")
+def vertices(n, stretch):
     verts = [np.linspace(0.0, 1.0 + d, q + 1) for d, q in enumerate(n)]
     if stretch is not None and n[stretch] > 1:
         t = np.linspace(-1.0, 1.0, n[stretch] + 1)
         verts[stretch] = np.tanh(1.5 * t) / np.tanh(1.5)
-    s = F.plan(verts)[0]
-    if n[s] < (3 if kinds[s] == "P" else 2):
-        pytest.skip("too few cells along the tridiagonal axis")
+    return verts
+
+
+def shapes():
+    """(n, stretched axis, kinds): periodic axes are uniform, and the
+    tridiagonal axis has at least two cells (three if periodic)."""
+    out = []
+    for n, stretch, kinds in itertools.product(
+            [(7, 9, 11), (6, 5, 8), (3, 2, 1), (2, 1, 3), (5, 70, 67)],
+            [0, 1, 2, None],
+            ["NDP", "PPN", "QRD", "PQP", "DNR", "PPP", "NNN", "RPQ"]):
+        if stretch is not None and kinds[stretch] == "P":
+            continue
+        s = F.plan(vertices(n, stretch))[0]
+        if n[s] >= (3 if kinds[s] == "P" else 2):
+            out.append((n, stretch, kinds))
+    return out
+
+
+@pytest.mark.parametrize("n,stretch,kinds", shapes())
+def test_odd_and_small_sizes(gpu, n, stretch, kinds):
+    verts = vertices(n, stretch)
     bc = [k for a in kinds for k in PAIRS[a]]
     print(f"[fft shapes] n={n} kinds={kinds} stretch={stretch}", flush=True)
     rng = np.random.default_rng(4)

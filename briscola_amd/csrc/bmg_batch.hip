@@ -118,6 +118,15 @@ struct BatchPlan
         layout(n, grid);
     }
 
+    // First virtual index of a share of n workgroups after index `at`: a
+    // multiple of 8 keeps its tiles on the XCDs they would have on their own;
+    // shares of one workgroup follow each other, else all of them would run
+    // on one XCD (103 legs 249 us so, 94 us spread)
+    static unsigned shareStart(unsigned at, unsigned n)
+    {
+        return n == 1 ? at : unsigned(alignUp(at, 8));
+    }
+
     void mergeSegment(std::vector<std::vector<LaunchRecord>>& seqs,
                       std::vector<size_t>& head,
                       const std::vector<size_t>& end)
@@ -159,7 +168,7 @@ struct BatchPlan
                 const unsigned wg = r.grid[0]*r.grid[1]*r.grid[2];
                 if (wg == 0) continue;
                 BatchItem it;
-                it.start = m.total;
+                it.start = shareStart(m.total, wg);
                 it.gx = r.grid[0];
                 it.gy = r.grid[1];
                 it.n = wg;
@@ -168,11 +177,11 @@ struct BatchPlan
                 m.grid0.push_back({r.grid[0], r.grid[1], r.grid[2]});
                 m.sys.push_back(int(s));
                 m.args.insert(m.args.end(), r.args.begin(), r.args.end());
-                // each share starts at a multiple of 8 (its XCD order)
-                m.total += unsigned(alignUp(wg, 8));
+                m.total = it.start + wg;
             }
             if (!m.items.empty())
             {
+                m.total = unsigned(alignUp(m.total, 8));
                 m.args0 = m.args;
                 launches.push_back(std::move(m));
             }
@@ -243,9 +252,10 @@ struct BatchPlan
                 it.gy = m.grid0[j][1];
                 it.n = m.grid0[j][0]*m.grid0[j][1]*m.grid0[j][2];
             }
-            it.start = m.total;
-            m.total += unsigned(alignUp(it.n, 8));
+            it.start = shareStart(m.total, it.n);
+            m.total = it.start + it.n;
         }
+        m.total = unsigned(alignUp(m.total, 8));
         m.ws = ws;
     }
 
@@ -263,12 +273,12 @@ struct BatchPlan
             {
                 if (!on[m.sys[j]]) continue;
                 BatchItem it = m.items[j];
-                it.start = total;
-                total += unsigned(alignUp(it.n, 8));
+                it.start = shareStart(total, it.n);
+                total = it.start + it.n;
                 out[k++] = it;
             }
             st[i].nitems = k;
-            st[i].total = total;
+            st[i].total = unsigned(alignUp(total, 8));
         }
     }
 

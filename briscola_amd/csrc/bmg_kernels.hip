@@ -5696,9 +5696,9 @@ struct BatchKind<KBcSource<OP>> { using type = KBcSourceAny; };
 // argument struct K::Args, its workgroup shape (K::bx, K::by), its body
 // K::run(workgroup, args) and K::launch (one launch of k_x).  k_many runs
 // one launch for many independent systems: the systems' workgroups are
-// concatenated into virtual indices (each system's share starting at a
-// multiple of 8, so a workgroup keeps the XCD it would have on its own), a
-// fixed grid (a multiple of 8 workgroups) walks them, and each workgroup
+// concatenated into virtual indices (a share of several workgroups starting
+// at a multiple of 8, so that they keep the XCDs they would have on their
+// own), a fixed grid (a multiple of 8 workgroups) walks them, and each workgroup
 // runs the body on its share's argument struct.  The shares and their
 // number are read from device memory, so the host can drop converged
 // systems between replays of a captured graph.

@@ -305,3 +305,17 @@ def test_small_level_legs_are_merged(gpu, precision, krylov):
     # of 16 cells have kernels of their own
     assert (run([(48, 48, 48), (16, 16, 32)])
             == run([(48, 48, 48)]) + (precision == bmg.FP64))
+
+
+@pytest.mark.parametrize("precision", [bmg.FP64, bmg.MIXED],
+                         ids=["fp64", "mixed"])
+def test_one_workgroup_shares_follow_each_other(gpu, precision):
+    """Shares of one workgroup (the small levels' legs) take consecutive
+    indices, so that they spread over the XCDs: 16 equal systems need fewer
+    virtual workgroups than 16 times one system's, by at least the seven
+    indices a share of its own group of eight would leave empty."""
+    def workgroups(n):
+        systems = [(0, (16, 16, 16), (N, D, D, D, N, D), precision)] * n
+        return solve_batched(systems, autotune=False)[1][1]
+
+    assert workgroups(16) <= 16*workgroups(1) - 7*16

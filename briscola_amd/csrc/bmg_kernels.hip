@@ -3550,8 +3550,8 @@ struct KCoarseWave
 // colour, their coefficients and b in registers for the level's whole leg,
 // and the block's eight residuals, which are the restriction's, in the pair.
 // Per-cell arithmetic is that of the launches (gs_update, pair_Ax's sum,
-// restrict_impl, prolong8_impl, coarse_inv_body), so results keep their
-// bits.  Measured at 16^3, 8^3, 4^3 in FP32: 41 us, of which the phases 13,
+// restrict_impl, prolong8_impl, coarse_inv_body), so FP64 results keep their
+// bits (FP32 cycles carry no such contract).  Measured at 16^3, 8^3, 4^3 in FP32: 41 us, of which the phases 13,
 // the first loads of coefficients 6, the coarse product 3, against about
 // 110 us of launches and gaps; in FP64, whose 16^3 phases one compute unit
 // runs no faster than a launch does, 35 + 16 + 33 us (down, coarse, up)

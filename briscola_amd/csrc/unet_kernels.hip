@@ -1481,8 +1481,7 @@ size_t wgrad_workspace(const WgradArgs& a)
                        reinterpret_cast<uintptr_t>(a.x) % 16 == 0 &&
                        reinterpret_cast<uintptr_t>(a.dz) % 16 == 0;
     if (!tiled) return 0;
-    // at most 512 workgroups, one share each; at least two tiles a share
-    // where the grid has them
+    // at most 512 workgroups, one share each, and no more shares than tiles
     const int S = a.g.W > 16 ? 4 : (a.g.W > 8 ? 2 : 1);
     const int nt = a.cout % 64 == 0 ? 4 : (a.cout % 32 == 0 ? 2 : 1);
     const int yt = nt <= 2 ? 8 : 4, zg = 4/S;

@@ -548,7 +548,9 @@ __global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
     constexpr int TY = 8, TZ = 4, HX = 18, HY = TY + 2, HZ = TZ + 2;
     constexpr int VOX = 16*TY*TZ;
     __shared__ __align__(16) unsigned char raw[VOX*32];
-    static_assert(VOX*32 >= HX*HY*HZ*4, "");
+    // the input tile, then zeros for the rows that are none
+    constexpr int ZERO = HX*HY*HZ, ZEROS = (TY - 1)*HX + 3;
+    static_assert(VOX*32 >= (ZERO + ZEROS)*4, "");
     unsigned* in = reinterpret_cast<unsigned*>(raw);
     bf16* lds = reinterpret_cast<bf16*>(raw);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -573,6 +575,7 @@ __global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
         }
         in[v] = two;
     }
+    if (tid < ZEROS) in[ZERO + tid] = 0;
     // weights of the lane's output channel, row 4s + g of the nine
     bf16x8 bw[3];
     int off[3];
@@ -588,8 +591,8 @@ __global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
                 bw[s][2*t] = w[size_t(row)*kp + (3*q + t)*8];
                 bw[s][2*t + 1] = w[size_t(row)*kp + (3*q + t)*8 + 1];
             }
-        const int qq = min(q, 8);
-        off[s] = ((qq/3)*HY + qq % 3)*HX;
+        // past the nine, zeros: an infinity times a zero weight is a NaN
+        off[s] = q < 9 ? ((wave + q/3)*HY + q % 3)*HX + row : ZERO;
     }
     __syncthreads();
     floatx4 acc[TY];
@@ -597,14 +600,14 @@ __global__ __launch_bounds__(256) void k_conv_first(Grid3 gr, const float* f,
     for (int i = 0; i < TY; i++)
     {
         acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-        const unsigned* p = in + (wave*HY + i)*HX + row;
+        const unsigned* p = in + i*HX;
 #pragma unroll
         for (int s = 0; s < 3; s++)
         {
             union { unsigned u[4]; bf16x8 v; } av;
 #pragma unroll
             for (int k = 0; k < 3; k++)
-                av.u[k] = 4*s + g < 9 ? p[off[s] + k] : 0;
+                av.u[k] = p[off[s] + k];
             av.u[3] = 0;   // not a neighbour: no value of its may enter
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av.v, bw[s],
                                                             acc[i], 0, 0, 0);

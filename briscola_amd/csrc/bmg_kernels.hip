@@ -3551,11 +3551,11 @@ struct KCoarseWave
 // and the block's eight residuals, which are the restriction's, in the pair.
 // Per-cell arithmetic is that of the launches (gs_update, pair_Ax's sum,
 // restrict_impl, prolong8_impl, coarse_inv_body), so FP64 results keep their
-// bits (FP32 cycles carry no such contract).  Measured at 16^3, 8^3, 4^3 in FP32: 41 us, of which the phases 13,
-// the first loads of coefficients 6, the coarse product 3, against about
-// 110 us of launches and gaps; in FP64, whose 16^3 phases one compute unit
-// runs no faster than a launch does, 35 + 16 + 33 us (down, coarse, up)
-// against 125 us.  Pitches that put the lanes of a half wavefront into
+// bits (FP32 cycles carry no such contract).  Measured at 16^3, 8^3, 4^3 in
+// FP32: 41 us, of which the phases 13, the first loads of coefficients 6,
+// the coarse product 3, against about 110 us of launches and gaps; in FP64,
+// whose 16^3 phases one compute unit runs no faster than a launch does,
+// 35 + 16 + 33 us (down, coarse, up) against 125 us.  Pitches that put the lanes of a half wavefront into
 // different banks, masks in place of index tests and the kernel's plan in
 // scalar loads took the FP32 leg from 61 to 41 us.
 constexpr int TAIL_NT = 1024;   // threads, one half each
@@ -4244,7 +4244,8 @@ struct KTail
     {
         extern __shared__ __align__(16) unsigned char tail_lds[];
         // read in scalar loads as k_tail's argument is (no kernel writes
-        // it); in vector loads the batch above took 4.26 ms instead of 3.82
+        // it); in vector loads the seven FP64 systems of launch_tail took
+        // 4.26 ms instead of 3.82
         typedef const __attribute__((address_space(4))) TailPlan<T> Plan;
         Plan* const p = (Plan*)(unsigned long long)a.plan;
         tail_body<T, PART>((const TailPlan<T>*)p,
@@ -5698,8 +5699,8 @@ struct BatchKind<KBcSource<OP>> { using type = KBcSourceAny; };
 // one launch for many independent systems: the systems' workgroups are
 // concatenated into virtual indices (a share of several workgroups starting
 // at a multiple of 8, so that they keep the XCDs they would have on their
-// own), a fixed grid (a multiple of 8 workgroups) walks them, and each workgroup
-// runs the body on its share's argument struct.  The shares and their
+// own), a fixed grid (a multiple of 8 workgroups) walks them, and each
+// workgroup runs the body on its share's argument struct.  The shares and their
 // number are read from device memory, so the host can drop converged
 // systems between replays of a captured graph.
 template <class K>

@@ -615,6 +615,10 @@ int bmg_unet_op_conv_rows(int D, int H, int W, const uint16_t* up, int ldu,
             c0 > cin || kp < 27*cin || (head ? !out : !y) || (head && pool) ||
             ((c0 > 0 || pool) && (D % 2 || H % 2 || W % 2)))
             throw UnetError("bad argument");
+        for (const void* p : {(const void*)up, (const void*)x, (const void*)w,
+                              (const void*)y, (const void*)pool})
+            if (reinterpret_cast<uintptr_t>(p) % 16)
+                throw UnetError("tensors must be aligned to 16 bytes");
         bmg::unet::TileConvArgs a{};
         a.g = bmg::unet::Grid3{D, H, W};
         a.up = reinterpret_cast<const bf16*>(up);
